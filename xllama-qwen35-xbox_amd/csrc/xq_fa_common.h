@@ -95,6 +95,8 @@ XQ_DEV uint32_t lds_u16(const uint8_t* p) { return *(const uint16_t*)p; }
 
 struct FaLaunch;
 hipError_t fa_mma_launch(FaArgs a, const FaLaunch& L, hipStream_t stream);
+// The matrix-core engine's 32-bit row indices.
+inline bool fa_mma_rows_ok(int64_t rows) { return rows < (int64_t)1 << 30; }
 // Mask layout the matrix-core engine can read (4-byte aligned rows).
 bool fa_mma_mask_ok(const FaArgs& a);
 // Separate split-merge kernel (used when the merge cannot run inside pass 1).

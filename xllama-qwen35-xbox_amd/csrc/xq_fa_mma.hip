@@ -26,6 +26,12 @@
 //           q4_0 nibbles n enter as the signed bytes 16*(n - 8) against
 //           d_q/16: the integer dot is 16x ggml's and the scale 1/16 of it,
 //           both exact, so every product, and so every score, is ggml's.
+//           q8_0 / q4_0 K under f32 Q (range calls): v_mfma_f32_16x16x32_f16
+//           per block on the exact integers as f16 against Q as f16 hi + lo,
+//           then times d_k in f32. Each pair's Q row enters times a power of
+//           two that puts its largest element in [2^14, 2^15) (undone exactly
+//           in the score factor), so hi + lo keep at least 22 bits of every
+//           element down to 2^-14 of the largest, whatever Q's range.
 //           F16 / E5M2 K: v_mfma_f32_16x16x32_f16 on the exact f16 K with Q
 //           split into f16 hi + lo parts (the NATIVE policy uses hi alone).
 //   values  O^T = V^T W^T, A = 16 head dims x the slice's rows, B = the
@@ -93,7 +99,7 @@ constexpr float kPOff = 4.0f;          // weights are exp2(x - max - 4), in (0, 
 // Mask source of calls without a mask: one zero f16 pair.
 __device__ uint32_t g_fa_zero_mask[1];
 
-template <int KT, int D, int MT>
+template <int KT, int D, int MT, bool QF = false>
 struct DecCfg {
     static constexpr int REC = rec_bytes(KT, D);
     static constexpr int SLICE = kSub * REC;
@@ -103,15 +109,21 @@ struct DecCfg {
     static constexpr int NB = D / kQK;                 // 32-element blocks per row
     static constexpr int NPP = 16 * MT;
     static constexpr bool QUANT = is_quant(KT);
-    static constexpr int QRB = QUANT ? D + 8 * NB : 0;      // LDS Q image row bytes (int8 path; d_q then 4*NB spare bytes that keep the stride)
+    static constexpr bool INTQ = QUANT && !QF;              // integer scores against a q8_0 Q image
+    // f32 Q on quantized K: the low parts of Q (two pair tiles: the high parts too)
+    // as one 1 KiB operand per (pair tile, block), 16 bytes per lane; in registers
+    // beside the accumulators they would spill
+    static constexpr bool QHL = MT == 2;
+    static constexpr int QLO = QUANT && QF ? (QHL ? 2 : 1) * MT * NB * 1024 : 0;
+    static constexpr int QRB = INTQ ? D + 8 * NB : 0;       // LDS Q image row bytes (int8 path; d_q then 4*NB spare bytes that keep the stride)
     static constexpr int RING_W = 2 * 2 * SLICE;            // per wave: 2 stages x (K, V)
     static constexpr int MASK_W = 2 * MT * 512;             // per wave: 2 stages x MT x 2 f16 pairs per lane
-    static constexpr int FIXED = NPP * QRB + 2 * 8 * NPP * 4 + 64;
+    static constexpr int FIXED = NPP * QRB + QLO + 2 * 8 * NPP * 4 + 64;
     static constexpr bool NW8 = 8 * (RING_W + MASK_W) + FIXED <= 160 * 1024 && !(MT == 2 && D == 256);
     static constexpr int NW = NW8 ? 8 : 4;
     static constexpr int RING = NW * RING_W;
     static constexpr int QIMG = RING;                       // Q image after the K/V rings
-    static constexpr int MASKR = QIMG + NPP * QRB;          // mask rings after the Q image
+    static constexpr int MASKR = QIMG + NPP * QRB + QLO;    // mask rings after the Q image
     static constexpr int MS = D + 4;                        // merge row stride (floats)
     static constexpr int MERGE = NW * 16 * MS * 4;
     static constexpr int LOOP = MASKR + NW * MASK_W;
@@ -148,6 +160,39 @@ XQ_DEV int64_t k_block_bytes(const uint8_t* rec, int b, int g) {
         w1 = __builtin_amdgcn_alignbyte(c, m, 2);
     }
     return (int64_t)(((uint64_t)w1 << 32) | w0);
+}
+
+// The same elements in the same order as f16 (exact): q8_0 byte q as
+// (1024 + (q ^ 0x80)) - 1152, q4_0's low nibble n as (1024 + n) - 1032 and its
+// high nibble as (1024 + 16n)/16 - 72.
+template <int KT>
+XQ_DEV h8 k_block_f16(const uint8_t* rec, int b, int g, uint32_t k6400) {
+    uint32_t h[4];
+    if constexpr (KT == XQ_TYPE_Q4_0) {
+        const int off = 18 * b + 2 + 4 * g;
+        const uint32_t w = ((18 * b + 2) & 3) == 0 ? lds_u32(rec + off)
+                                                   : __builtin_amdgcn_alignbyte(lds_u32(rec + off + 2), lds_u32(rec + off - 2), 2);
+        const uint32_t p[2] = {__builtin_amdgcn_perm(0u, w, 0x0c010c00u), __builtin_amdgcn_perm(0u, w, 0x0c030c02u)};
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const h2 lo = __builtin_bit_cast(h2, (p[e] & 0x000f000fu) | k6400);
+            const h2 hi = __builtin_bit_cast(h2, (p[e] & 0x00f000f0u) | k6400);
+            h[e] = __builtin_bit_cast(uint32_t, lo + h2{(_Float16)-1032.0f, (_Float16)-1032.0f});
+            h[2 + e] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(hi, h2{(_Float16)0.0625f, (_Float16)0.0625f},
+                                                                              h2{(_Float16)-72.0f, (_Float16)-72.0f}));
+        }
+    } else {
+        const uint64_t q = (uint64_t)k_block_bytes<KT>(rec, b, g) ^ 0x8080808080808080ull;
+        const uint32_t w[2] = {(uint32_t)q, (uint32_t)(q >> 32)};
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const h2 x = __builtin_bit_cast(h2, __builtin_amdgcn_perm(k6400, w[e], 0x05010500u));
+            const h2 y = __builtin_bit_cast(h2, __builtin_amdgcn_perm(k6400, w[e], 0x05030502u));
+            h[2 * e] = __builtin_bit_cast(uint32_t, x + h2{(_Float16)-1152.0f, (_Float16)-1152.0f});
+            h[2 * e + 1] = __builtin_bit_cast(uint32_t, y + h2{(_Float16)-1152.0f, (_Float16)-1152.0f});
+        }
+    }
+    return __builtin_bit_cast(h8, uint4{h[0], h[1], h[2], h[3]});
 }
 
 // V^T operands of one q8_0 block: the signed bytes 0 (tile 0) and 1 (tile 1)
@@ -300,12 +345,12 @@ XQ_DEV int acc_dim(int c, int t, int lg, int i) {
     return KT == XQ_TYPE_Q4_0 ? 32 * c + 16 * t + 4 * lg + i : 32 * c + 8 * lg + 2 * i + t;
 }
 
-template <int KT, int D, int MT, bool SOFTCAP, bool HI_ONLY>
-__global__ __launch_bounds__((64 * DecCfg<KT, D, MT>::NW)) void fa_dec(FaArgs a) {
-    using C = DecCfg<KT, D, MT>;
+template <int KT, int D, int MT, bool SOFTCAP, bool HI_ONLY, bool QF = false>
+__global__ __launch_bounds__((64 * DecCfg<KT, D, MT, QF>::NW)) void fa_dec(FaArgs a) {
+    using C = DecCfg<KT, D, MT, QF>;
     constexpr int REC = C::REC, SLICE = C::SLICE, CS = C::CS, CPS = C::CPS, NIS = C::NIS;
     constexpr int NB = C::NB, NPP = C::NPP, NW = C::NW, QRB = C::QRB;
-    constexpr bool QUANT = C::QUANT;
+    constexpr bool QUANT = C::QUANT, INTQ = C::INTQ;
     constexpr int BB = KT == XQ_TYPE_Q8_0 ? 34 : 18;
     constexpr int NT = 64 * NW;
     constexpr uint32_t kNegInfH2 = 0xfc00fc00u;  // f16 pair (-inf, -inf)
@@ -477,10 +522,11 @@ __global__ __launch_bounds__((64 * DecCfg<KT, D, MT>::NW)) void fa_dec(FaArgs a)
     //      waited for alone (loads complete in order), so Q does not wait behind
     //      the ring; stage 1's units follow once the rows are read.
     //      Float K: the f16 hi / lo B operands straight from Q, then the units.
-    constexpr bool QSTAGE = QUANT && PPW * D * 4 <= 2 * SLICE;
+    constexpr bool QSTAGE = INTQ && PPW * D * 4 <= 2 * SLICE;
     uint8_t* sQ = smem + C::QIMG;
-    h8 qh[QUANT ? 1 : MT][QUANT ? 1 : NB], ql[QUANT ? 1 : MT][QUANT ? 1 : NB];
-    if constexpr (QUANT) {
+    h8 qh[INTQ || (QUANT && C::QHL) ? 1 : MT][INTQ || (QUANT && C::QHL) ? 1 : NB], ql[QUANT ? 1 : MT][QUANT ? 1 : NB];
+    float qf[MT];  // f32 Q on quantized K: the pair's score factor, scale * log2 e / its power of two
+    if constexpr (INTQ) {
         constexpr int LPB = kQK / VD;
         float x[PPW][VD];
         if constexpr (QSTAGE) {
@@ -585,21 +631,48 @@ __global__ __launch_bounds__((64 * DecCfg<KT, D, MT>::NW)) void fa_dec(FaArgs a)
 #pragma unroll
             for (int c = 0; c < NB; ++c)
 #pragma unroll
-                for (int j = 0; j < 8; ++j) xq[m][c][j] = src[32 * c + 8 * lg + j];
+                for (int j = 0; j < 8; ++j)  // in K's order
+                    xq[m][c][j] = src[32 * c + (KT == XQ_TYPE_Q4_0 ? 4 * lg + 12 * (j >> 2) + j : 8 * lg + j)];
         }
 #pragma unroll
         for (int m = 0; m < MT; ++m) {
             const bool ok = 16 * m + lr < npa;
+            if constexpr (QUANT) {
+                // the row's power of two: its largest element (Inf as the largest
+                // finite exponent) to [2^14, 2^15)
+                float amax = 0.0f;
+#pragma unroll
+                for (int c = 0; c < NB; ++c)
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(xq[m][c][j]));
+                const int e = min((int)(__float_as_uint(xrow_max(amax)) >> 23), 254);
+                const int up = 141 - e;
+                qf[m] = __builtin_ldexpf(a.scale * kLog2e, -up);
+#pragma unroll
+                for (int c = 0; c < NB; ++c)
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) xq[m][c][j] = __builtin_ldexpf(xq[m][c][j], up);
+            }
 #pragma unroll
             for (int c = 0; c < NB; ++c) {
                 // Q = f16 hi + f16 lo (lo = 0 for the NATIVE policy); NaN as ggml's f16 conversion
+                h8 hi, lo;
 #pragma unroll
                 for (int j = 0; j < 8; ++j) {
                     const float xv = ok ? xq[m][c][j] : 0.0f;
                     const uint32_t hb = f32_to_f16_bits(xv);
-                    qh[m][c][j] = __builtin_bit_cast(_Float16, (uint16_t)hb);
-                    ql[m][c][j] = HI_ONLY ? (_Float16)0.0f
+                    hi[j] = __builtin_bit_cast(_Float16, (uint16_t)hb);
+                    // (quantized K: an infinite element keeps a zero low part, so its
+                    // products stay infinite)
+                    lo[j] = HI_ONLY || (QUANT && !__builtin_isfinite(xv)) ? (_Float16)0.0f
                                             : __builtin_bit_cast(_Float16, (uint16_t)f32_to_f16_bits(xv - f16_bits_to_f32(hb)));
+                }
+                if constexpr (!QUANT || !C::QHL) qh[m][c] = hi;
+                if constexpr (!QUANT) {
+                    ql[m][c] = lo;
+                } else if ((m * NB + c) % NW == wave) {  // every wave forms the same operands
+                    *(h8*)(sQ + (m * NB + c) * 1024 + 16 * lane) = lo;
+                    if constexpr (C::QHL) *(h8*)(sQ + ((MT + m) * NB + c) * 1024 + 16 * lane) = hi;
                 }
             }
         }
@@ -611,11 +684,11 @@ __global__ __launch_bounds__((64 * DecCfg<KT, D, MT>::NW)) void fa_dec(FaArgs a)
     __syncthreads();
 
     // ---- B operands of the score product: pair 16m + lr, elements 8lg..8lg+7 of each block
-    int64_t qb[QUANT ? MT : 1][QUANT ? NB : 1];
+    int64_t qb[INTQ ? MT : 1][INTQ ? NB : 1];
     // dqb[m][q]: d_q of block 4q + lg of the lane's pair (the B operand of the
     // 4-block scale product)
-    float dqb[QUANT ? MT : 1][QUANT ? NB / 4 : 1];
-    if constexpr (QUANT) {
+    float dqb[INTQ ? MT : 1][INTQ ? NB / 4 : 1];
+    if constexpr (INTQ) {
 #pragma unroll
         for (int m = 0; m < MT; ++m) {
             const uint8_t* img = sQ + (16 * m + lr) * QRB;
@@ -639,7 +712,7 @@ __global__ __launch_bounds__((64 * DecCfg<KT, D, MT>::NW)) void fa_dec(FaArgs a)
     // q4_0 value operand half then takes one v_and_or (a VOP3 cannot hold it
     // as a literal)
     uint32_t k6400 = 0;
-    if constexpr (KT == XQ_TYPE_Q4_0) asm("v_mov_b32 %0, 0x64006400" : "=v"(k6400));
+    if constexpr (KT == XQ_TYPE_Q4_0 || (QUANT && QF)) asm("v_mov_b32 %0, 0x64006400" : "=v"(k6400));
 #pragma unroll
     for (int m = 0; m < MT; ++m)
 #pragma unroll
@@ -649,7 +722,41 @@ __global__ __launch_bounds__((64 * DecCfg<KT, D, MT>::NW)) void fa_dec(FaArgs a)
     auto scores = [&](auto st_tag, float (&s)[MT][4]) {
         constexpr int ST = decltype(st_tag)::value;
         const uint8_t* Ks = ring + ST * 2 * SLICE;
-        if constexpr (QUANT) {
+        if constexpr (QUANT && QF) {
+#pragma unroll
+            for (int m = 0; m < MT; ++m)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) s[m][i] = 0.0f;
+            // blocks in batches of four: dks[m][4j + i] = d_k(row 4lg + i, block
+            // c0 + j) * the pair's factor, then s += dks * (K . Q of the block). An
+            // Inf block scale enters as NaN: its row's score is never finite, and
+            // the range's poisoning must see it whatever the dot's sign
+#pragma unroll
+            for (int c0 = 0; c0 < NB; c0 += 4) {
+                const float dk = (float)*(const _Float16*)(Ks + lr * REC + BB * (c0 + lg));
+                const float dkl = __builtin_isfinite(dk) ? dk : NAN;
+                f16v dks[MT];
+#pragma unroll
+                for (int m = 0; m < MT; ++m) dks[m] = __builtin_amdgcn_mfma_f32_16x16x1f32(dkl, qf[m], f16v{}, 0, 0, 0);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const h8 kf = k_block_f16<KT>(Ks + lr * REC, c0 + j, lg, k6400);
+#pragma unroll
+                    for (int m = 0; m < MT; ++m) {
+                        h8 hi;
+                        if constexpr (C::QHL)
+                            hi = *(const h8*)(sQ + ((MT + m) * NB + c0 + j) * 1024 + 16 * lane);
+                        else
+                            hi = qh[m][c0 + j];
+                        f4 dot = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, hi, f4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+                        const h8 lo = *(const h8*)(sQ + (m * NB + c0 + j) * 1024 + 16 * lane);
+                        dot = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, lo, dot, 0, 0, 0);
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) s[m][i] = fmaf(dot[i], dks[m][4 * j + i], s[m][i]);
+                    }
+                }
+            }
+        } else if constexpr (QUANT) {
 #pragma unroll
             for (int m = 0; m < MT; ++m)
 #pragma unroll
@@ -1298,9 +1405,18 @@ __global__ __launch_bounds__((64 * DecCfg<KT, D, MT>::NW)) void fa_dec(FaArgs a)
 using DecFn = void (*)(FaArgs);
 
 // Variant of (type, head dim, pair tiles) for the call's softcap and Q policy
-// (hi-only f16 Q exists for float K only).
+// (hi-only f16 Q exists for float K only; f32 Q on quantized K for range calls,
+// which have no softcap).
 template <int KT, int D, int MT>
-static DecFn dec_inst(bool softcap, bool hi_only) {
+static DecFn dec_inst(bool softcap, bool hi_only, bool qf) {
+    if constexpr (is_quant(KT)) {
+        if (qf) {
+            if constexpr (DecCfg<KT, D, MT, true>::FITS)
+                return softcap ? nullptr : fa_dec<KT, D, MT, false, false, true>;
+            else
+                return nullptr;
+        }
+    }
     if constexpr (DecCfg<KT, D, MT>::FITS) {
         if constexpr (is_quant(KT)) {
             return softcap ? fa_dec<KT, D, MT, true, false> : fa_dec<KT, D, MT, false, false>;
@@ -1314,18 +1430,17 @@ static DecFn dec_inst(bool softcap, bool hi_only) {
 }
 
 template <int KT, int D>
-static DecFn dec_for(int mt, bool softcap, bool hi_only) {
-    return mt == 1 ? dec_inst<KT, D, 1>(softcap, hi_only) : mt == 2 ? dec_inst<KT, D, 2>(softcap, hi_only) : nullptr;
+static DecFn dec_for(int mt, int* waves, bool softcap, bool hi_only, bool qf) {
+    if (mt != 1 && mt != 2) return nullptr;
+    *waves = mt == 1 ? (qf ? DecCfg<KT, D, 1, true>::NW : DecCfg<KT, D, 1>::NW)
+                     : (qf ? DecCfg<KT, D, 2, true>::NW : DecCfg<KT, D, 2>::NW);
+    return mt == 1 ? dec_inst<KT, D, 1>(softcap, hi_only, qf) : dec_inst<KT, D, 2>(softcap, hi_only, qf);
 }
 
-template <int KT, int D>
-static int waves_for(int mt) {
-    return mt == 1 ? DecCfg<KT, D, 1>::NW : DecCfg<KT, D, 2>::NW;
-}
-
-static DecFn dec_lookup(int kt, int d, int mt, int* waves, bool softcap = false, bool hi_only = false) {
+// qf: f32 Q on quantized K (float K always takes f32 Q)
+static DecFn dec_lookup(int kt, int d, int mt, int* waves, bool qf, bool softcap = false, bool hi_only = false) {
 #define XQ_DEC_CASE(T, DD) \
-    case T: *waves = waves_for<T, DD>(mt); return dec_for<T, DD>(mt, softcap, hi_only);
+    case T: return dec_for<T, DD>(mt, waves, softcap, hi_only, qf);
     if (d == 128) {
         switch (kt) {
             XQ_DEC_CASE(XQ_TYPE_Q8_0, 128)
@@ -1347,15 +1462,8 @@ static DecFn dec_lookup(int kt, int d, int mt, int* waves, bool softcap = false,
 
 bool fa_mma_available(int kt, int d, int qk_mode, int n_pairs) {
     if (n_pairs < 1 || n_pairs > 32) return false;
-    if (is_quant(kt) && qk_mode != kQkInt8) return false;  // f32-Q scores on quantized K stay on VALU
     int w = 0;
-    return dec_lookup(kt, d, (n_pairs + 15) / 16, &w) != nullptr;
-}
-
-int fa_mma_waves(int kt, int d, int n_pairs) {
-    int w = 4;
-    if (!dec_lookup(kt, d, (n_pairs + 15) / 16, &w)) return 0;
-    return w;
+    return dec_lookup(kt, d, (n_pairs + 15) / 16, &w, is_quant(kt) && qk_mode != kQkInt8) != nullptr;
 }
 
 // The mask rows are read as 4-byte pairs: every row base must be 4-byte aligned.
@@ -1367,10 +1475,10 @@ hipError_t fa_mma_launch(FaArgs a, const FaLaunch& L, hipStream_t stream) {
     const int D = (int)L.q->ne[0];
     const int kt = L.k->type;
     const int mt = (a.QT * a.G + 15) / 16;
-    if (a.L >= (int64_t)1 << 30) return hipErrorInvalidValue;  // 32-bit row indices
+    if (!fa_mma_rows_ok(a.L)) return hipErrorInvalidValue;
     a.hi_only = is_quant(kt) ? 0 : (L.q_round_f16 ? 1 : 0);
     int waves = 0;
-    DecFn fn = dec_lookup(kt, D, mt, &waves, a.softcap != 0.0f, a.hi_only != 0);
+    DecFn fn = dec_lookup(kt, D, mt, &waves, is_quant(kt) && L.qk_mode != kQkInt8, a.softcap != 0.0f, a.hi_only != 0);
     if (!fn) return hipErrorInvalidValue;
     a.q = (const uint8_t*)L.q->data;
     a.q_nb1 = (int64_t)L.q->nb[1];
