@@ -543,83 +543,86 @@ __global__ __launch_bounds__(kThreads) void fa_pass1(FaArgs a, const uint32_t* _
     }
 }
 
-// One wave per (sequence, query, head) row; lane owns dims VPL*lane ..
-// VPL*lane + VPL - 1 and walks the splits in ascending order with the same
-// (wave-uniform) split states and weights as every other lane, so the row
-// needs no barrier and no LDS. The states and the numerators of the first CH
-// splits are loaded together: one memory round trip for up to CH splits (the
-// automatic policy's counts), CH at a time beyond.
-template <int D, int CH>
-__global__ __launch_bounds__(64) void fa_reduce(FaArgs a) {
-    constexpr int VPL = D / 64;
-    using V = typename std::conditional<VPL == 4, float4, float2>::type;
+// Merge of one (sequence, query, head) row's splits in ascending split order, by
+// D / VPL threads: a thread owns VPL dims. The split states are spread over the
+// lanes of every wave (lane l holds splits l, l + 64, ..), so their exponentials
+// are formed once per split and in parallel, and the sums then walk the splits in
+// order with each state read from its lane. The states and the numerators of the
+// first CH splits are loaded together: one memory round trip for up to CH splits,
+// CH at a time beyond.
+// Bound by that round trip and the kernel boundary. Up to 16 splits (the calls
+// with several sequences) one wave takes a row, 16 or 8 bytes a lane; beyond, D
+// lanes do, with 32 or 64 splits in flight. The 64 splits of a one-sequence range
+// call (24 rows of D 256) take 5.4 us, against 17.3 us with one wave per row that
+// held 32 splits and read the other states one after another. Every load of a
+// chunk is unconditional and the numerators are masked by value: with the loads or
+// the sums under branches the compiler serialises them (20 us).
+template <int D, int VPL, int CH>
+__global__ __launch_bounds__(D / VPL) void fa_reduce(FaArgs a) {
+    using V = typename std::conditional<VPL == 4, float4, typename std::conditional<VPL == 2, float2, float>::type>::type;
     const int64_t row = blockIdx.x;
     const int S = a.n_splits;
-    const int lane = threadIdx.x;
+    const int lane = lane_id();
     const int64_t rows_per_seq = (int64_t)a.NQ * a.H;
     const int b = (int)(row / rows_per_seq);
     const int h = (int)(row % a.H);
     const float2* ml = a.part_ml + row * S;
-    const float* po = a.part_o + row * S * D + VPL * lane;
+    const float* po = a.part_o + row * S * D + VPL * threadIdx.x;
     auto ldv = [&](int s) { return *(const V*)(po + (int64_t)s * D); };
-    float2 st[CH];
-    V v0[CH];
+    static_assert(64 % CH == 0, "a chunk's states sit in one register");
+    constexpr int NC = CH < 64 ? 1 : kMaxSplits / 64;  // state registers a lane needs (CH < 64: at most CH splits)
+    float2 st[NC];
 #pragma unroll
-    for (int i = 0; i < CH; ++i) {
-        st[i] = i < S ? ml[i] : make_float2(0.0f, 0.0f);
-        v0[i] = i < S ? ldv(i) : V{};
-    }
+    for (int c = 0; c < NC; ++c) st[c] = 64 * c + lane < S ? ml[64 * c + lane] : make_float2(0.0f, 0.0f);
+    // (past the last split its row again: no branch between the loads)
+    V v[CH];
+#pragma unroll
+    for (int i = 0; i < CH; ++i) v[i] = ldv(min(i, S - 1));
     // participating splits (den != 0): the maximum; a non-finite or negative
     // den or a non-finite maximum is bad (shaders/rkva/rkva_range_reduce_opt.hlsl:39-56)
     float M = -3.402823466e38f;
     bool bad = false;
-    auto visit = [&](float2 x) {
-        if (x.y != 0.0f) {
-            if (!__builtin_isfinite(x.y) || x.y < 0.0f || !__builtin_isfinite(x.x))
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+        if (st[c].y != 0.0f) {
+            if (!__builtin_isfinite(st[c].y) || st[c].y < 0.0f || !__builtin_isfinite(st[c].x))
                 bad = true;
             else
-                M = fmaxf(M, x.x);
+                M = fmaxf(M, st[c].x);
         }
-    };
-#pragma unroll
-    for (int i = 0; i < CH; ++i) visit(st[i]);
-    for (int s = CH; s < S; ++s) visit(ml[s]);
-    float w0[CH];
-    float L = 0.0f;
-#pragma unroll
-    for (int i = 0; i < CH; ++i) {
-        w0[i] = st[i].y != 0.0f ? expf(st[i].x - M) : 0.0f;
-        if (st[i].y != 0.0f) L = fmaf(st[i].y, w0[i], L);
     }
-    for (int s = CH; s < S; ++s) {
-        const float2 x = ml[s];
-        if (x.y != 0.0f) L = fmaf(x.y, expf(x.x - M), L);
+    M = wave_max(M);
+    bad = __builtin_amdgcn_ballot_w64(bad) != 0;
+    float w[NC];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) w[c] = st[c].y != 0.0f ? expf(st[c].x - M) : 0.0f;
+    // the sum and the numerators, split by split. A split that holds no state
+    // (den 0, weight 0) leaves the sum as it is, and its numerators, whatever they
+    // hold, enter as -0, which times 0 leaves every accumulator as it is.
+    float L = 0.0f, acc[VPL];
+#pragma unroll
+    for (int j = 0; j < VPL; ++j) acc[j] = 0.0f;
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+        const int s0 = CH * c;
+        if (s0 >= S) break;
+        if (c > 0) {
+#pragma unroll
+            for (int i = 0; i < CH; ++i) v[i] = ldv(min(s0 + i, S - 1));
+        }
+        const uint64_t part = __builtin_amdgcn_ballot_w64(st[c].y != 0.0f);
+#pragma unroll
+        for (int i = 0; i < CH; ++i) {
+            const float ws = lane_read(w[c], i);
+            L = fmaf(lane_read(st[c].y, i), ws, L);
+            const float* e = (const float*)&v[i];
+#pragma unroll
+            for (int j = 0; j < VPL; ++j) acc[j] = fmaf((part >> i) & 1u ? e[j] : -0.0f, ws, acc[j]);
+        }
     }
     float a1, inv, lse;
     fa_finalize(L == 0.0f ? -INFINITY : M, L, a.sinks != nullptr, a.sinks ? a.sinks[h] : 0.0f, a1, inv, lse);
     bad = bad || !__builtin_isfinite(L) || !__builtin_isfinite(inv) || (L != 0.0f && !__builtin_isfinite(lse));
-    float acc[VPL];
-#pragma unroll
-    for (int j = 0; j < VPL; ++j) acc[j] = 0.0f;
-    auto add = [&](const V& v, float w) {
-        const float* e = (const float*)&v;
-#pragma unroll
-        for (int j = 0; j < VPL; ++j) acc[j] = fmaf(e[j], w, acc[j]);
-    };
-#pragma unroll
-    for (int i = 0; i < CH; ++i)
-        if (st[i].y != 0.0f) add(v0[i], w0[i]);
-    for (int s0 = CH; s0 < S; s0 += CH) {
-        V v[CH];
-#pragma unroll
-        for (int i = 0; i < CH; ++i) v[i] = s0 + i < S ? ldv(s0 + i) : V{};
-#pragma unroll
-        for (int i = 0; i < CH; ++i) {
-            if (s0 + i >= S) break;
-            const float2 x = ml[s0 + i];
-            if (x.y != 0.0f) add(v[i], expf(x.x - M));
-        }
-    }
     float out[VPL];
     bool nonfin = false;
 #pragma unroll
@@ -629,14 +632,14 @@ __global__ __launch_bounds__(64) void fa_reduce(FaArgs a) {
     }
     // range calls: any non-finite participating state, numerator or result
     // poisons the whole row (shaders/rkva/rkva_range_reduce_opt.hlsl:126-132)
-    if (a.poison && (bad || __builtin_amdgcn_ballot_w64(nonfin) != 0)) {
+    if (a.poison && __syncthreads_or(bad || nonfin)) {
 #pragma unroll
         for (int j = 0; j < VPL; ++j) out[j] = NAN;
         lse = NAN;
     }
-    if (lane == 0 && a.lse) a.lse[row] = lse;
+    if (threadIdx.x == 0 && a.lse) a.lse[row] = lse;
     const int iq = (int)((row % rows_per_seq) / a.H);
-    float* o = (float*)(a.dst + (int64_t)b * a.d_nb3 + (int64_t)iq * a.d_nb2 + (int64_t)h * a.d_nb1) + VPL * lane;
+    float* o = (float*)(a.dst + (int64_t)b * a.d_nb3 + (int64_t)iq * a.d_nb2 + (int64_t)h * a.d_nb1) + VPL * threadIdx.x;
     V ov;
     float* oe = (float*)&ov;
 #pragma unroll
@@ -810,15 +813,22 @@ size_t fa_mask_pack_bytes(const xq_tensor* mask, int64_t L, int n_q) {
     return align256((size_t)mask->ne[3] * mask->ne[2] * n_q * mask_pack_cols(L) * 2);
 }
 
+// Mask pairs per workgroup: a row is spread over as many workgroups as its length
+// gives (four rows of 12 289 elements: 4.6 us against 8.6 us with one workgroup per row)
+constexpr int kPackPairs = 512;
 __global__ __launch_bounds__(256) void fa_mask_pack(const uint8_t* __restrict__ src, int64_t nb1, int64_t nb2,
-                                                    int64_t nb3, int n_q, int ne2, int64_t L,
+                                                    int64_t nb3, int n_q, int ne2, int64_t L, uint32_t n_part,
                                                     uint32_t* __restrict__ dst) {
-    const int row = blockIdx.x;  // (b * ne2 + h) * n_q + q
+    const int row = blockIdx.x / n_part;  // (b * ne2 + h) * n_q + q
     const int qi = row % n_q, h = (row / n_q) % ne2, b = row / (n_q * ne2);
     const uint16_t* s = (const uint16_t*)(src + qi * nb1 + h * nb2 + b * nb3);
     const int64_t pairs = mask_pack_cols(L) / 2;
-    uint32_t* d = dst + row * pairs;
-    for (int64_t c = threadIdx.x; c < pairs; c += 256) {
+    uint32_t* d = dst + (int64_t)row * pairs;
+    const int64_t c0 = (int64_t)(blockIdx.x % n_part) * kPackPairs + threadIdx.x;
+#pragma unroll
+    for (int i = 0; i < kPackPairs / 256; ++i) {
+        const int64_t c = c0 + 256 * i;
+        if (c >= pairs) break;
         const uint32_t lo = s[2 * c];
         const uint32_t hi = 2 * c + 1 < L ? s[2 * c + 1] : 0xFC00u;
         d[c] = lo | (hi << 16);
@@ -906,15 +916,25 @@ size_t fa_workspace_bytes(int64_t n_rows, int d, int qk_mode, int kt, int n_spli
     return bytes;
 }
 
+template <int D>
+static void fa_reduce_d(const FaArgs& a, uint32_t n_rows, hipStream_t stream) {
+    const int S = a.n_splits;
+    if (S <= 4)
+        launch("fa_reduce", fa_reduce<D, D / 64, 4>, dim3(n_rows), dim3(64), stream, a);
+    else if (S <= 16)
+        launch("fa_reduce", fa_reduce<D, D / 64, 16>, dim3(n_rows), dim3(64), stream, a);
+    else if (S <= 32)
+        launch("fa_reduce", fa_reduce<D, 1, 32>, dim3(n_rows), dim3(D), stream, a);
+    else
+        launch("fa_reduce", fa_reduce<D, 1, 64>, dim3(n_rows), dim3(D), stream, a);
+}
+
 hipError_t fa_reduce_launch(const FaArgs& a, int d, hipStream_t stream) {
     const int64_t n_rows = (int64_t)a.B * a.NQ * a.H;
-    const bool wide = a.n_splits > 16;
     if (d == 128)
-        launch("fa_reduce", wide ? fa_reduce<128, 32> : fa_reduce<128, 16>, dim3((uint32_t)n_rows), dim3(64),
-               stream, a);
+        fa_reduce_d<128>(a, (uint32_t)n_rows, stream);
     else
-        launch("fa_reduce", wide ? fa_reduce<256, 32> : fa_reduce<256, 16>, dim3((uint32_t)n_rows), dim3(64),
-               stream, a);
+        fa_reduce_d<256>(a, (uint32_t)n_rows, stream);
     return hipGetLastError();
 }
 
@@ -991,8 +1011,9 @@ hipError_t fa_launch(const FaLaunch& L, hipStream_t stream) {
             if (L.workspace_bytes < base + fa_mask_pack_bytes(L.mask, a.L, NQ)) return hipErrorInvalidValue;
             uint32_t* packed = (uint32_t*)(ws + base);
             const int n_pack = NQ * a.m_ne2 * a.m_ne3;
-            launch("fa_mask_pack", fa_mask_pack, dim3((uint32_t)n_pack), dim3(256), stream, a.mask, a.m_nb1,
-                   a.m_nb2, a.m_nb3, NQ, a.m_ne2, a.L, packed);
+            const uint32_t n_part = (uint32_t)((mask_pack_cols(a.L) / 2 + kPackPairs - 1) / kPackPairs);
+            launch("fa_mask_pack", fa_mask_pack, dim3((uint32_t)n_pack * n_part), dim3(256), stream, a.mask, a.m_nb1,
+                   a.m_nb2, a.m_nb3, NQ, a.m_ne2, a.L, n_part, packed);
             a.mask = (const uint8_t*)packed;
             a.m_nb1 = mask_pack_cols(a.L) * 2;
             a.m_nb2 = (int64_t)NQ * a.m_nb1;
