@@ -28,7 +28,7 @@ def _call(torch, q, positions, kraw, vraw, hkv, kv, origin, active, scale, split
 @pytest.mark.parametrize("d,hkv,group,n_q,active", [
     (128, 2, 1, 1, 17),     # one pair of a tile, one row past a wave slice
     (128, 2, 4, 8, 300),    # 32 pairs: two pair tiles
-    (256, 4, 6, 9, 1000),   # query tiles of a part-filled pair tile
+    (256, 4, 6, 9, 1000),   # four pair tiles, two of them ending inside a query's heads
     (256, 1, 20, 2, 515),   # a group above 16 at head dim 256: two pair tiles, four waves
 ])
 def test_fa_range_quant_query_scale(torch_gpu, kv, d, hkv, group, n_q, active):

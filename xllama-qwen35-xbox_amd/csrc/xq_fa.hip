@@ -1001,7 +1001,7 @@ hipError_t fa_launch(const FaLaunch& L, hipStream_t stream) {
 
     // f32 Q on quantized K (range calls) keeps the VALU engine only for rows beyond
     // the matrix-core engine's 32-bit indices: 28 672 q8_0 rows, 24 over 4 heads at
-    // D 256, one query, fa_dec 27.6 us against 76 us and 4.7 us for the Q image
+    // D 256, one query, fa_dec 20.8 us against 76 us and 4.7 us for the Q image
     const bool mma = L.engine != XQ_FA_ENGINE_VALU && fa_mma_available(kt, D, L.qk_mode, QT * G) &&
                      (fa_mma_rows_ok(a.L) || L.qk_mode == kQkInt8 || (kt != XQ_TYPE_Q8_0 && kt != XQ_TYPE_Q4_0));
     if (L.engine == XQ_FA_ENGINE_MFMA && !mma) return hipErrorInvalidValue;

@@ -50,6 +50,7 @@ struct FaArgs {
     int32_t H, Hkv, G, NQ, B, QT, n_qtiles, n_splits, rk3, rv3;
     float scale, softcap, max_bias, m0, m1;
     int32_t n_head_log2;
+    uint32_t g_magic;  // fa_dec: division of a pair index by G
     int32_t poison;
     // matrix-core engine: f32 Q rows (quantised inside the kernel), hi-only
     // f16 Q for the NATIVE policy

@@ -6,8 +6,8 @@
 // workgroup needs to merge inside this kernel: 64.4 against 70.4 us per call
 // on the 32k q8_0 decode, 21.4 against 28.8 us on the 4k f16 decode).
 //
-// Work decomposition. A workgroup owns one (sequence, KV head, query tile,
-// KV split). A split is a contiguous row range, or (AUTO and LENGTH split
+// Work decomposition. A workgroup owns one (sequence, KV head, tile of 16 or 32
+// (query, head) pairs, KV split). A split is a contiguous row range, or (AUTO and LENGTH split
 // modes) every n_splits-th group of NW slices. Its NW waves stream disjoint
 // 16-row slices of the split (slice j goes to wave j % NW) through private
 // double-buffered LDS rings filled by
@@ -110,20 +110,21 @@ struct DecCfg {
     static constexpr int NPP = 16 * MT;
     static constexpr bool QUANT = is_quant(KT);
     static constexpr bool INTQ = QUANT && !QF;              // integer scores against a q8_0 Q image
-    // f32 Q on quantized K: the low parts of Q (two pair tiles: the high parts too)
-    // as one 1 KiB operand per (pair tile, block), 16 bytes per lane; in registers
-    // beside the accumulators they would spill
-    static constexpr bool QHL = MT == 2;
-    static constexpr int QLO = QUANT && QF ? (QHL ? 2 : 1) * MT * NB * 1024 : 0;
+    // f32 Q on quantized K (range calls, which have no mask): Q's high and low parts
+    // as one 1 KiB operand per (part, pair tile, block), 16 bytes per lane, then the
+    // pairs' score factors; in registers beside the accumulators they would spill
+    static constexpr bool QFQ = QUANT && QF;
+    static constexpr int QOPS = QFQ ? 2 * MT * NB * 1024 + 64 * MT : 0;
     static constexpr int QRB = INTQ ? D + 8 * NB : 0;       // LDS Q image row bytes (int8 path; d_q then 4*NB spare bytes that keep the stride)
     static constexpr int RING_W = 2 * 2 * SLICE;            // per wave: 2 stages x (K, V)
-    static constexpr int MASK_W = 2 * MT * 512;             // per wave: 2 stages x MT x 2 f16 pairs per lane
-    static constexpr int FIXED = NPP * QRB + QLO + 2 * 8 * NPP * 4 + 64;
+    static constexpr int ML = QFQ ? 0 : 2 * MT;             // mask loads per slice
+    static constexpr int MASK_W = ML * 512;             // per wave: 2 stages x MT x 2 f16 pairs per lane
+    static constexpr int FIXED = NPP * QRB + QOPS + 2 * 8 * NPP * 4 + 64;
     static constexpr bool NW8 = 8 * (RING_W + MASK_W) + FIXED <= 160 * 1024 && !(MT == 2 && D == 256);
     static constexpr int NW = NW8 ? 8 : 4;
     static constexpr int RING = NW * RING_W;
     static constexpr int QIMG = RING;                       // Q image after the K/V rings
-    static constexpr int MASKR = QIMG + NPP * QRB + QLO;    // mask rings after the Q image
+    static constexpr int MASKR = QIMG + NPP * QRB + QOPS;    // mask rings after the Q image
     static constexpr int MS = D + 4;                        // merge row stride (floats)
     static constexpr int MERGE = NW * 16 * MS * 4;
     static constexpr int LOOP = MASKR + NW * MASK_W;
@@ -350,7 +351,8 @@ __global__ __launch_bounds__((64 * DecCfg<KT, D, MT, QF>::NW)) void fa_dec(FaArg
     using C = DecCfg<KT, D, MT, QF>;
     constexpr int REC = C::REC, SLICE = C::SLICE, CS = C::CS, CPS = C::CPS, NIS = C::NIS;
     constexpr int NB = C::NB, NPP = C::NPP, NW = C::NW, QRB = C::QRB;
-    constexpr bool QUANT = C::QUANT, INTQ = C::INTQ;
+    constexpr bool QUANT = C::QUANT, INTQ = C::INTQ, QFQ = C::QFQ;
+    constexpr int ML = C::ML;
     constexpr int BB = KT == XQ_TYPE_Q8_0 ? 34 : 18;
     constexpr int NT = 64 * NW;
     constexpr uint32_t kNegInfH2 = 0xfc00fc00u;  // f16 pair (-inf, -inf)
@@ -361,7 +363,7 @@ __global__ __launch_bounds__((64 * DecCfg<KT, D, MT, QF>::NW)) void fa_dec(FaArg
 
     const uint32_t n_wg = (uint32_t)a.n_splits * a.n_qtiles * a.Hkv * a.B;
     uint32_t wg = xcd_remap(blockIdx.x, n_wg);
-    // logical order: query tile fastest, then KV head, split, sequence, so the
+    // logical order: pair tile fastest, then KV head, split, sequence, so the
     // heads reading the same rows are neighbours on one XCD (shared L2)
     const int qt = wg % a.n_qtiles;
     wg /= a.n_qtiles;
@@ -369,9 +371,15 @@ __global__ __launch_bounds__((64 * DecCfg<KT, D, MT, QF>::NW)) void fa_dec(FaArg
     wg /= a.Hkv;
     const int split = wg % a.n_splits;
     const int b = wg / a.n_splits;
-    const int iq0 = qt * a.QT;
-    const int nqt = min(a.QT, a.NQ - iq0);
-    const int npa = nqt * a.G;
+    // the tile's pairs: p0 .. p0 + npa - 1 of the KV head's n_q x G (query, head)
+    // pairs, query-major
+    const int p0 = qt * NPP;
+    const int npa = min(NPP, a.NQ * a.G - p0);
+    auto pair_q = [&](int p) {
+        const uint32_t i = (uint32_t)(p0 + p);
+        return (int)(a.g_magic ? __umulhi(i, a.g_magic) : i);
+    };
+    auto pair_h = [&](int p) { return g_kv * a.G + (p0 + p) - pair_q(p) * a.G; };
     const int wave = wave_id();
     const int lane = lane_id();
     const int tid = threadIdx.x;
@@ -388,8 +396,8 @@ __global__ __launch_bounds__((64 * DecCfg<KT, D, MT, QF>::NW)) void fa_dec(FaArg
     int r_all = r_end;  // rows below every pair's limit (per-row limits apply past it)
     if (a.positions) {
         int lmax = 0, lmin = (int)a.L;
-        for (int qq = 0; qq < nqt; ++qq) {
-            const int32_t pos = a.positions[iq0 + qq];
+        for (int iq = pair_q(0); iq <= pair_q(npa - 1); ++iq) {
+            const int32_t pos = a.positions[iq];
             const int lim = pos < a.origin ? 0 : (int)min(a.L, (int64_t)pos - a.origin + 1);
             lmax = max(lmax, lim);
             lmin = min(lmin, lim);
@@ -413,7 +421,7 @@ __global__ __launch_bounds__((64 * DecCfg<KT, D, MT, QF>::NW)) void fa_dec(FaArg
         vo[i] = (uint32_t)(crow[i] * a.v_nb1 + (c % (REC / CS)) * CS);
     }
     // The ring is refilled in half-slice units: the K unit of a slice (NIS K
-    // loads, then its 2*MT mask loads) and its V unit (NIS V loads), each
+    // loads, then its ML mask loads) and its V unit (NIS V loads), each
     // exactly that many vector-memory instructions. A unit reads constant
     // per-lane offsets from a wave-uniform row base; in the slice that holds the
     // last live row, the rows past it re-read that row.
@@ -454,17 +462,17 @@ __global__ __launch_bounds__((64 * DecCfg<KT, D, MT, QF>::NW)) void fa_dec(FaArg
         lim[m] = r_end;  // padding pairs (zero Q, never stored) run like valid ones
         const int p = 16 * m + lr;
         const bool ok = p < npa;
-        const int qq = ok ? p / a.G : 0, h = g_kv * a.G + (ok ? p % a.G : 0);
+        const int iq = pair_q(ok ? p : 0), h = pair_h(ok ? p : 0);
         if (ok) {
             if (a.positions) {
-                const int32_t pos = a.positions[iq0 + qq];
+                const int32_t pos = a.positions[iq];
                 lim[m] = pos < a.origin ? 0 : (int)min((int64_t)r_end, (int64_t)pos - a.origin + 1);
             }
             slope2[m] = alibi_slope(a, h) * kLog2e;
         }
         // padding pairs read the first pair's mask row (always valid memory); with
         // no mask every pair reads the first f16 pair of a zero row
-        moff[m] = a.mask ? (uint32_t)((int64_t)(iq0 + qq) * a.m_nb1 + (int64_t)(h % a.m_ne2) * a.m_nb2) + 8u * lg : 0u;
+        moff[m] = a.mask ? (uint32_t)((int64_t)iq * a.m_nb1 + (int64_t)(h % a.m_ne2) * a.m_nb2) + 8u * lg : 0u;
     }
     // mask of a slice: lane (lr, lg) brings rows t + 4lg + 2k, +1 (k = 0, 1) of its
     // pair's mask row as one f16 pair into its slot of the wave's mask ring, in the
@@ -481,6 +489,7 @@ __global__ __launch_bounds__((64 * DecCfg<KT, D, MT, QF>::NW)) void fa_dec(FaArg
     uint8_t* mring = smem + C::MASKR + wave * C::MASK_W;
     const uint8_t* mplane = a.mask ? a.mask + (int64_t)(b % a.m_ne3) * a.m_nb3 : (const uint8_t*)g_fa_zero_mask;
     auto load_mask = [&](int t, int st) {
+        if constexpr (QFQ) return;
         if (!a.mask) {
 #pragma unroll
             for (int m = 0; m < MT; ++m)
@@ -522,11 +531,11 @@ __global__ __launch_bounds__((64 * DecCfg<KT, D, MT, QF>::NW)) void fa_dec(FaArg
     //      waited for alone (loads complete in order), so Q does not wait behind
     //      the ring; stage 1's units follow once the rows are read.
     //      Float K: the f16 hi / lo B operands straight from Q, then the units.
-    constexpr bool QSTAGE = INTQ && PPW * D * 4 <= 2 * SLICE;
+    constexpr bool QSTAGE = QUANT && PPW * D * 4 <= 2 * SLICE;
     uint8_t* sQ = smem + C::QIMG;
-    h8 qh[INTQ || (QUANT && C::QHL) ? 1 : MT][INTQ || (QUANT && C::QHL) ? 1 : NB], ql[QUANT ? 1 : MT][QUANT ? 1 : NB];
-    float qf[MT];  // f32 Q on quantized K: the pair's score factor, scale * log2 e / its power of two
-    if constexpr (INTQ) {
+    float* sQf = (float*)(sQ + 2 * MT * NB * 1024);  // QFQ: the pairs' score factors
+    h8 qh[QUANT ? 1 : MT][QUANT ? 1 : NB], ql[QUANT ? 1 : MT][QUANT ? 1 : NB];
+    if constexpr (QUANT) {
         constexpr int LPB = kQK / VD;
         float x[PPW][VD];
         if constexpr (QSTAGE) {
@@ -535,8 +544,8 @@ __global__ __launch_bounds__((64 * DecCfg<KT, D, MT, QF>::NW)) void fa_dec(FaArg
             for (int k = 0; k < PPW; ++k) {
                 const int p = wave + k * NW;  // wave-uniform
                 if (p < npa) {
-                    const int qq = p / a.G, h = g_kv * a.G + p % a.G;
-                    const uint8_t* row = a.q + (int64_t)b * a.q_nb3 + (int64_t)(iq0 + qq) * a.q_nb1 + (int64_t)h * a.q_nb2;
+                    const int iq = __builtin_amdgcn_readfirstlane(pair_q(p)), h = __builtin_amdgcn_readfirstlane(pair_h(p));
+                    const uint8_t* row = a.q + (int64_t)b * a.q_nb3 + (int64_t)iq * a.q_nb1 + (int64_t)h * a.q_nb2;
 #pragma unroll
                     for (int i = 0; i < VD; ++i) lds_dma<4>(row, (uint32_t)(64 * i + lane) * 4u, qst + (k * D + 64 * i) * 4);
                 }
@@ -544,7 +553,7 @@ __global__ __launch_bounds__((64 * DecCfg<KT, D, MT, QF>::NW)) void fa_dec(FaArg
             if (t0 < r_end) {
                 k_unit(t0, 0);
                 v_unit(t0, 0);
-                asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * NIS + 2 * MT) : "memory");  // Q rows landed
+                asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * NIS + ML) : "memory");  // Q rows landed
             } else {
                 asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             }
@@ -562,8 +571,7 @@ __global__ __launch_bounds__((64 * DecCfg<KT, D, MT, QF>::NW)) void fa_dec(FaArg
                 const bool ok = p < npa;
                 const float* src = (const float*)a.q;
                 if (ok) {
-                    const int qq = p / a.G, h = g_kv * a.G + p % a.G;
-                    src = (const float*)(a.q + (int64_t)b * a.q_nb3 + (int64_t)(iq0 + qq) * a.q_nb1 + (int64_t)h * a.q_nb2);
+                    src = (const float*)(a.q + (int64_t)b * a.q_nb3 + (int64_t)pair_q(p) * a.q_nb1 + (int64_t)pair_h(p) * a.q_nb2);
                 }
 #pragma unroll
                 for (int j = 0; j < VD; ++j) x[k][j] = ok ? src[lane * VD + j] : 0.0f;
@@ -577,6 +585,36 @@ __global__ __launch_bounds__((64 * DecCfg<KT, D, MT, QF>::NW)) void fa_dec(FaArg
         for (int k = 0; k < PPW; ++k) {
             const int p = wave + k * NW;
             if (p >= NPP) break;
+            if constexpr (QFQ) {
+                // the row's power of two: its largest element (Inf as the largest
+                // finite exponent) to [2^14, 2^15); then f16 hi + lo in the score
+                // operand's layout, VD neighbouring slots of one lane's 16 bytes (one
+                // wave per pair: with every wave converting all pairs the prologue
+                // took 19 k cycles, of 47 k in all on a nine-query q4_0 call)
+                float amax = 0.0f;
+#pragma unroll
+                for (int j = 0; j < VD; ++j) amax = fmaxf(amax, fabsf(x[k][j]));
+                const int e = min((int)(__float_as_uint(wave_max(amax)) >> 23), 254);
+                const int up = 141 - e;
+                const int el = (lane * VD) % kQK;  // in its block
+                const int slot = KT == XQ_TYPE_Q4_0 ? 8 * ((el % 16) / 4) + el / 16 * 4 + el % 4 : el;  // 8 lg + slot
+                uint8_t* op = sQ + ((p / 16) * NB + lane * VD / kQK) * 1024 + (slot / 8) * 256 + (p % 16) * 16 + (slot % 8) * 2;
+                uint32_t hb[VD], lb[VD];
+#pragma unroll
+                for (int j = 0; j < VD; ++j) {
+                    const float xv = __builtin_ldexpf(x[k][j], up);
+                    hb[j] = f32_to_f16_bits(xv);
+                    // an infinite element keeps a zero low part: its products stay infinite
+                    lb[j] = __builtin_isfinite(xv) ? f32_to_f16_bits(xv - f16_bits_to_f32(hb[j])) : 0u;
+                }
+#pragma unroll
+                for (int j = 0; j < VD; j += 2) {
+                    *(uint32_t*)(op + 2 * j) = hb[j] | (hb[j + 1] << 16);
+                    *(uint32_t*)(op + MT * NB * 1024 + 2 * j) = lb[j] | (lb[j + 1] << 16);
+                }
+                if (lane == 0) sQf[p] = __builtin_ldexpf(a.scale * kLog2e, -up);
+                continue;
+            }
             uint8_t* img = sQ + p * QRB;
             // ggml-cpu x86 quantize_row_q8_0: d = amax/127 (stored as f16),
             // id = 127/amax, q = round-half-even(x * id)
@@ -626,53 +664,25 @@ __global__ __launch_bounds__((64 * DecCfg<KT, D, MT, QF>::NW)) void fa_dec(FaArg
         for (int m = 0; m < MT; ++m) {
             const int p = 16 * m + lr;
             const int pp = p < npa ? p : 0;
-            const int qq = pp / a.G, h = g_kv * a.G + pp % a.G;
-            const float* src = (const float*)(a.q + (int64_t)b * a.q_nb3 + (int64_t)(iq0 + qq) * a.q_nb1 + (int64_t)h * a.q_nb2);
+            const float* src = (const float*)(a.q + (int64_t)b * a.q_nb3 + (int64_t)pair_q(pp) * a.q_nb1 + (int64_t)pair_h(pp) * a.q_nb2);
 #pragma unroll
             for (int c = 0; c < NB; ++c)
 #pragma unroll
-                for (int j = 0; j < 8; ++j)  // in K's order
-                    xq[m][c][j] = src[32 * c + (KT == XQ_TYPE_Q4_0 ? 4 * lg + 12 * (j >> 2) + j : 8 * lg + j)];
+                for (int j = 0; j < 8; ++j) xq[m][c][j] = src[32 * c + 8 * lg + j];
         }
 #pragma unroll
         for (int m = 0; m < MT; ++m) {
             const bool ok = 16 * m + lr < npa;
-            if constexpr (QUANT) {
-                // the row's power of two: its largest element (Inf as the largest
-                // finite exponent) to [2^14, 2^15)
-                float amax = 0.0f;
-#pragma unroll
-                for (int c = 0; c < NB; ++c)
-#pragma unroll
-                    for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(xq[m][c][j]));
-                const int e = min((int)(__float_as_uint(xrow_max(amax)) >> 23), 254);
-                const int up = 141 - e;
-                qf[m] = __builtin_ldexpf(a.scale * kLog2e, -up);
-#pragma unroll
-                for (int c = 0; c < NB; ++c)
-#pragma unroll
-                    for (int j = 0; j < 8; ++j) xq[m][c][j] = __builtin_ldexpf(xq[m][c][j], up);
-            }
 #pragma unroll
             for (int c = 0; c < NB; ++c) {
                 // Q = f16 hi + f16 lo (lo = 0 for the NATIVE policy); NaN as ggml's f16 conversion
-                h8 hi, lo;
 #pragma unroll
                 for (int j = 0; j < 8; ++j) {
                     const float xv = ok ? xq[m][c][j] : 0.0f;
                     const uint32_t hb = f32_to_f16_bits(xv);
-                    hi[j] = __builtin_bit_cast(_Float16, (uint16_t)hb);
-                    // (quantized K: an infinite element keeps a zero low part, so its
-                    // products stay infinite)
-                    lo[j] = HI_ONLY || (QUANT && !__builtin_isfinite(xv)) ? (_Float16)0.0f
+                    qh[m][c][j] = __builtin_bit_cast(_Float16, (uint16_t)hb);
+                    ql[m][c][j] = HI_ONLY ? (_Float16)0.0f
                                             : __builtin_bit_cast(_Float16, (uint16_t)f32_to_f16_bits(xv - f16_bits_to_f32(hb)));
-                }
-                if constexpr (!QUANT || !C::QHL) qh[m][c] = hi;
-                if constexpr (!QUANT) {
-                    ql[m][c] = lo;
-                } else if ((m * NB + c) % NW == wave) {  // every wave forms the same operands
-                    *(h8*)(sQ + (m * NB + c) * 1024 + 16 * lane) = lo;
-                    if constexpr (C::QHL) *(h8*)(sQ + ((MT + m) * NB + c) * 1024 + 16 * lane) = hi;
                 }
             }
         }
@@ -688,6 +698,11 @@ __global__ __launch_bounds__((64 * DecCfg<KT, D, MT, QF>::NW)) void fa_dec(FaArg
     // dqb[m][q]: d_q of block 4q + lg of the lane's pair (the B operand of the
     // 4-block scale product)
     float dqb[INTQ ? MT : 1][INTQ ? NB / 4 : 1];
+    float qf[MT];  // QFQ: the pair's score factor, scale * log2 e / its power of two
+    if constexpr (QFQ) {
+#pragma unroll
+        for (int m = 0; m < MT; ++m) qf[m] = sQf[16 * m + lr];
+    }
     if constexpr (INTQ) {
 #pragma unroll
         for (int m = 0; m < MT; ++m) {
@@ -712,7 +727,7 @@ __global__ __launch_bounds__((64 * DecCfg<KT, D, MT, QF>::NW)) void fa_dec(FaArg
     // q4_0 value operand half then takes one v_and_or (a VOP3 cannot hold it
     // as a literal)
     uint32_t k6400 = 0;
-    if constexpr (KT == XQ_TYPE_Q4_0 || (QUANT && QF)) asm("v_mov_b32 %0, 0x64006400" : "=v"(k6400));
+    if constexpr (KT == XQ_TYPE_Q4_0 || QFQ) asm("v_mov_b32 %0, 0x64006400" : "=v"(k6400));
 #pragma unroll
     for (int m = 0; m < MT; ++m)
 #pragma unroll
@@ -722,7 +737,7 @@ __global__ __launch_bounds__((64 * DecCfg<KT, D, MT, QF>::NW)) void fa_dec(FaArg
     auto scores = [&](auto st_tag, float (&s)[MT][4]) {
         constexpr int ST = decltype(st_tag)::value;
         const uint8_t* Ks = ring + ST * 2 * SLICE;
-        if constexpr (QUANT && QF) {
+        if constexpr (QFQ) {
 #pragma unroll
             for (int m = 0; m < MT; ++m)
 #pragma unroll
@@ -743,14 +758,9 @@ __global__ __launch_bounds__((64 * DecCfg<KT, D, MT, QF>::NW)) void fa_dec(FaArg
                     const h8 kf = k_block_f16<KT>(Ks + lr * REC, c0 + j, lg, k6400);
 #pragma unroll
                     for (int m = 0; m < MT; ++m) {
-                        h8 hi;
-                        if constexpr (C::QHL)
-                            hi = *(const h8*)(sQ + ((MT + m) * NB + c0 + j) * 1024 + 16 * lane);
-                        else
-                            hi = qh[m][c0 + j];
-                        f4 dot = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, hi, f4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
-                        const h8 lo = *(const h8*)(sQ + (m * NB + c0 + j) * 1024 + 16 * lane);
-                        dot = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, lo, dot, 0, 0, 0);
+                        const uint8_t* op = sQ + (m * NB + c0 + j) * 1024 + 16 * lane;
+                        f4 dot = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, *(const h8*)op, f4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+                        dot = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, *(const h8*)(op + MT * NB * 1024), dot, 0, 0, 0);
 #pragma unroll
                         for (int i = 0; i < 4; ++i) s[m][i] = fmaf(dot[i], dks[m][4 * j + i], s[m][i]);
                     }
@@ -995,7 +1005,7 @@ __global__ __launch_bounds__((64 * DecCfg<KT, D, MT, QF>::NW)) void fa_dec(FaArg
         // V_j, then (when slice j+1 exists) K_j+1 + mask_j+1 and V_j+1; loads
         // complete in order
         if (n1)
-            asm volatile("s_waitcnt vmcnt(%0)" ::"n"(3 * NIS + 2 * MT) : "memory");
+            asm volatile("s_waitcnt vmcnt(%0)" ::"n"(3 * NIS + ML) : "memory");
         else
             asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NIS) : "memory");
         __builtin_amdgcn_wave_barrier();
@@ -1008,8 +1018,8 @@ __global__ __launch_bounds__((64 * DecCfg<KT, D, MT, QF>::NW)) void fa_dec(FaArg
         const uint8_t* ms = mring + S * MT * 512 + 4 * lane;
 #pragma unroll
         for (int m = 0; m < MT; ++m) {
-            mw[m][0] = lds_u32(ms + m * 512);
-            mw[m][1] = lds_u32(ms + m * 512 + 256);
+            mw[m][0] = QFQ ? 0u : lds_u32(ms + m * 512);
+            mw[m][1] = QFQ ? 0u : lds_u32(ms + m * 512 + 256);
         }
         if (n2) {
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // K and mask reads of this stage done
@@ -1018,9 +1028,9 @@ __global__ __launch_bounds__((64 * DecCfg<KT, D, MT, QF>::NW)) void fa_dec(FaArg
 
         // -- V_j complete: later units K_j+1 + mask, V_j+1, K_j+2 + mask
         if (n2)
-            asm volatile("s_waitcnt vmcnt(%0)" ::"n"(3 * NIS + 4 * MT) : "memory");
+            asm volatile("s_waitcnt vmcnt(%0)" ::"n"(3 * NIS + 2 * ML) : "memory");
         else if (n1)
-            asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * NIS + 2 * MT) : "memory");
+            asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * NIS + ML) : "memory");
         else
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __builtin_amdgcn_wave_barrier();
@@ -1091,7 +1101,7 @@ __global__ __launch_bounds__((64 * DecCfg<KT, D, MT, QF>::NW)) void fa_dec(FaArg
             for (int i = 0; i < 4; ++i) {
                 const h2 mh = __builtin_bit_cast(h2, mw[m][i >> 1]);
                 const float v = SOFTCAP ? cap2 * tanhf(s[m][i] * a.scale) : QUANT ? s[m][i] : s[m][i] * sc2;
-                x[m][i] = fmaf(slope2[m], (float)mh[i & 1], v);
+                x[m][i] = QFQ ? v : fmaf(slope2[m], (float)mh[i & 1], v);
             }
             // a sum of finite scores (|x| far below the f32 range) is finite
             // exactly when every score is: one test for -inf, +inf and NaN
@@ -1107,7 +1117,7 @@ __global__ __launch_bounds__((64 * DecCfg<KT, D, MT, QF>::NW)) void fa_dec(FaArg
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     const h2 mh = __builtin_bit_cast(h2, mw[m][i >> 1]);
-                    const bool seen = t + 4 * lg + i < lim[m] && (float)mh[i & 1] != -INFINITY;
+                    const bool seen = t + 4 * lg + i < lim[m] && (QFQ || (float)mh[i & 1] != -INFINITY);
                     x[m][i] = seen ? x[m][i] : -INFINITY;
                 }
         }
@@ -1368,7 +1378,7 @@ __global__ __launch_bounds__((64 * DecCfg<KT, D, MT, QF>::NW)) void fa_dec(FaArg
                 Ls = fmaf(sL[w][p], ew, Ls);
                 o += ew * *(const f4*)(mb + w * WST + pl * MS + 4 * d4);
             }
-            const int qq = p / a.G, h = g_kv * a.G + p % a.G, iq = iq0 + qq;
+            const int iq = pair_q(p), h = pair_h(p);
             const int64_t row = (int64_t)b * rows_per_seq + (int64_t)iq * a.H + h;
             const float Mn = M == -INFINITY ? -INFINITY : M * kLn2;  // natural-log units
             if (a.n_splits == 1) {
@@ -1474,7 +1484,14 @@ bool fa_mma_mask_ok(const FaArgs& a) {
 hipError_t fa_mma_launch(FaArgs a, const FaLaunch& L, hipStream_t stream) {
     const int D = (int)L.q->ne[0];
     const int kt = L.k->type;
-    const int mt = (a.QT * a.G + 15) / 16;
+    // tiles of 16 or 32 (query, head) pairs, packed across queries: 9 queries of 6
+    // heads are 4 tiles of 16 pairs (whole queries per tile: 5)
+    const int n_pairs = a.NQ * a.G, max_pairs = fa_max_pairs(D, a.G);
+    const int mt = (min(n_pairs, max_pairs) + 15) / 16;
+    a.n_qtiles = (n_pairs + 16 * mt - 1) / (16 * mt);
+    // x / G = mulhi(x, floor(2^32 / G) + 1) for x below 2^32 / G (0: G is 1)
+    a.g_magic = a.G > 1 ? (uint32_t)(((uint64_t)1 << 32) / a.G) + 1u : 0u;
+    if ((uint64_t)(n_pairs + 32) * a.G >= (uint64_t)1 << 31) return hipErrorInvalidValue;
     if (!fa_mma_rows_ok(a.L)) return hipErrorInvalidValue;
     a.hi_only = is_quant(kt) ? 0 : (L.q_round_f16 ? 1 : 0);
     int waves = 0;
