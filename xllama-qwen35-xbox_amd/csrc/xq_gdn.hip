@@ -6,7 +6,7 @@
 // each lane holds 8 elements as two float4 at i = 4*li + 64*r (r = 0, 1), so a
 // row's state read/write is two fully coalesced 256-byte transactions. Both
 // column dot products reduce inside the DPP row (4 steps, no LDS, no barrier).
-// A 256-thread workgroup covers 128 columns of one (sequence, v-head); tokens
+// A 256-thread workgroup covers 16 to 128 columns of one (sequence, v-head); tokens
 // run chronologically with the state in registers, so the state is read once
 // and each kept snapshot written once.
 #include "xq_kernels.h"
@@ -182,20 +182,43 @@ __global__ __launch_bounds__(256) void gdn_step_kernel(GdnStepArgs a) {
     }
 }
 
-// Eight columns per row: one 256-thread workgroup owns all 128 columns (64 KB
-// of state) of one (sequence, v-head), so the whole state read is in flight at
-// once; with 8 sequences x 32 heads that is one workgroup per CU. Measured
-// against one, two and four columns per row at 8 sequences x 32 heads, eight
-// was fastest (6.5 us per call against 7.1 us for four).
-constexpr int kStepCpt = 8;
+template <bool BF16, bool VEC, int CPT>
+static void step_launch(const GdnStepArgs& a, hipStream_t stream) {
+    const dim3 grid(a.B * 32 * (128 / (16 * CPT)));
+    if (a.T == 1)
+        launch("gdn_step", gdn_step_kernel<BF16, VEC, CPT, true>, grid, dim3(256), stream, a);
+    else
+        launch("gdn_step", gdn_step_kernel<BF16, VEC, CPT, false>, grid, dim3(256), stream, a);
+}
+
+// Columns per 16-lane row. With eight, one 256-thread workgroup owns all 128
+// columns (64 KB of state) of a (sequence, v-head), so its whole state read is in
+// flight at once; 8 sequences x 32 heads are one workgroup per CU. A single token
+// is bound by that traffic: 8 sequences take 5.7 us per call with eight columns,
+// 5.8-6.8 us with two or four, 6 sequences 5.2 us with two against 5.4 us. Several
+// tokens are bound by the chain of a row's columns, run one after another for
+// every token, and by CUs that hold no workgroup: fewer columns per row pay until
+// the rows' repeated loads of q and k do not (us per call, f32 rows, with 1 / 2 / 4
+// / 8 columns):
+//   1 sequence, 5 tokens and their snapshots   5.3  5.9  7.6 10.9
+//   4 sequences, 5 tokens                     11.6  9.4  9.0 11.3
+//   1 sequence, 40 tokens                     15.7 21.9 32.9 55.3
+//   8 sequences, 40 tokens                    52.9 38.8 41.6 59.7
+//   16 sequences, 40 tokens (bf16 rows)        110   80   86   75
+static int step_columns(int T, int B) {
+    if (T == 1) return B <= 6 ? 2 : 8;
+    if (T <= 8) return B <= 1 ? 1 : B <= 4 ? 2 : B <= 12 ? 4 : 8;
+    return B <= 3 ? 1 : B <= 8 ? 2 : B <= 12 ? 4 : 8;
+}
 
 template <bool BF16, bool VEC>
 static void step_dispatch(const GdnStepArgs& a, hipStream_t stream) {
-    const dim3 grid(a.B * 32 * (128 / (16 * kStepCpt)));
-    if (a.T == 1)
-        launch("gdn_step", gdn_step_kernel<BF16, VEC, kStepCpt, true>, grid, dim3(256), stream, a);
-    else
-        launch("gdn_step", gdn_step_kernel<BF16, VEC, kStepCpt, false>, grid, dim3(256), stream, a);
+    switch (step_columns(a.T, a.B)) {
+    case 1: step_launch<BF16, VEC, 1>(a, stream); break;
+    case 2: step_launch<BF16, VEC, 2>(a, stream); break;
+    case 4: step_launch<BF16, VEC, 4>(a, stream); break;
+    default: step_launch<BF16, VEC, 8>(a, stream); break;
+    }
 }
 
 hipError_t gdn_step_launch(const GdnLaunch& L, hipStream_t stream) {
