@@ -17,46 +17,32 @@
 //
 // Two kernels:
 //   gdn_chunk_prep  one workgroup per (sequence, k-head, chunk), all chunks in
-//                   parallel, for the two v-heads that share the k-head: K K^T on
-//                   f16 MFMA once (f32 accumulation) and, per v-head, the unit
-//                   lower-triangular inverse for T in f32 (by 16 x 16 blocks,
-//                   the products on f32 MFMA); stores T as f16 hi + lo
-//                   planes, the decay vectors, the cumulative log-decays G,
-//                   the chunk's largest |v| per 16-column block and, for bf16
-//                   rows read as 16-byte words, the P tiles (f16 hi + lo; 27 KB
-//                   per chunk) in the workspace. f32 k rows enter as f16 hi + lo
-//                   (the products take hi*hi + hi*lo + lo*hi); bf16 rows enter
-//                   as f16 (their 8 significant bits fit; a bf16 value below
-//                   2^-14 keeps an absolute precision of 2^-25 there, not its
-//                   relative one), or as bf16 on bf16 MFMA when read as
-//                   16-byte words (exact).
-//   gdn_chunk_scan  one workgroup per (sequence, v-head, 16 value columns) runs
-//                   the chunks in order with its 128 x 16 state block in
-//                   registers (f32). Every MFMA operand that does not depend on
-//                   the state (K and Q rows straight from the inputs, as f16,
-//                   or f16 hi + lo for f32 rows; T rows from the workspace; V,
-//                   the decays and G) is loaded into registers a chunk ahead,
-//                   in four parts spread over the chunk's phases. K^T is formed
-//                   in the scan from the K rows it already holds (the waves
-//                   share them through LDS: written transposed, or for bf16
-//                   rows read as 16-byte words written as loaded and read
-//                   with gfx950's transposing LDS read), which keeps 16 KB per
-//                   chunk out of every workgroup's operand fetch. P is formed
-//                   by the prep for bf16 rows read as 16-byte words (10 KB per
-//                   chunk, off the scan's chain; its products and decays are
-//                   the scan's own), and by the scan from its K and Q rows
-//                   (shared through LDS) otherwise. LDS otherwise
-//                   carries the state-dependent exchanges (S^T, X^T, U^T). The products run
-//                   on f16 MFMA with f32 operands split into f16 hi + lo (about
-//                   22 significant bits), so the result stays within
-//                   f32-recurrence tolerances. bf16 rows read as 16-byte words
-//                   skip the f16 conversion: they are the operands of bf16
-//                   MFMAs as loaded, and the f32 operands that meet them (the
-//                   state, e^{G_C - G} U) enter as three bf16 terms hi + mid + lo,
-//                   which hold the f32 value exactly; 30 % fewer VALU
-//                   instructions and 6 % less time per scan than the f16 form.
-// The 8 column blocks of a head run on one XCD (consecutive logical workgroups)
+//                   parallel, for the two v-heads that share the k-head: K K^T
+//                   and Q K^T once on the matrix cores (f32 accumulation) and, per
+//                   v-head, the unit lower-triangular inverse for T in f32 (by
+//                   16 x 16 blocks, the products on f32 MFMA); stores T and the P
+//                   tiles as f16 hi + lo, the decay vectors and
+//                   the chunk's largest |v| per 16-column block in the workspace
+//                   (27 KB per chunk and v-head). bf16 rows are
+//                   operands of bf16 MFMA as they are (exact); f32 rows enter f16
+//                   MFMA as hi + lo (the products take hi*hi + hi*lo + lo*hi).
+//   gdn_chunk_scan  one workgroup per (sequence, v-head, NC tiles of 16 value
+//                   columns) runs the chunks in order with its 128 x 16 NC state
+//                   block in registers (f32). Every MFMA operand that does not
+//                   depend on the state (K and Q rows, T and P from the workspace,
+//                   V, the decays) is loaded into registers a chunk ahead, in
+//                   four parts spread over the chunk's phases. The state update
+//                   reads K^T from the chunk's K rows in LDS with gfx950's
+//                   transposing LDS read. LDS otherwise carries the
+//                   state-dependent exchanges (S^T, X^T, U^T), every f32 value as
+//                   f16 hi + lo (about 22 significant bits), or, where it meets
+//                   bf16 rows (the state, e^{G_C - G} U), as three bf16 terms
+//                   hi + mid + lo, which hold it exactly.
+// The column groups of a head run on one XCD (consecutive logical workgroups)
 // so the chunk rows and T, P they share are read from HBM once.
+//
+// Against forming P and converting and transposing f32 rows in the scan: 1531 f32
+// tokens of one sequence 144 -> 100 us per call.
 //
 // Range. The recurrence is linear in (V, S): the scan runs on V and S times a
 // power of two 2^a per (sequence, v-head, column block), chosen from the largest
@@ -64,7 +50,7 @@
 // that they lie in [1, 2), and divides Y and the final state by 2^a (exact). V
 // and the state may so have any finite f32 magnitude: f16's range holds a state
 // that grows 2^15-fold beyond them. q and k rows enter as f16 (or hi + lo) and
-// meet in f16 planes (the P tiles): the prep records per chunk whether they
+// meet in the f16 P tiles: the prep records per chunk whether they
 // lie in the range those operands hold (qk_in_range: |k| < 16, |q| < 2^15,
 // |q| |k| < 256 per element, finite; L2-normalised rows lie far inside) and
 // whether every decay e^g lies in [0, 1] and beta is finite (g finite and at
@@ -93,11 +79,10 @@ constexpr int kColBlocks = 128 / kCols;
 // write neighbouring records.
 constexpr int kRecTHi = 0;                       // f16 [64][64]
 constexpr int kRecTLo = kRecTHi + 64 * 64 * 2;
-constexpr int kRecDec = kRecTLo + 64 * 64 * 2;  // f32 e^G[64], e^{G_C - G}[64], e^{G_C}, range flag at 129, max|v|[8] at 136, G[64] at 192
-constexpr int kRecG = 192;                      // G offset in floats within the decays
+constexpr int kRecDec = kRecTLo + 64 * 64 * 2;  // f32 e^G[64], e^{G_C - G}[64], e^{G_C}, range flag at 129, max|v|[8] at 136
 constexpr int kRecVmax = 136;                   // largest |v| of the chunk per 16-column block (floats)
 constexpr int kRecRange = 129;                  // 1.0f when the chunk's q / k leave the operands' range, else 0
-// P tiles (bf16 rows with 16-byte loads): tile (w, jt), jt <= w, of scan wave w
+// P tiles: tile (w, jt), jt <= w, of scan wave w
 // is 1 KB at kRecP + (w (w + 1) / 2 + jt) KB; lane l's 16 bytes at 16 l are its
 // four values of P[16w + l % 16][16jt + 4(l / 16) + i] as f16 hi, then f16 lo
 constexpr int kRecP = kRecDec + 1024;
@@ -130,12 +115,20 @@ struct GdnChunkArgs {
 XQ_DEV _Float16 f16_hi(float x) { return (_Float16)x; }
 XQ_DEV _Float16 f16_lo(float x) { return (_Float16)(x - (float)(_Float16)x); }
 
-// Eight consecutive elements of an input row (bf16 or f32) as f32; VEC reads
-// them with 16-byte loads (the host checks the alignment).
+// Row words as the caller's strides leave them: 16-byte loads that need no more
+// than the elements' alignment.
+typedef uint32_t w4_f32 __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t w4_bf16 __attribute__((ext_vector_type(4), aligned(2)));
+
+XQ_DEV uint4 ld_words_f32(const uint8_t* p) { return __builtin_bit_cast(uint4, *(const w4_f32*)p); }
+XQ_DEV uint4 ld_words_bf16(const uint8_t* p) { return __builtin_bit_cast(uint4, *(const w4_bf16*)p); }
+
+// Eight consecutive elements of an input row (bf16 or f32) as f32; VEC reads them
+// as 16-byte words, else element by element.
 template <bool BF16, bool VEC>
 XQ_DEV void load8(const uint8_t* row, int i0, float (&x)[8]) {
     if constexpr (VEC && BF16) {
-        const uint4 w = *(const uint4*)(row + 2 * i0);
+        const uint4 w = ld_words_bf16(row + 2 * i0);
         const uint32_t u[4] = {w.x, w.y, w.z, w.w};
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
@@ -143,15 +136,31 @@ XQ_DEV void load8(const uint8_t* row, int i0, float (&x)[8]) {
             x[2 * e + 1] = bf16_bits_to_f32(u[e] >> 16);
         }
     } else if constexpr (VEC) {
-        const float4 a = *(const float4*)(row + 4 * i0);
-        const float4 b = *(const float4*)(row + 4 * i0 + 16);
-        x[0] = a.x; x[1] = a.y; x[2] = a.z; x[3] = a.w;
-        x[4] = b.x; x[5] = b.y; x[6] = b.z; x[7] = b.w;
+        const uint4 w0 = ld_words_f32(row + 4 * i0), w1 = ld_words_f32(row + 4 * i0 + 16);
+        const uint32_t u[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] = __uint_as_float(u[e]);
     } else {
 #pragma unroll
-        for (int e = 0; e < 8; ++e)
-            x[e] = BF16 ? bf16_bits_to_f32(((const uint16_t*)row)[i0 + e]) : ((const float*)row)[i0 + e];
+        for (int e = 0; e < 8; ++e) x[e] = BF16 ? bf16_bits_to_f32(((const uint16_t*)row)[i0 + e]) : ((const float*)row)[i0 + e];
     }
+}
+
+// f32 words x0 .. x3 as f16 high parts and remainders, pairs (0, 1) and (2, 3): the
+// remainder x - hi is exact in f32. s_nop: the two wait states an MFMA needs after a
+// VALU write that the compiler's hazard tracking does not see.
+XQ_DEV void f16_split4(uint4 x, uint32_t& h01, uint32_t& h23, uint32_t& l01, uint32_t& l23) {
+    asm("v_fma_mixlo_f16 %0, %4, 1.0, 0 op_sel:[0,0,0] op_sel_hi:[0,0,0]\n\t"
+        "v_fma_mixhi_f16 %0, %5, 1.0, 0 op_sel:[0,0,0] op_sel_hi:[0,0,0]\n\t"
+        "v_fma_mixlo_f16 %1, %6, 1.0, 0 op_sel:[0,0,0] op_sel_hi:[0,0,0]\n\t"
+        "v_fma_mixhi_f16 %1, %7, 1.0, 0 op_sel:[0,0,0] op_sel_hi:[0,0,0]\n\t"
+        "v_fma_mixlo_f16 %2, %4, 1.0, -%0 op_sel:[0,0,0] op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixhi_f16 %2, %5, 1.0, -%0 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixlo_f16 %3, %6, 1.0, -%1 op_sel:[0,0,0] op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixhi_f16 %3, %7, 1.0, -%1 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
+        "s_nop 1"
+        : "=&v"(h01), "=&v"(h23), "=&v"(l01), "=&v"(l23)
+        : "v"(x.x), "v"(x.y), "v"(x.z), "v"(x.w));
 }
 
 XQ_DEV h8 to_h8(const float (&x)[8]) {
@@ -232,7 +241,7 @@ XQ_DEV uint32_t wave_max_u32(uint32_t v) {
 
 // ---------------------------------------------------------------- prep
 
-template <bool BF16, bool VEC>
+template <bool BF16>
 __global__ __launch_bounds__(256, BF16 ? 2 : 1) void gdn_chunk_prep(GdnChunkArgs a) {
     constexpr int KP = 136;  // padded f16 row stride (halves)
     constexpr int FP = 68;   // padded f32 row stride (16-byte rows, conflict-free MFMA stores)
@@ -248,10 +257,9 @@ __global__ __launch_bounds__(256, BF16 ? 2 : 1) void gdn_chunk_prep(GdnChunkArgs
     __shared__ __attribute__((aligned(16))) _Float16 sKl[NKL];
     static_assert(64 * FP * 4 <= 64 * KP * 2, "LDS aliases");
 
-    // bf16 rows read as 16-byte words (RAW): K and Q stay bf16 in LDS and the
-    // products run on bf16 MFMA (exact operands); the P tiles are formed here
-    constexpr bool RAW = BF16 && VEC;
-    _Float16* sQ = (_Float16*)sKK;  // RAW: Q [t][i] until the products are done
+    // bf16 rows: K and Q stay bf16 in LDS and the products run on bf16 MFMA
+    // (exact operands). f32 rows: f16 hi + lo
+    _Float16* sQ = (_Float16*)sKK;  // bf16 rows: Q [t][i] until the products are done
     static_assert(64 * FP * 4 >= 64 * KP * 2, "Q rows fit the L buffer");
 
     // v-heads kh and kh + 16 share k-head kh: K K^T is formed once for both.
@@ -262,15 +270,16 @@ __global__ __launch_bounds__(256, BF16 ? 2 : 1) void gdn_chunk_prep(GdnChunkArgs
     const int wave = wave_id(), lane = lane_id(), lr = lane & 15, lg = lane >> 4;
     const int t0 = n * kChunk;
 
-    // ---- chunk rows -> LDS as f16 (tokens past T are zero, with g = beta = 0):
-    //      thread = (token, quarter of 32 elements), 8 elements per load
+    // ---- chunk rows -> LDS as bf16, or f16 hi + lo (tokens past T are zero, with
+    //      g = beta = 0): thread = (token, quarter of 32 elements), 8 elements per load
+    h8 qhi[BF16 ? 1 : 4], qlo[BF16 ? 1 : 4];  // f32 rows: Q of row 16w + lr
     {
         const int t = tid >> 2, qt = tid & 3;
         const int tg = t0 + t;
         const bool ok = tg < a.T;
         const uint8_t* kr = a.k + (int64_t)b * a.k_nb3 + (int64_t)tg * a.k_nb2 + (int64_t)kh * a.k_nb1;
         uint32_t kmx = 0, qmx = 0;  // the largest |k|, |q| of the thread's elements (f32 bits)
-        if constexpr (RAW) {
+        if constexpr (BF16) {
             // rows past T: loads of row T - 1, zeroed (no conditional loads)
             const int tc = min(tg, a.T - 1);
             const uint8_t* kc = a.k + (int64_t)b * a.k_nb3 + (int64_t)tc * a.k_nb2 + (int64_t)kh * a.k_nb1;
@@ -278,47 +287,56 @@ __global__ __launch_bounds__(256, BF16 ? 2 : 1) void gdn_chunk_prep(GdnChunkArgs
             uint4 wk[4], wq[4];
 #pragma unroll
             for (int gi = 0; gi < 4; ++gi) {
-                wk[gi] = *(const uint4*)(kc + 2 * (32 * qt + 8 * gi));
-                wq[gi] = *(const uint4*)(qc + 2 * (32 * qt + 8 * gi));
+                wk[gi] = ld_words_bf16(kc + 2 * (32 * qt + 8 * gi));
+                wq[gi] = ld_words_bf16(qc + 2 * (32 * qt + 8 * gi));
             }
             const uint32_t m = ok ? ~0u : 0u;  // a mask, not a select of the arrays
 #pragma unroll
             for (int gi = 0; gi < 4; ++gi) {
-                const uint4 x = wk[gi], y = wq[gi];
-                *(uint4*)(sK + t * KP + 32 * qt + 8 * gi) = make_uint4(x.x & m, x.y & m, x.z & m, x.w & m);
-                *(uint4*)(sQ + t * KP + 32 * qt + 8 * gi) = make_uint4(y.x & m, y.y & m, y.z & m, y.w & m);
-                kmx = bf16x2_absmax(bf16x2_absmax(bf16x2_absmax(bf16x2_absmax(kmx, x.x & m), x.y & m), x.z & m), x.w & m);
-                qmx = bf16x2_absmax(bf16x2_absmax(bf16x2_absmax(bf16x2_absmax(qmx, y.x & m), y.y & m), y.z & m), y.w & m);
+                const uint4 x = make_uint4(wk[gi].x & m, wk[gi].y & m, wk[gi].z & m, wk[gi].w & m);
+                const uint4 y = make_uint4(wq[gi].x & m, wq[gi].y & m, wq[gi].z & m, wq[gi].w & m);
+                const int i0 = 32 * qt + 8 * gi;
+                *(uint4*)(sK + t * KP + i0) = x;
+                *(uint4*)(sQ + t * KP + i0) = y;
+                kmx = bf16x2_absmax(bf16x2_absmax(bf16x2_absmax(bf16x2_absmax(kmx, x.x), x.y), x.z), x.w);
+                qmx = bf16x2_absmax(bf16x2_absmax(bf16x2_absmax(bf16x2_absmax(qmx, y.x), y.y), y.z), y.w);
             }
             kmx = bf16x2_max_bits(kmx);
             qmx = bf16x2_max_bits(qmx);
-        }
+        } else {
 #pragma unroll
-        for (int gi = 0; gi < 4; ++gi) {
-            if constexpr (RAW) break;
-            const int i0 = 32 * qt + 8 * gi;
-            float xk[8];
-            if (ok) {
-                load8<BF16, VEC>(kr, i0, xk);
-            } else {
+            for (int gi = 0; gi < 4; ++gi) {
+                const int i0 = 32 * qt + 8 * gi;
+                float xk[8];
+                if (ok) {
+                    load8<BF16, true>(kr, i0, xk);
+                } else {
 #pragma unroll
-                for (int e = 0; e < 8; ++e) xk[e] = 0.0f;
+                    for (int e = 0; e < 8; ++e) xk[e] = 0.0f;
+                }
+                const h8 hk = to_h8(xk), lk = lo_h8(xk, hk);
+                *(h8*)(sK + t * KP + i0) = hk;
+                *(h8*)(sKl + t * KP + i0) = lk;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) kmx = max(kmx, __float_as_uint(xk[e]) & 0x7fffffffu);
             }
-            const h8 hk = to_h8(xk);
-            *(h8*)(sK + t * KP + i0) = hk;
-            if constexpr (!BF16) *(h8*)(sKl + t * KP + i0) = lo_h8(xk, hk);
-            // q rows, read here for their range only (the scan forms P from them)
-            float xq[8];
-            if (ok) {
-                load8<BF16, VEC>(a.q + (int64_t)b * a.q_nb3 + (int64_t)tg * a.q_nb2 + (int64_t)kh * a.q_nb1, i0, xq);
-            } else {
+            // q rows in the layout of P's B operand: row 16w + lr, no LDS
+            const int tq = 16 * wave + lr;
+            const uint8_t* qr = a.q + (int64_t)b * a.q_nb3 + (int64_t)(t0 + tq) * a.q_nb2 + (int64_t)kh * a.q_nb1;
 #pragma unroll
-                for (int e = 0; e < 8; ++e) xq[e] = 0.0f;
-            }
+            for (int ks = 0; ks < 4; ++ks) {
+                const int i0 = 32 * ks + 8 * lg;
+                float xq[8];
+                if (t0 + tq < a.T) {
+                    load8<BF16, true>(qr, i0, xq);
+                } else {
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                kmx = max(kmx, __float_as_uint(xk[e]) & 0x7fffffffu);
-                qmx = max(qmx, __float_as_uint(xq[e]) & 0x7fffffffu);
+                    for (int e = 0; e < 8; ++e) xq[e] = 0.0f;
+                }
+                qhi[ks] = to_h8(xq);
+                qlo[ks] = lo_h8(xq, qhi[ks]);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) qmx = max(qmx, __float_as_uint(xq[e]) & 0x7fffffffu);
             }
         }
         // largest |v| of the token's 32 columns 32qt.. (two column blocks) for
@@ -382,7 +400,7 @@ __global__ __launch_bounds__(256, BF16 ? 2 : 1) void gdn_chunk_prep(GdnChunkArgs
         const int tile = wave * 4 + tt;
         const int mt = tile >> 2, nt = tile & 3;
         kk[tt] = f4{0.0f, 0.0f, 0.0f, 0.0f};
-        if constexpr (RAW) {
+        if constexpr (BF16) {
 #pragma unroll
             for (int ks = 0; ks < 4; ++ks)
                 kk[tt] = mfma_bf(*(const uint4*)(sK + (mt * 16 + lr) * KP + ks * 32 + 8 * lg),
@@ -394,7 +412,7 @@ __global__ __launch_bounds__(256, BF16 ? 2 : 1) void gdn_chunk_prep(GdnChunkArgs
             const h8 bk = *(const h8*)(sK + (nt * 16 + lr) * KP + ks * 32 + 8 * lg);
             const h8 ak = *(const h8*)(sK + (mt * 16 + lr) * KP + ks * 32 + 8 * lg);
             kk[tt] = mfma32(ak, bk, kk[tt]);
-            if constexpr (!BF16) {
+            {
                 const h8 bkl = *(const h8*)(sKl + (nt * 16 + lr) * KP + ks * 32 + 8 * lg);
                 const h8 akl = *(const h8*)(sKl + (mt * 16 + lr) * KP + ks * 32 + 8 * lg);
                 kk[tt] = mfma32(ak, bkl, kk[tt]);
@@ -402,18 +420,25 @@ __global__ __launch_bounds__(256, BF16 ? 2 : 1) void gdn_chunk_prep(GdnChunkArgs
             }
         }
     }
-    // RAW: P^T = K Q^T for the scan wave w's tiles (token tile w of q, tiles
-    // jt <= w of k), the products the scan would form: lane (lr, lg) holds
-    // q_t . k_j for t = 16w + lr, j = 16jt + 4lg + i
+    // P^T = K Q^T for the scan wave w's tiles (token tile w of q, tiles jt <= w
+    // of k): lane (lr, lg) holds q_t . k_j for t = 16w + lr, j = 16jt + 4lg + i
     f4 pq[4];
 #pragma unroll
     for (int jt = 0; jt < 4; ++jt) {
         pq[jt] = f4{0.0f, 0.0f, 0.0f, 0.0f};
-        if (RAW && jt <= wave) {  // wave-uniform
+        if (jt <= wave) {  // wave-uniform
 #pragma unroll
-            for (int ks = 0; ks < 4; ++ks)
-                pq[jt] = mfma_bf(*(const uint4*)(sK + (16 * jt + lr) * KP + 32 * ks + 8 * lg),
-                                 *(const uint4*)(sQ + (16 * wave + lr) * KP + 32 * ks + 8 * lg), pq[jt]);
+            for (int ks = 0; ks < 4; ++ks) {
+                const int ko = (16 * jt + lr) * KP + 32 * ks + 8 * lg;
+                if constexpr (BF16) {
+                    pq[jt] = mfma_bf(*(const uint4*)(sK + ko), *(const uint4*)(sQ + (16 * wave + lr) * KP + 32 * ks + 8 * lg), pq[jt]);
+                } else {
+                    const h8 kj = *(const h8*)(sK + ko);
+                    pq[jt] = mfma32(kj, qhi[ks], pq[jt]);
+                    pq[jt] = mfma32(kj, qlo[ks], pq[jt]);
+                    pq[jt] = mfma32(*(const h8*)(sKl + ko), qhi[ks], pq[jt]);
+                }
+            }
         }
     }
     __syncthreads();  // K and Q no longer read; G ready
@@ -508,7 +533,7 @@ __global__ __launch_bounds__(256, BF16 ? 2 : 1) void gdn_chunk_prep(GdnChunkArgs
         }
         __syncthreads();
 
-        // ---- the record: T (f16 hi + lo) with 16-byte stores, the decays and G
+        // ---- the record: T (f16 hi + lo) with 16-byte stores, the decays
         uint8_t* rec = a.ws + (((int64_t)b * a.n_chunks + n) * 32 + h) * kRecBytes;
         {
             const int t = tid >> 2, j0 = 16 * (tid & 3);
@@ -531,12 +556,11 @@ __global__ __launch_bounds__(256, BF16 ? 2 : 1) void gdn_chunk_prep(GdnChunkArgs
             float* dec = (float*)(rec + kRecDec);
             dec[tid] = __expf(G);
             dec[64 + tid] = __expf(GC - G);
-            dec[kRecG + tid] = G;
             if (tid == 0) dec[128] = __expf(GC);
             if (tid == 1) dec[kRecRange] = qk_in_range(sQKmax[0], sQKmax[1]) && !sGBout[e2] ? 0.0f : 1.0f;
             if (tid < kColBlocks) dec[kRecVmax + tid] = __uint_as_float(sVmax[e2][tid]);
         }
-        if constexpr (RAW) {  // P[t][j] = (q_t . k_j) e^{G_t - G_j} (j <= t), f16 hi + lo
+        {  // P[t][j] = (q_t . k_j) e^{G_t - G_j} (j <= t), f16 hi + lo
             uint8_t* pr = rec + 16 * lane;
             const float gt = sEG[e2][16 * wave + lr];
 #pragma unroll
@@ -560,84 +584,35 @@ __global__ __launch_bounds__(256, BF16 ? 2 : 1) void gdn_chunk_prep(GdnChunkArgs
 
 // ---------------------------------------------------------------- scan
 
+// Column tiles of a scan workgroup. Lane lr of a 16-column operand tile ct holds
+// value column 16 NC cb + NC lr + ct, so a lane's NC columns are neighbours (one
+// load of V, one store of Y) and lie in one 16-column block of the prep's maxima.
+// V words of a lane's NC columns in one token
+template <bool F32, int NC> struct VWords { using T = std::conditional_t<NC == 1, uint32_t, uint2>; };
+template <> struct VWords<false, 1> { using T = uint16_t; };
+template <> struct VWords<false, 2> { using T = uint32_t; };
+
 // Operands of one chunk for one wave of a scan workgroup, loaded a chunk ahead:
 // A operands (row 16w + lr of the wave's token tile, k = 32 ks + 8 lg .. +7) of
-// K and Q (raw input words, decoded when used) and of T (hi, lo); the raw V
-// values and e^G, e^{G_C - G} of the lane's four tokens 16w + 4lg + r (column
-// 16cb + lr), e^{G_C}; for bf16 rows read as 16-byte words the wave's P tiles
-// from the record, otherwise the G values the scan's P needs (token 16w + lr,
-// tokens 16jt + 4lg + i). The loads are unconditional but for the P tiles (one
-// per tile jt <= w, a count fixed per wave): token and chunk indices are
-// clamped into range and out-of-range tokens masked at use, so the compiler's
-// waits for a chunk's operands never include the next chunk's loads.
-template <bool BF16, bool VEC>
+// K and Q (raw words) and of T (hi, lo); the raw V
+// values and e^G, e^{G_C - G} of the lane's four tokens 16w + 4lg + r, e^{G_C};
+// the wave's P tiles from the record. The loads are unconditional but for the P
+// tiles (one per tile jt <= w, a count fixed per wave): chunk indices are clamped
+// into range and out-of-range tokens masked at use, so the compiler's waits for
+// a chunk's operands never include the next chunk's loads.
+template <bool F32, int NC>
 struct ScanOps {
-    static constexpr int KW = VEC ? (BF16 ? 1 : 2) : 4;  // 16-byte words per 8 elements (VEC), else raw dwords
-    uint4 kw[4][KW], qw[4][KW];
-    uint4 pw[4];  // bf16 rows with 16-byte loads: the wave's P tiles (w, jt <= w) from the record
+    static constexpr int NK = F32 ? 2 : 1;  // 16-byte words per 8 elements
+    uint4 kw[4][NK], qw[4][NK];
+    uint4 pw[4];
     h8 th[2], tl[2];
     // raw V words, in the input's width: a 16-bit load widened at use (widened
     // here, the compiler copies the value at the loop edge and waits for it)
-    std::conditional_t<BF16, uint16_t, uint32_t> vw[4];
+    typename VWords<F32, NC>::T vw[4];
     float4 eg, egc;
     float eGC;
-    float gt;       // G of token 16w + lr
-    f4 gj[4];       // G of tokens 16jt + 4lg + i
-    bool ok;        // the A-operand token is in range
     uint32_t vok;   // bit r: token 16w + 4lg + r is in range
 };
-
-// 8 elements of a K / Q row: raw words at element i0
-template <bool BF16, bool VEC, int KW>
-XQ_DEV void load_raw8(const uint8_t* row, int i0, uint4 (&w)[KW]) {
-    if constexpr (VEC) {
-        const uint8_t* p = row + (BF16 ? 2 : 4) * i0;
-#pragma unroll
-        for (int u = 0; u < KW; ++u) w[u] = *(const uint4*)(p + 16 * u);
-    } else {
-        uint32_t e[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j)
-            e[j] = BF16 ? (uint32_t)((const uint16_t*)row)[i0 + j] : ((const uint32_t*)row)[i0 + j];
-        w[0] = make_uint4(e[0], e[1], e[2], e[3]);
-        w[1] = make_uint4(e[4], e[5], e[6], e[7]);
-        w[2] = w[3] = make_uint4(0, 0, 0, 0);
-    }
-}
-
-// f32 rows: the f16 remainder x - f16(x) of the same eight elements
-template <int KW>
-XQ_DEV h8 decode8_lo(const uint4 (&w)[KW], bool ok) {
-    const uint32_t u[8] = {w[0].x, w[0].y, w[0].z, w[0].w, w[1].x, w[1].y, w[1].z, w[1].w};
-    h8 r;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        const float x = __uint_as_float(u[e]);
-        r[e] = ok ? (_Float16)(x - (float)(_Float16)x) : (_Float16)0.0f;
-    }
-    return r;
-}
-
-template <bool BF16, bool VEC, int KW>
-XQ_DEV h8 decode8(const uint4 (&w)[KW], bool ok) {
-    float x[8];
-    if constexpr (VEC && BF16) {
-        const uint32_t u[4] = {w[0].x, w[0].y, w[0].z, w[0].w};
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            x[2 * e] = bf16_bits_to_f32(u[e] & 0xffffu);
-            x[2 * e + 1] = bf16_bits_to_f32(u[e] >> 16);
-        }
-    } else {
-        const uint32_t u[8] = {w[0].x, w[0].y, w[0].z, w[0].w, w[1].x, w[1].y, w[1].z, w[1].w};
-#pragma unroll
-        for (int e = 0; e < 8; ++e) x[e] = BF16 ? bf16_bits_to_f32(u[e] & 0xffffu) : __uint_as_float(u[e]);
-    }
-    h8 r;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) r[e] = ok ? (_Float16)x[e] : (_Float16)0.0f;
-    return r;
-}
 
 // Four 16-bit elements read transposed from LDS (gfx950 ds_read_b64_tr_b16):
 // in each group of 16 lanes, lane 4j + q addresses 4 consecutive elements of
@@ -659,10 +634,10 @@ XQ_DEV __amdgpu_buffer_rsrc_t rec_rsrc(const uint8_t* rec) {
 // The operands of chunk n in four parts, each issued in its own phase of the
 // previous chunk's step (between its barriers), in the order the step uses
 // them: a burst of all of them at the start of a step stalls the wave while
-// the loads queue. Part 0: K and Q rows; 1: T; 2: the decays and G; 3: V.
-template <int PART, bool BF16, bool VEC>
+// the loads queue. Part 0: K and Q rows; 1: T; 2: the decays and P; 3: V.
+template <int PART, bool F32, int NC>
 XQ_DEV void scan_load(const GdnChunkArgs& a, int b, int h, int cb, int n, int wave, int lr, int lg,
-                      ScanOps<BF16, VEC>& L) {
+                      ScanOps<F32, NC>& L) {
     const int kh = h % 16;
     n = min(n, a.n_chunks - 1);  // the prefetch past the last chunk re-reads it
     const int row0 = n * kChunk;      // the chunk's first token
@@ -673,40 +648,31 @@ XQ_DEV void scan_load(const GdnChunkArgs& a, int b, int h, int cb, int n, int wa
     // below 2^25 bytes), so the loads take their base from SGPRs and the
     // per-chunk address arithmetic stays off the vector ALU.
     if constexpr (PART == 0) {
-        const int r = 16 * wave + lr;  // A-operand row of the chunk
-        L.ok = r <= last;
-        const uint32_t rc = (uint32_t)min(r, last);
+        const uint32_t rc = (uint32_t)min(16 * wave + lr, last);  // A-operand row of the chunk
         const uint8_t* kb = a.k + (int64_t)b * a.k_nb3 + (int64_t)row0 * a.k_nb2 + (int64_t)kh * a.k_nb1;
         const uint8_t* qb = a.q + (int64_t)b * a.q_nb3 + (int64_t)row0 * a.q_nb2 + (int64_t)kh * a.q_nb1;
+        // the lane's part of the offset in one 32-bit word
+        constexpr uint32_t ES = F32 ? 4 : 2;
+        const uint32_t eo = 8u * ES * (uint32_t)lg;
+        const uint32_t ko = rc * (uint32_t)a.k_nb2 + eo, qo = rc * (uint32_t)a.q_nb2 + eo;
 #pragma unroll
-        for (int ks = 0; ks < 4; ++ks) {
-            if constexpr (VEC) {  // the lane's part of the offset in one 32-bit word
-                const uint32_t eo = (BF16 ? 2u : 4u) * (8u * (uint32_t)lg);
-                const uint32_t ko = rc * (uint32_t)a.k_nb2 + eo, qo = rc * (uint32_t)a.q_nb2 + eo;
+        for (int ks = 0; ks < 4; ++ks)
 #pragma unroll
-                for (int u = 0; u < ScanOps<BF16, VEC>::KW; ++u) {
-                    L.kw[ks][u] = *(const uint4*)(kb + (BF16 ? 64 : 128) * ks + 16 * u + ko);
-                    L.qw[ks][u] = *(const uint4*)(qb + (BF16 ? 64 : 128) * ks + 16 * u + qo);
-                }
-            } else {
-                load_raw8<BF16, VEC>(kb + rc * (uint32_t)a.k_nb2, 32 * ks + 8 * lg, L.kw[ks]);
-                load_raw8<BF16, VEC>(qb + rc * (uint32_t)a.q_nb2, 32 * ks + 8 * lg, L.qw[ks]);
+            for (int u = 0; u < ScanOps<F32, NC>::NK; ++u) {
+                const uint8_t* kp = kb + 32 * ES * ks + 16 * u + ko;
+                const uint8_t* qp = qb + 32 * ES * ks + 16 * u + qo;
+                L.kw[ks][u] = F32 ? ld_words_f32(kp) : ld_words_bf16(kp);
+                L.qw[ks][u] = F32 ? ld_words_f32(qp) : ld_words_bf16(qp);
             }
-        }
     } else if constexpr (PART == 1) {
+        const __amdgpu_buffer_rsrc_t r = rec_rsrc(rec);
 #pragma unroll
         for (int ks = 0; ks < 2; ++ks) {
             const uint32_t o = ((uint32_t)(16 * wave + lr) * 64u + 32u * ks + 8u * lg) * 2u;
-            if constexpr (BF16 && VEC) {
-                const __amdgpu_buffer_rsrc_t r = rec_rsrc(rec);
-                L.th[ks] = __builtin_bit_cast(h8, __builtin_amdgcn_raw_buffer_load_b128(r, o, kRecTHi, 0));
-                L.tl[ks] = __builtin_bit_cast(h8, __builtin_amdgcn_raw_buffer_load_b128(r, o, kRecTLo, 0));
-            } else {
-                L.th[ks] = *(const h8*)(rec + kRecTHi + o);
-                L.tl[ks] = *(const h8*)(rec + kRecTLo + o);
-            }
+            L.th[ks] = __builtin_bit_cast(h8, __builtin_amdgcn_raw_buffer_load_b128(r, o, kRecTHi, 0));
+            L.tl[ks] = __builtin_bit_cast(h8, __builtin_amdgcn_raw_buffer_load_b128(r, o, kRecTLo, 0));
         }
-    } else if constexpr (PART == 2 && BF16 && VEC) {
+    } else if constexpr (PART == 2) {
         // the record through a buffer resource: uniform parts of the offsets in
         // SGPRs, the lane's part in one VGPR, no per-load address arithmetic
         const __amdgpu_buffer_rsrc_t r = rec_rsrc(rec);
@@ -718,54 +684,64 @@ XQ_DEV void scan_load(const GdnChunkArgs& a, int b, int h, int cb, int n, int wa
         for (int jt = 0; jt < 4; ++jt)
             if (jt <= wave)  // wave-uniform
                 L.pw[jt] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(r, 16u * (uint32_t)(lr + 16 * lg), p_tile(wave, jt), 0));
-    } else if constexpr (PART == 2) {
-        const uint8_t* dec = rec + kRecDec;  // f32 values, byte offsets below
-        L.eg = *(const float4*)(dec + 4u * (uint32_t)(16 * wave + 4 * lg));
-        L.egc = *(const float4*)(dec + 4u * (uint32_t)(64 + 16 * wave + 4 * lg));
-        L.eGC = *(const float*)(dec + 4u * 128u);
-        L.gt = *(const float*)(dec + 4u * (uint32_t)(kRecG + 16 * wave + lr));
-#pragma unroll
-        for (int jt = 0; jt < 4; ++jt) L.gj[jt] = *(const f4*)(dec + 4u * (uint32_t)(kRecG + 16 * jt + 4 * lg));
-    } else if constexpr (BF16 && VEC) {
+    } else {
         // the chunk's V rows through a buffer resource whose range ends after
         // row `last` (row offsets below 2^25 bytes): a row past it reads 0
         // without touching memory (and is masked at use), so the lane offsets
         // need no clamp and stay the same for every chunk
+        constexpr uint32_t ES = F32 ? 4 : 2;
         L.vok = 0;
         const uint8_t* vb = a.v + (int64_t)b * a.v_nb3 + (int64_t)row0 * a.v_nb2 + (int64_t)h * a.v_nb1;
         const __amdgpu_buffer_rsrc_t r =
-            __builtin_amdgcn_make_buffer_rsrc((void*)vb, (short)0, (int)((uint32_t)min(last, kChunk - 1) * (uint32_t)a.v_nb2 + 256u), 0x00020000);
-        const uint32_t co = (uint32_t)(kCols * cb + lr) * 2u;
+            __builtin_amdgcn_make_buffer_rsrc((void*)vb, (short)0, (int)((uint32_t)min(last, kChunk - 1) * (uint32_t)a.v_nb2 + 128u * ES), 0x00020000);
+        const uint32_t co = (uint32_t)(kCols * NC * cb + NC * lr) * ES;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             const int rr = 16 * wave + 4 * lg + q;
             L.vok |= (rr <= last ? 1u : 0u) << q;
-            L.vw[q] = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(r, (uint32_t)rr * (uint32_t)a.v_nb2 + co, 0, 0);
-        }
-    } else {
-        L.vok = 0;
-        const uint8_t* vb = a.v + (int64_t)b * a.v_nb3 + (int64_t)row0 * a.v_nb2 + (int64_t)h * a.v_nb1;
-        const uint32_t co = (uint32_t)(kCols * cb + lr) * (BF16 ? 2u : 4u);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int rr = 16 * wave + 4 * lg + r;
-            L.vok |= (rr <= last ? 1u : 0u) << r;
-            const uint8_t* vr = vb + ((uint32_t)min(rr, last) * (uint32_t)a.v_nb2 + co);
-            if constexpr (BF16)
-                L.vw[r] = *(const uint16_t*)vr;
+            const uint32_t o = (uint32_t)rr * (uint32_t)a.v_nb2 + co;
+            if constexpr (ES * NC == 2)
+                L.vw[q] = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(r, o, 0, 0);
+            else if constexpr (ES * NC == 4)
+                L.vw[q] = __builtin_amdgcn_raw_buffer_load_b32(r, o, 0, 0);
             else
-                L.vw[r] = *(const uint32_t*)vr;
+                L.vw[q] = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(r, o, 0, 0));
         }
     }
 }
 
-template <bool BF16, bool VEC>
+template <bool F32, int NC>
 XQ_DEV void scan_load_all(const GdnChunkArgs& a, int b, int h, int cb, int n, int wave, int lr, int lg,
-                          ScanOps<BF16, VEC>& L) {
+                          ScanOps<F32, NC>& L) {
     scan_load<0>(a, b, h, cb, n, wave, lr, lg, L);
     scan_load<1>(a, b, h, cb, n, wave, lr, lg, L);
     scan_load<2>(a, b, h, cb, n, wave, lr, lg, L);
     scan_load<3>(a, b, h, cb, n, wave, lr, lg, L);
+}
+
+// Eight f32 words as f16 hi (r[0]) and lo (r[1])
+XQ_DEV void split8(const uint4 (&w)[2], uint4 (&r)[2]) {
+    f16_split4(w[0], r[0].x, r[0].y, r[1].x, r[1].y);
+    f16_split4(w[1], r[0].z, r[0].w, r[1].z, r[1].w);
+}
+
+// V of the lane's column ct as f32
+template <bool F32, int NC, typename T>
+XQ_DEV float v_value(const T& w, int ct) {
+    if constexpr (F32 && NC == 1)
+        return __uint_as_float(w);
+    else if constexpr (F32)
+        return __uint_as_float(ct ? w.y : w.x);
+    else if constexpr (NC == 1)
+        return bf16_bits_to_f32(w);
+    else {
+        uint32_t x;
+        if constexpr (NC == 2)
+            x = w;
+        else
+            x = ct & 2 ? w.y : w.x;
+        return __uint_as_float(ct & 1 ? x & 0xffff0000u : x << 16);
+    }
 }
 
 // The token-by-token recurrence for a scan workgroup's 16 columns, in f32: the
@@ -814,366 +790,352 @@ XQ_DEV void scan_sequential(const GdnChunkArgs& a, int b, int h, int cb, int wav
     for (int e = 0; e < 8; ++e) so[e] = s[e];
 }
 
-// NTY: the outputs Y are stored non-temporally (one workgroup per CU; see the
-// stores)
-template <bool BF16, bool VEC, bool NTY>
+// NC: column tiles of 16 value columns per workgroup. NTY: the outputs Y are
+// stored non-temporally (see the stores).
+template <bool F32, bool NTY, int NC>
 __global__ __launch_bounds__(256) void gdn_chunk_scan(GdnChunkArgs a) {
     constexpr int TP = 72;   // X^T, U^T rows [c][t] (halves)
     constexpr int SP = 136;  // S^T rows [c][i] (halves)
-    // bf16 rows with 16-byte row loads (RAW): the raw rows are the operands of
-    // bf16 products (exact), the state and e^{G_C - G} U enter as three bf16
-    // terms (hi, mid, lo; the f32 value exactly); otherwise f16 hi + lo
-    constexpr bool RAW = BF16 && VEC;
-    __shared__ __attribute__((aligned(16))) _Float16 sSh[kCols * SP], sSl[kCols * SP];  // S^T hi, lo
-    __shared__ __attribute__((aligned(16))) _Float16 sSm[RAW ? kCols * SP : 8];        // S^T mid (RAW)
-    __shared__ __attribute__((aligned(16))) _Float16 sXh[kCols * TP], sXl[kCols * TP];  // X^T
-    __shared__ __attribute__((aligned(16))) _Float16 sUh[kCols * TP], sUl[kCols * TP];  // U^T
-    __shared__ __attribute__((aligned(16))) _Float16 sWh[kCols * TP], sWl[kCols * TP];  // (e^{G_C - G} U)^T
-    __shared__ __attribute__((aligned(16))) _Float16 sWm[RAW ? kCols * TP : 8];
-    // K rows of the chunk [t][i] (f16 hi, and lo for f32 rows): the A operands of P^T = K Q^T
-    __shared__ __attribute__((aligned(16))) _Float16 sKh[RAW ? 8 : 64 * SP], sKl[BF16 ? 8 : 64 * SP];
-    // The state update's A operands K^T, by chunk parity (read after the step's
-    // last barrier, so the next chunk writes the other one): K^T [i][t] (f16
-    // hi, and lo for f32 rows), or in the bf16 operand form (RAW) the chunk's K
-    // rows [t][i] as loaded, pitch KRP, which the update reads transposed
-    // (lds_read_tr16). Both layouts take 128 x KTP = 64 x KRP halves.
-    constexpr int KTP = 72;   // K^T rows (halves)
-    constexpr int KRP = 144;  // RAW: K rows (halves; 288 bytes, rows 8 banks apart)
-    static_assert(128 * KTP == 64 * KRP, "one buffer for both layouts");
-    __shared__ __attribute__((aligned(16))) _Float16 sKTh[2][128 * KTP], sKTl[2][BF16 ? 8 : 128 * KTP];
+    constexpr int KRP = 144;  // K rows [t][i] (halves; 288 bytes, rows 8 banks apart)
+    constexpr int NCol = kCols * NC;
+    constexpr int kBlk = kColBlocks / NC;  // column groups per head
+    // bf16 rows are the operands of bf16 products as they are (exact), and the
+    // state and e^{G_C - G} U meet them as three bf16 terms (hi, mid, lo; the f32
+    // value exactly). f32 rows enter f16 products as hi + lo, and so does what
+    // meets them.
+    constexpr int NS = F32 ? 2 : 3;  // planes of the state and of e^{G_C - G} U
+    constexpr int NK = F32 ? 2 : 1;  // planes of K
+    __shared__ __attribute__((aligned(16))) _Float16 sS[NS][NCol * SP];   // S^T
+    __shared__ __attribute__((aligned(16))) _Float16 sXh[NCol * TP], sXl[NCol * TP];  // X^T
+    __shared__ __attribute__((aligned(16))) _Float16 sUh[NCol * TP], sUl[NCol * TP];  // U^T
+    __shared__ __attribute__((aligned(16))) _Float16 sW[NS][NCol * TP];   // (e^{G_C - G} U)^T
+    // The chunk's K rows, by chunk parity (the state update reads them
+    // transposed, after the step's last barrier, so the next chunk writes the
+    // other set)
+    __shared__ __attribute__((aligned(16))) _Float16 sK[2][NK][64 * KRP];
+    __shared__ uint32_t sAm[NC], sOut;
 
-    const uint32_t n_wg = (uint32_t)a.B * 32 * kColBlocks;
-    // column blocks of a head adjacent, then the two v-heads kh, kh + 16 that
-    // read the same K and Q rows: the 16 workgroups on one XCD (shared L2)
+    const uint32_t n_wg = (uint32_t)a.B * 32 * kBlk;
+    // column groups of a head adjacent, then the two v-heads kh, kh + 16 that
+    // read the same K and Q rows: the workgroups of both on one XCD (shared L2)
     const uint32_t wg = xcd_remap(blockIdx.x, n_wg);
-    const int cb = (int)(wg % kColBlocks);
-    const int h = (int)((wg / (2 * kColBlocks)) % 16) + 16 * (int)((wg / kColBlocks) % 2);
-    const int b = (int)(wg / (kColBlocks * 32));
+    const int cb = (int)(wg % kBlk);
+    const int h = (int)((wg / (2 * kBlk)) % 16) + 16 * (int)((wg / kBlk) % 2);
+    const int b = (int)(wg / (kBlk * 32));
     const int wave = wave_id(), lane = lane_id(), lr = lane & 15, lg = lane >> 4;
+    const int col0 = NCol * cb + NC * lr;  // the lane's first column
+    const int vb = NC * lr / kCols;        // its 16-column block within the group
 
-    // state tiles of this wave: key-dim tiles 2w, 2w + 1 of the 128 x 16 block;
-    // lane holds S[i = 16 it + 4 lg + r][c = 16 cb + lr]
+    // state tiles of this wave: key-dim tiles 2w, 2w + 1; lane holds
+    // S[i = 16 it + 4 lg + r][c = col0 + ct]
     const float* st = a.state + (int64_t)b * (a.s_nb3 / 4) + (int64_t)h * 16384;
-    f4 S[2];
+    f4 S[2][NC];
 #pragma unroll
-    for (int a2 = 0; a2 < 2; ++a2) {
-        const int it = 2 * wave + a2;
-        const float4 v = *(const float4*)(st + (int64_t)(kCols * cb + lr) * 128 + 16 * it + 4 * lg);
-        S[a2] = f4{v.x, v.y, v.z, v.w};
-    }
+    for (int a2 = 0; a2 < 2; ++a2)
+#pragma unroll
+        for (int ct = 0; ct < NC; ++ct) {
+            const float4 v = *(const float4*)(st + (int64_t)(col0 + ct) * 128 + 16 * (2 * wave + a2) + 4 * lg);
+            S[a2][ct] = f4{v.x, v.y, v.z, v.w};
+        }
     float* out = a.dst + (int64_t)b * (a.dst_nb2 / 4);
     // the first chunk's operands do not depend on 2^a (V is scaled at use): their
     // loads go out with the state's and the maxima's
-    ScanOps<BF16, VEC> ops[2];
-    scan_load_all<BF16, VEC>(a, b, h, cb, 0, wave, lr, lg, ops[0]);
+    ScanOps<F32, NC> ops[2];
+    scan_load_all<F32, NC>(a, b, h, cb, 0, wave, lr, lg, ops[0]);
 
-    // ---- 2^a: the largest |S| entering the block and |v| of its columns over
-    //      the prefill (the chunks' maxima from the prep) brought into [1, 2)
-    //      (and whether some chunk's q / k leave the operands' range)
-    __shared__ uint32_t sAm[4], sOut[4];
+    // ---- 2^a per 16-column block: the largest |S| entering the block and |v| of
+    //      its columns over the prefill (the chunks' maxima from the prep) brought
+    //      into [1, 2) (and whether some chunk's q / k leave the operands' range)
+    if (threadIdx.x < NC) sAm[threadIdx.x] = 0;
+    if (threadIdx.x == 0) sOut = 0;
+    __syncthreads();
     {
-        uint32_t am = 0;
+        uint32_t am = 0, vm[NC];
         bool out_of_range = false;
 #pragma unroll
         for (int a2 = 0; a2 < 2; ++a2)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) am = max(am, __float_as_uint(S[a2][r]) & 0x7fffffffu);
+            for (int ct = 0; ct < NC; ++ct)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) am = max(am, __float_as_uint(S[a2][ct][r]) & 0x7fffffffu);
+#pragma unroll
+        for (int j = 0; j < NC; ++j) vm[j] = j == vb ? am : 0u;
         for (int n = lane; n < a.n_chunks; n += 64) {
             const float* dec = (const float*)(a.ws + (((int64_t)b * a.n_chunks + n) * 32 + h) * kRecBytes + kRecDec);
-            am = max(am, __float_as_uint(dec[kRecVmax + cb]) & 0x7fffffffu);
+#pragma unroll
+            for (int j = 0; j < NC; ++j) vm[j] = max(vm[j], __float_as_uint(dec[kRecVmax + NC * cb + j]) & 0x7fffffffu);
             out_of_range |= dec[kRecRange] != 0.0f;
         }
-        const bool wave_out = __builtin_amdgcn_ballot_w64(out_of_range) != 0;  // every lane of the wave
-        if (lane == 0) sOut[wave] = wave_out ? 1u : 0u;
-        am = max(am, (uint32_t)dpp_i<0xB1>((int)am));
-        am = max(am, (uint32_t)dpp_i<0x4E>((int)am));
-        am = max(am, (uint32_t)dpp_i<0x141>((int)am));
-        am = max(am, (uint32_t)dpp_i<0x140>((int)am));
-        am = max(am, (uint32_t)__shfl_xor((int)am, 16));
-        am = max(am, (uint32_t)__shfl_xor((int)am, 32));
-        if (lane == 0) sAm[wave] = am;
+        if (__builtin_amdgcn_ballot_w64(out_of_range) != 0 && lane == 0) atomicOr(&sOut, 1u);
+#pragma unroll
+        for (int j = 0; j < NC; ++j) {
+            const uint32_t m = wave_max_u32(vm[j]);
+            if (lane == 0) atomicMax(&sAm[j], m);
+        }
     }
     __syncthreads();
-    // an Inf or NaN among the column block's v or entering state: the chunked
-    // products would carry it into earlier tokens of its chunk (a zero of T
-    // times it is NaN), so the block runs token by token, as the recurrence
-    // spreads it
-    const uint32_t am_all = max(max(sAm[0], sAm[1]), max(sAm[2], sAm[3]));
-    if ((sOut[0] | sOut[1] | sOut[2] | sOut[3]) || am_all >= 0x7f800000u) {  // workgroup-uniform
-        scan_sequential<BF16>(a, b, h, cb, wave, lane);
+    if (sOut) {  // workgroup-uniform
+        for (int j = 0; j < NC; ++j) scan_sequential<!F32>(a, b, h, NC * cb + j, wave, lane);
         return;
     }
-    int pa = 0;  // the power a
+    int pa = 0;  // the power a of the lane's block
     {
-        const float m = __uint_as_float(am_all);
-        if (m > 0.0f) {
+        const uint32_t mb = sAm[vb];
+        if (mb > 0 && mb < 0x7f800000u) {
             int ex;
-            (void)frexpf(m, &ex);  // m = f 2^ex, f in [0.5, 1)
+            (void)frexpf(__uint_as_float(mb), &ex);  // m = f 2^ex, f in [0.5, 1)
             pa = min(max(1 - ex, -100), 100);
         }
     }
     const float vscale = __builtin_ldexpf(1.0f, pa), unscale = __builtin_ldexpf(1.0f, -pa);
     const float yscale = a.scale * unscale;
 #pragma unroll
-    for (int a2 = 0; a2 < 2; ++a2) S[a2] *= vscale;
+    for (int a2 = 0; a2 < 2; ++a2)
+#pragma unroll
+        for (int ct = 0; ct < NC; ++ct) S[a2][ct] *= vscale;
 
     // One chunk: C holds its operands (loaded a chunk ahead), the next chunk's
     // operands are loaded into Nx part by part.
-    auto chunk = [&](const int nn, ScanOps<BF16, VEC>& C, ScanOps<BF16, VEC>& Nx, _Float16* kth, _Float16* ktl) {
+    auto chunk = [&](const int nn, ScanOps<F32, NC>& C, ScanOps<F32, NC>& Nx, _Float16 (*kt)[64 * KRP]) {
         scan_load<0>(a, b, h, cb, nn + 1, wave, lr, lg, Nx);
 
-        // ---- the wave's K rows -> LDS transposed (the state update's
-        //      operands) and, when the scan forms P, as rows (every wave forms
-        //      its P from all of them)
-        h8 ak[4], aq[4];
-        uint4 rk[4], rq[4];  // RAW: the rows as loaded
+        // ---- the wave's K rows -> LDS (f32 rows: as f16 hi and lo). Rows past T
+        //      are real rows (clamped loads): every product they enter meets a zero
+        //      T row or column, so they add nothing
+        uint4 rk[4][NK], rq[4][NK];
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) {
-            if constexpr (RAW) {
-                // rows past T are real rows (clamped loads): every product they
-                // enter meets a zero T row or column, so they add nothing
-                rk[ks] = C.kw[ks][0];
-                rq[ks] = C.qw[ks][0];
-                *(uint4*)(kth + (16 * wave + lr) * KRP + 32 * ks + 8 * lg) = rk[ks];
-                continue;
+            if constexpr (F32) {
+                split8(C.kw[ks], rk[ks]);
+                split8(C.qw[ks], rq[ks]);
+            } else {
+                rk[ks][0] = C.kw[ks][0];
+                rq[ks][0] = C.qw[ks][0];
             }
-            ak[ks] = decode8<BF16, VEC>(C.kw[ks], C.ok);
-            aq[ks] = decode8<BF16, VEC>(C.qw[ks], C.ok);
-            const int ko = (16 * wave + lr) * SP + 32 * ks + 8 * lg;
-            *(h8*)(sKh + ko) = ak[ks];
 #pragma unroll
-            for (int e = 0; e < 8; ++e) kth[(32 * ks + 8 * lg + e) * KTP + 16 * wave + lr] = ak[ks][e];
-            if constexpr (!BF16) {
-                const h8 al = decode8_lo(C.kw[ks], C.ok);
-                *(h8*)(sKl + ko) = al;
-#pragma unroll
-                for (int e = 0; e < 8; ++e) ktl[(32 * ks + 8 * lg + e) * KTP + 16 * wave + lr] = al[e];
-            }
+            for (int u = 0; u < NK; ++u) *(uint4*)(kt[u] + (16 * wave + lr) * KRP + 32 * ks + 8 * lg) = rk[ks][u];
         }
 
-        // ---- S (hi, lo) -> LDS as S^T [c][i]: the B operand rows of K S and Q S
+        // ---- S -> LDS as S^T [c][i]: the B operand rows of K S and Q S
 #pragma unroll
-        for (int a2 = 0; a2 < 2; ++a2) {
-            const int it = 2 * wave + a2;
-            if constexpr (RAW) {
-                uint2 t3[3];
-                split3_x4(S[a2], t3);
-                *(uint2*)(sSh + lr * SP + 16 * it + 4 * lg) = t3[0];
-                *(uint2*)(sSm + lr * SP + 16 * it + 4 * lg) = t3[1];
-                *(uint2*)(sSl + lr * SP + 16 * it + 4 * lg) = t3[2];
-                continue;
+        for (int ct = 0; ct < NC; ++ct)
+#pragma unroll
+            for (int a2 = 0; a2 < 2; ++a2) {
+                const int o = (kCols * ct + lr) * SP + 16 * (2 * wave + a2) + 4 * lg;
+                if constexpr (F32) {
+                    h4 sh, sl;
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) sh[r] = f16_hi(S[a2][ct][r]), sl[r] = f16_lo(S[a2][ct][r]);
+                    *(h4*)(sS[0] + o) = sh;
+                    *(h4*)(sS[1] + o) = sl;
+                } else {
+                    uint2 t3[3];
+                    split3_x4(S[a2][ct], t3);
+#pragma unroll
+                    for (int p = 0; p < 3; ++p) *(uint2*)(sS[p] + o) = t3[p];
+                }
             }
-            h4 sh, sl;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) sh[r] = f16_hi(S[a2][r]), sl[r] = f16_lo(S[a2][r]);
-            *(h4*)(sSh + lr * SP + 16 * it + 4 * lg) = sh;
-            *(h4*)(sSl + lr * SP + 16 * it + 4 * lg) = sl;
-        }
         __syncthreads();
         scan_load<1>(a, b, h, cb, nn + 1, wave, lr, lg, Nx);
 
-        // ---- K S and Q S for token tile w (16 tokens x 16 columns)
-        f4 ksh = f4{0.0f, 0.0f, 0.0f, 0.0f}, ksl = ksh, qsh = ksh, qsl = ksh;
+        // ---- K S and Q S for token tile w (16 tokens x the columns)
+        f4 ksh[NC], ksl[NC], qsh[NC], qsl[NC];
 #pragma unroll
-        for (int ks = 0; ks < 4; ++ks) {
-            const int bo = lr * SP + 32 * ks + 8 * lg;
-            if constexpr (RAW) {
-                const uint4 b0 = *(const uint4*)(sSh + bo), b1 = *(const uint4*)(sSm + bo),
-                            b2 = *(const uint4*)(sSl + bo);
-                ksh = mfma_bf(rk[ks], b0, ksh);
-                qsh = mfma_bf(rq[ks], b0, qsh);
-                ksl = mfma_bf(rk[ks], b1, ksl);
-                qsl = mfma_bf(rq[ks], b1, qsl);
-                ksl = mfma_bf(rk[ks], b2, ksl);
-                qsl = mfma_bf(rq[ks], b2, qsl);
-                continue;
+        for (int ct = 0; ct < NC; ++ct) ksh[ct] = ksl[ct] = qsh[ct] = qsl[ct] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+            for (int ct = 0; ct < NC; ++ct) {
+                const int bo = (kCols * ct + lr) * SP + 32 * ks + 8 * lg;
+                if constexpr (F32) {
+                    const h8 bh = *(const h8*)(sS[0] + bo), bl = *(const h8*)(sS[1] + bo);
+                    const h8 ak = __builtin_bit_cast(h8, rk[ks][0]), al = __builtin_bit_cast(h8, rk[ks][NK - 1]);
+                    const h8 aq = __builtin_bit_cast(h8, rq[ks][0]), ql = __builtin_bit_cast(h8, rq[ks][NK - 1]);
+                    ksh[ct] = mfma32(ak, bh, ksh[ct]);
+                    ksl[ct] = mfma32(ak, bl, ksl[ct]);
+                    qsh[ct] = mfma32(aq, bh, qsh[ct]);
+                    qsl[ct] = mfma32(aq, bl, qsl[ct]);
+                    ksl[ct] = mfma32(al, bh, ksl[ct]);
+                    qsl[ct] = mfma32(ql, bh, qsl[ct]);
+                } else {
+                    const uint4 b0 = *(const uint4*)(sS[0] + bo), b1 = *(const uint4*)(sS[1] + bo),
+                                b2 = *(const uint4*)(sS[NS - 1] + bo);
+                    ksh[ct] = mfma_bf(rk[ks][0], b0, ksh[ct]);
+                    qsh[ct] = mfma_bf(rq[ks][0], b0, qsh[ct]);
+                    ksl[ct] = mfma_bf(rk[ks][0], b1, ksl[ct]);
+                    qsl[ct] = mfma_bf(rq[ks][0], b1, qsl[ct]);
+                    ksl[ct] = mfma_bf(rk[ks][0], b2, ksl[ct]);
+                    qsl[ct] = mfma_bf(rq[ks][0], b2, qsl[ct]);
+                }
             }
-            const h8 bh = *(const h8*)(sSh + bo), bl = *(const h8*)(sSl + bo);
-            ksh = mfma32(ak[ks], bh, ksh);
-            ksl = mfma32(ak[ks], bl, ksl);
-            qsh = mfma32(aq[ks], bh, qsh);
-            qsl = mfma32(aq[ks], bl, qsl);
-            if constexpr (!BF16) {
-                ksl = mfma32(decode8_lo(C.kw[ks], C.ok), bh, ksl);
-                qsl = mfma32(decode8_lo(C.qw[ks], C.ok), bh, qsl);
-            }
-        }
-        // ---- X = V - e^G (K S) -> LDS as X^T [c][t] (hi, lo); lane: column lr,
+        // ---- X = V - e^G (K S) -> LDS as X^T [c][t] (hi, lo); lane: its columns,
         //      tokens 16w + 4lg + r
-        f4 QS;
-        h4 xh, xl;
+        f4 QS[NC];
         const float egr[4] = {C.eg.x, C.eg.y, C.eg.z, C.eg.w};
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const float vv =
-                (C.vok >> r) & 1 ? (BF16 ? bf16_bits_to_f32(C.vw[r]) : __uint_as_float(C.vw[r])) * vscale : 0.0f;
-            const float x = vv - egr[r] * (ksh[r] + ksl[r]);
-            QS[r] = egr[r] * (qsh[r] + qsl[r]);
-            xh[r] = f16_hi(x), xl[r] = f16_lo(x);
+        for (int ct = 0; ct < NC; ++ct) {
+            h4 xh, xl;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float vv = (C.vok >> r) & 1 ? v_value<F32, NC>(C.vw[r], ct) * vscale : 0.0f;
+                const float x = vv - egr[r] * (ksh[ct][r] + ksl[ct][r]);
+                QS[ct][r] = egr[r] * (qsh[ct][r] + qsl[ct][r]);
+                xh[r] = f16_hi(x), xl[r] = f16_lo(x);
+            }
+            const int o = (kCols * ct + lr) * TP + 16 * wave + 4 * lg;
+            *(h4*)(sXh + o) = xh;
+            *(h4*)(sXl + o) = xl;
         }
-        *(h4*)(sXh + lr * TP + 16 * wave + 4 * lg) = xh;
-        *(h4*)(sXl + lr * TP + 16 * wave + 4 * lg) = xl;
-
         // ---- P[t][j] = (q_t . k_j) e^{G_t - G_j} (j <= t) for t in the wave's
-        //      tile, as P^T = K Q^T per token tile jt <= w: lane (lr, lg) gets
-        //      t = 16w + lr, j = 16jt + 4lg + i, which is the A operand layout of
-        //      the 16x16x16 product Y += P U below. RAW: the prep formed them
-        //      (the same products), so they stay off the step's chain
+        //      tile, as P^T = K Q^T per token tile jt <= w: the prep formed them
+        //      in the A operand layout of the 16x16x16 product Y += P U below
         h4 ph[4], pl[4];
 #pragma unroll
         for (int jt = 0; jt < 4; ++jt) {
             ph[jt] = h4{0, 0, 0, 0};
             pl[jt] = ph[jt];
-            if constexpr (RAW) {  // the prep's tiles, loaded a chunk ahead
-                if (jt > wave) continue;  // wave-uniform
-                ph[jt] = __builtin_bit_cast(h4, make_uint2(C.pw[jt].x, C.pw[jt].y));
-                pl[jt] = __builtin_bit_cast(h4, make_uint2(C.pw[jt].z, C.pw[jt].w));
-            } else {
-                if (jt > wave) continue;  // wave-uniform
-                f4 pt = f4{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-                for (int ks = 0; ks < 4; ++ks) {
-                    const int ko = (16 * jt + lr) * SP + 32 * ks + 8 * lg;
-                    const h8 kj = *(const h8*)(sKh + ko);
-                    pt = mfma32(kj, aq[ks], pt);
-                    if constexpr (!BF16) {
-                        pt = mfma32(kj, decode8_lo(C.qw[ks], C.ok), pt);
-                        pt = mfma32(*(const h8*)(sKl + ko), aq[ks], pt);
-                    }
-                }
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const bool causal = jt < wave || 4 * lg + i <= lr;
-                    const float pv = causal ? pt[i] * __expf(C.gt - C.gj[jt][i]) : 0.0f;
-                    ph[jt][i] = f16_hi(pv), pl[jt][i] = f16_lo(pv);
-                }
-            }
+            if (jt > wave) continue;  // wave-uniform
+            ph[jt] = __builtin_bit_cast(h4, make_uint2(C.pw[jt].x, C.pw[jt].y));
+            pl[jt] = __builtin_bit_cast(h4, make_uint2(C.pw[jt].z, C.pw[jt].w));
         }
         __syncthreads();
         scan_load<2>(a, b, h, cb, nn + 1, wave, lr, lg, Nx);
 
         // ---- U = T X for token tile w; U and e^{G_C - G} U -> LDS as [c][t]
-        f4 u = f4{0.0f, 0.0f, 0.0f, 0.0f}, u2 = u;
 #pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
-            const int bo = lr * TP + 32 * ks + 8 * lg;
-            const h8 bh = *(const h8*)(sXh + bo), bl = *(const h8*)(sXl + bo);
-            u = mfma32(C.th[ks], bh, u);
-            u2 = mfma32(C.th[ks], bl, u2);
-            u2 = mfma32(C.tl[ks], bh, u2);
-        }
-        u += u2;
-        {
+        for (int ct = 0; ct < NC; ++ct) {
+            f4 u = f4{0.0f, 0.0f, 0.0f, 0.0f}, u2 = u;
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks) {
+                const int bo = (kCols * ct + lr) * TP + 32 * ks + 8 * lg;
+                const h8 bh = *(const h8*)(sXh + bo), bl = *(const h8*)(sXl + bo);
+                u = mfma32(C.th[ks], bh, u);
+                u2 = mfma32(C.th[ks], bl, u2);
+                u2 = mfma32(C.tl[ks], bh, u2);
+            }
+            u += u2;
             const float egcr[4] = {C.egc.x, C.egc.y, C.egc.z, C.egc.w};
-            h4 uh, ul, wh, wl;
+            h4 uh, ul;
+            f4 w;
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const float w = u[r] * egcr[r];
+                w[r] = u[r] * egcr[r];
                 uh[r] = f16_hi(u[r]), ul[r] = f16_lo(u[r]);
-                wh[r] = f16_hi(w), wl[r] = f16_lo(w);
             }
-            const int o = lr * TP + 16 * wave + 4 * lg;
+            const int o = (kCols * ct + lr) * TP + 16 * wave + 4 * lg;
             *(h4*)(sUh + o) = uh;
             *(h4*)(sUl + o) = ul;
-            if constexpr (RAW) {
-                uint2 w3[3];
-                split3_x4(f4{u[0] * egcr[0], u[1] * egcr[1], u[2] * egcr[2], u[3] * egcr[3]}, w3);
-                *(uint2*)(sWh + o) = w3[0];
-                *(uint2*)(sWm + o) = w3[1];
-                *(uint2*)(sWl + o) = w3[2];
+            if constexpr (F32) {
+                h4 wh, wl;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) wh[r] = f16_hi(w[r]), wl[r] = f16_lo(w[r]);
+                *(h4*)(sW[0] + o) = wh;
+                *(h4*)(sW[1] + o) = wl;
             } else {
-                *(h4*)(sWh + o) = wh;
-                *(h4*)(sWl + o) = wl;
+                uint2 w3[3];
+                split3_x4(w, w3);
+#pragma unroll
+                for (int p = 0; p < 3; ++p) *(uint2*)(sW[p] + o) = w3[p];
             }
         }
         __syncthreads();
         scan_load<3>(a, b, h, cb, nn + 1, wave, lr, lg, Nx);
 
         // ---- Y = scale (e^G Q S + P U) for token tile w (P is zero past tile w)
-        f4 y = QS, y2 = f4{0.0f, 0.0f, 0.0f, 0.0f};
+        f4 Y[NC];
 #pragma unroll
-        for (int jt = 0; jt < 4; ++jt) {
-            if (jt > wave) continue;  // wave-uniform
-            const int bo = lr * TP + 16 * jt + 4 * lg;
-            const h4 bh = *(const h4*)(sUh + bo), bl = *(const h4*)(sUl + bo);
-            y = mfma16(ph[jt], bh, y);
-            y2 = mfma16(ph[jt], bl, y2);
-            y2 = mfma16(pl[jt], bh, y2);
+        for (int ct = 0; ct < NC; ++ct) {
+            f4 y = QS[ct], y2 = f4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int jt = 0; jt < 4; ++jt) {
+                if (jt > wave) continue;  // wave-uniform
+                const int bo = (kCols * ct + lr) * TP + 16 * jt + 4 * lg;
+                const h4 bh = *(const h4*)(sUh + bo), bl = *(const h4*)(sUl + bo);
+                y = mfma16(ph[jt], bh, y);
+                y2 = mfma16(ph[jt], bl, y2);
+                y2 = mfma16(pl[jt], bh, y2);
+            }
+            Y[ct] = y + y2;
         }
-        y += y2;
-        if constexpr (RAW) {
+        {
             // through a buffer resource over the chunk's output rows: the
-            // (head, column block) part of the offset in an SGPR, the lane's
+            // (head, column group) part of the offset in an SGPR, the lane's
             // token and column in one VGPR. Non-temporal when the scan runs one
             // workgroup per CU (nothing here reads the outputs again, and the
-            // operands keep the L2); with two per CU (several sequences) the
-            // column blocks' partial lines merge better in L2
+            // operands keep the L2); with two per CU the column blocks' partial
+            // lines merge better in L2
             const __amdgpu_buffer_rsrc_t r =
                 __builtin_amdgcn_make_buffer_rsrc((void*)(out + (int64_t)nn * kChunk * 4096), (short)0, 0x7fffffff, 0x00020000);
-            const uint32_t so = 4u * (uint32_t)(h * 128 + kCols * cb);
+            const uint32_t so = 4u * (uint32_t)(h * 128 + NCol * cb);
+            typedef uint32_t yv2 __attribute__((ext_vector_type(2)));
+            typedef uint32_t yv4 __attribute__((ext_vector_type(4)));
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 const int tl = 16 * wave + 4 * lg + q;  // token within the chunk
                 if (nn * kChunk + tl < a.T) {
-                    const uint32_t yv = __builtin_bit_cast(uint32_t, y[q] * yscale), vo = (uint32_t)tl * 16384u + 4u * (uint32_t)lr;
-                    __builtin_amdgcn_raw_buffer_store_b32(yv, r, vo, so, NTY ? 2 : 0);
-                }
-            }
-        } else {
+                    uint32_t yv[NC];
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int t = nn * kChunk + 16 * wave + 4 * lg + q;
-                if (t < a.T) {
-                    float* o = out + (int64_t)t * 4096 + h * 128 + kCols * cb + lr;
-                    if constexpr (NTY)
-                        __builtin_nontemporal_store(y[q] * yscale, o);
+                    for (int ct = 0; ct < NC; ++ct) yv[ct] = __builtin_bit_cast(uint32_t, Y[ct][q] * yscale);
+                    const uint32_t vo = (uint32_t)tl * 16384u + 4u * (uint32_t)(NC * lr);
+                    if constexpr (NC == 1)
+                        __builtin_amdgcn_raw_buffer_store_b32(yv[0], r, vo, so, NTY ? 2 : 0);
+                    else if constexpr (NC == 2)
+                        __builtin_amdgcn_raw_buffer_store_b64(yv2{yv[0], yv[1]}, r, vo, so, NTY ? 2 : 0);
                     else
-                        *o = y[q] * yscale;
+                        __builtin_amdgcn_raw_buffer_store_b128(yv4{yv[0], yv[1], yv[2], yv[3]}, r, vo, so, NTY ? 2 : 0);
                 }
             }
         }
 
         // ---- S = e^{G_C} S + K^T (e^{G_C - G} U) for this wave's key-dim tiles
-        if constexpr (RAW) {  // the three bf16 terms of (e^{G_C - G} U)^T read once for both tiles
-            uint4 bw[2][3];
+        // K^T[16 it + lr][32 ks + 8 lg + j], j = 0..7: the 4 x 16 blocks at tokens
+        // 32 ks + 8 lg (+ 4), key dims 16 it ..
+        auto k_t = [&](int a2, int ks, int u) {
+            const _Float16* kb = kt[u] + (32 * ks + 8 * lg + (lr >> 2)) * KRP + 16 * (2 * wave + a2) + 4 * (lr & 3);
+            const uint2 k0 = lds_read_tr16(kb), k1 = lds_read_tr16(kb + 4 * KRP);
+            return make_uint4(k0.x, k0.y, k1.x, k1.y);
+        };
+        // the terms of (e^{G_C - G} U)^T of a column tile, read once for both key-dim tiles
+        auto w_terms = [&](int ct, uint4 (&bw)[2][NS]) {
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+                for (int p = 0; p < NS; ++p) bw[ks][p] = *(const uint4*)(sW[p] + (kCols * ct + lr) * TP + 32 * ks + 8 * lg);
+        };
+        auto update = [&](int a2, int ct, const uint4 (&ka)[2][NK], const uint4 (&bw)[2][NS]) {
+            f4 acc = S[a2][ct] * C.eGC, acc2 = f4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
             for (int ks = 0; ks < 2; ++ks) {
-                const int bo = lr * TP + 32 * ks + 8 * lg;
-                bw[ks][0] = *(const uint4*)(sWh + bo);
-                bw[ks][1] = *(const uint4*)(sWm + bo);
-                bw[ks][2] = *(const uint4*)(sWl + bo);
-            }
-#pragma unroll
-            for (int a2 = 0; a2 < 2; ++a2) {
-                f4 acc = S[a2] * C.eGC, acc2 = f4{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-                for (int ks = 0; ks < 2; ++ks) {
-                    // K^T[16 it + lr][32 ks + 8 lg + j], j = 0..7: the 4 x 16 blocks
-                    // at tokens 32 ks + 8 lg (+ 4), key dims 16 it ..
-                    const _Float16* kb = kth + (32 * ks + 8 * lg + (lr >> 2)) * KRP + 16 * (2 * wave + a2) + 4 * (lr & 3);
-                    const uint2 k0 = lds_read_tr16(kb), k1 = lds_read_tr16(kb + 4 * KRP);
-                    const uint4 kt = make_uint4(k0.x, k0.y, k1.x, k1.y);
-                    acc = mfma_bf(kt, bw[ks][0], acc);
-                    acc2 = mfma_bf(kt, bw[ks][1], acc2);
-                    acc2 = mfma_bf(kt, bw[ks][2], acc2);
+                if constexpr (F32) {
+                    const h8 kh = __builtin_bit_cast(h8, ka[ks][0]), kl = __builtin_bit_cast(h8, ka[ks][NK - 1]);
+                    acc = mfma32(kh, __builtin_bit_cast(h8, bw[ks][0]), acc);
+                    acc2 = mfma32(kh, __builtin_bit_cast(h8, bw[ks][1]), acc2);
+                    acc2 = mfma32(kl, __builtin_bit_cast(h8, bw[ks][0]), acc2);
+                } else {
+                    acc = mfma_bf(ka[ks][0], bw[ks][0], acc);
+                    acc2 = mfma_bf(ka[ks][0], bw[ks][1], acc2);
+                    acc2 = mfma_bf(ka[ks][0], bw[ks][NS - 1], acc2);
                 }
-                S[a2] = acc + acc2;
             }
-            return;
-        }
+            S[a2][ct] = acc + acc2;
+        };
+        uint4 ka[2][2][NK], bw[2][NS];
+        if constexpr (NC == 1) w_terms(0, bw);
 #pragma unroll
         for (int a2 = 0; a2 < 2; ++a2) {
-            f4 acc = S[a2] * C.eGC, acc2 = f4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-            for (int ks = 0; ks < 2; ++ks) {
-                const int bo = lr * TP + 32 * ks + 8 * lg;
-                const int ko = (16 * (2 * wave + a2) + lr) * KTP + 32 * ks + 8 * lg;
-                const h8 wh = *(const h8*)(sWh + bo), kt = *(const h8*)(kth + ko);
-                acc = mfma32(kt, wh, acc);
-                acc2 = mfma32(kt, *(const h8*)(sWl + bo), acc2);
-                if constexpr (!BF16) acc2 = mfma32(*(const h8*)(ktl + ko), wh, acc2);
+            for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+                for (int u = 0; u < NK; ++u) ka[a2][ks][u] = k_t(a2, ks, u);
+            if constexpr (NC == 1) update(a2, 0, ka[a2], bw);
+        }
+        if constexpr (NC > 1) {
+#pragma unroll
+            for (int ct = 0; ct < NC; ++ct) {
+                w_terms(ct, bw);
+#pragma unroll
+                for (int a2 = 0; a2 < 2; ++a2) update(a2, ct, ka[a2], bw);
             }
-            S[a2] = acc + acc2;
         }
     };
     // Chunk pairs in the loop (the two operand sets stay in fixed registers)
@@ -1182,18 +1144,32 @@ __global__ __launch_bounds__(256) void gdn_chunk_scan(GdnChunkArgs a) {
     // iteration and never waits for the next chunk's operands early.
     int n = 0;
     for (; n + 1 < a.n_chunks; n += 2) {
-        chunk(n, ops[0], ops[1], sKTh[0], sKTl[0]);
-        chunk(n + 1, ops[1], ops[0], sKTh[1], sKTl[1]);
+        chunk(n, ops[0], ops[1], sK[0]);
+        chunk(n + 1, ops[1], ops[0], sK[1]);
     }
-    if (n < a.n_chunks) chunk(n, ops[0], ops[1], sKTh[0], sKTl[0]);
+    if (n < a.n_chunks) chunk(n, ops[0], ops[1], sK[0]);
 
     // ---- final state (transposed layout: element (i, c) of head h at h*16384 + c*128 + i)
     float* so = a.state_out + (int64_t)b * (a.so_nb3 / 4) + (int64_t)h * 16384;
 #pragma unroll
-    for (int a2 = 0; a2 < 2; ++a2) {
-        const int it = 2 * wave + a2;
-        *(float4*)(so + (int64_t)(kCols * cb + lr) * 128 + 16 * it + 4 * lg) =
-            make_float4(S[a2][0] * unscale, S[a2][1] * unscale, S[a2][2] * unscale, S[a2][3] * unscale);
+    for (int a2 = 0; a2 < 2; ++a2)
+#pragma unroll
+        for (int ct = 0; ct < NC; ++ct)
+            *(float4*)(so + (int64_t)(col0 + ct) * 128 + 16 * (2 * wave + a2) + 4 * lg) =
+                make_float4(S[a2][ct][0] * unscale, S[a2][ct][1] * unscale, S[a2][ct][2] * unscale, S[a2][ct][3] * unscale);
+
+    // an Inf or NaN among a column block's v or entering state: the chunked
+    // products carry it into earlier tokens of its chunk (a zero of T times it is
+    // NaN), in its own columns only, so the block runs again token by token, as
+    // the recurrence spreads it
+    bool again = false;
+#pragma unroll
+    for (int j = 0; j < NC; ++j) again |= sAm[j] >= 0x7f800000u;  // workgroup-uniform
+    if (again) {
+        __threadfence();  // the block's stores above come first
+        __syncthreads();
+        for (int j = 0; j < NC; ++j)
+            if (sAm[j] >= 0x7f800000u) scan_sequential<!F32>(a, b, h, NC * cb + j, wave, lane);
     }
 }
 
@@ -1205,21 +1181,48 @@ size_t gdn_chunked_workspace_bytes(int64_t T, int64_t B, int32_t slots, bool bf1
     const int64_t Tc = chunked_tokens(T, slots);
     if (Tc < 1) return 0;
     const int64_t nch = (Tc + kChunk - 1) / kChunk;
-    (void)bf16_rows;  // the record holds f16 planes whatever the row type
+    (void)bf16_rows;  // the same record whatever the row type
     return (size_t)B * 32 * nch * kRecBytes;
 }
 
 bool gdn_chunked_available() { return true; }
 
-template <bool BF16, bool VEC>
-static void chunked_kernels(const GdnChunkArgs& a, hipStream_t stream) {
-    launch("gdn_chunk_prep", gdn_chunk_prep<BF16, VEC>, dim3(16, a.n_chunks, (uint32_t)a.B), dim3(256), stream, a);
-    // one sequence: one scan workgroup per CU, non-temporal output stores
-    const uint32_t n_wg = (uint32_t)a.B * 32 * kColBlocks;
-    if (n_wg <= 256)
-        launch("gdn_chunk_scan", gdn_chunk_scan<BF16, VEC, true>, dim3(n_wg), dim3(256), stream, a);
+template <bool F32, int NC>
+static void scan_launch(const GdnChunkArgs& a, hipStream_t stream) {
+    const uint32_t n_wg = (uint32_t)a.B * 32 * (kColBlocks / NC);
+    if (NC > 1 || n_wg <= 256)
+        launch("gdn_chunk_scan", gdn_chunk_scan<F32, true, NC>, dim3(n_wg), dim3(256), stream, a);
     else
-        launch("gdn_chunk_scan", gdn_chunk_scan<BF16, VEC, false>, dim3(n_wg), dim3(256), stream, a);
+        launch("gdn_chunk_scan", gdn_chunk_scan<F32, false, NC>, dim3(n_wg), dim3(256), stream, a);
+}
+
+// Column tiles per scan workgroup for bf16 rows. A workgroup of one tile (66 KB of
+// LDS) takes 1.75 us per chunk alone on a CU and shares the CU evenly with a
+// second one; one of two or four tiles fetches the chunk's K, Q, T and P once for
+// them and takes 2.9 or 5.2 us, one per CU. In tenths of 0.25 us per chunk, over the
+// rounds that 256 B workgroups of one tile, 128 B of two and 64 B of four make
+// (4096 tokens, us per call with 1 / 2 / 4 tiles): 1 sequence 151 / 210 / 354, 2
+// sequences 289 / 237 / 384, 3 445 / 442 / 413, 4 584 / 480 / 439, 8 1133 / 933 / 863;
+// 5 sequences of 1000 tokens 186 / 187 / 212.
+// (f32 rows, with K in two planes, leave room for one workgroup per CU whatever the
+// tiles, so two tiles pay from two sequences on: with one and two, 2 x 2000 tokens
+// took 261 and 195 us, 3 x 1000 214 and 190, 8 x 1000 564 and 412 in one build.)
+static int scan_tiles_bf16(int B) {
+    const int one = 70 * B, two = 117 * ((B + 1) / 2), four = 209 * ((B + 3) / 4);
+    return one <= two && one <= four ? 1 : two <= four ? 2 : 4;
+}
+
+template <bool BF16>
+static void chunked_kernels(const GdnChunkArgs& a, hipStream_t stream) {
+    launch("gdn_chunk_prep", gdn_chunk_prep<BF16>, dim3(16, a.n_chunks, (uint32_t)a.B), dim3(256), stream, a);
+    int nc = BF16 ? scan_tiles_bf16(a.B) : a.B > 1 ? 2 : 1;
+    // a lane reads its columns of a V row with one load, aligned to 4 bytes
+    if (((uintptr_t)a.v | a.v_nb1 | a.v_nb2 | a.v_nb3) % 4) nc = 1;
+    if constexpr (BF16) {
+        if (nc == 4) return scan_launch<false, 4>(a, stream);
+    }
+    if (nc == 2) return scan_launch<!BF16, 2>(a, stream);
+    scan_launch<!BF16, 1>(a, stream);
 }
 
 hipError_t gdn_chunked_launch(const GdnLaunch& L, hipStream_t stream) {
@@ -1257,19 +1260,10 @@ hipError_t gdn_chunked_launch(const GdnLaunch& L, hipStream_t stream) {
     a.B = (int32_t)B;
     a.scale = 1.0f / sqrtf(128.0f);
     const bool bf16 = L.q->type == XQ_TYPE_BF16;
-    // 16-byte row loads need 16-byte aligned q/k row bases
-    bool vec = true;
-    for (const xq_tensor* t : {L.q, L.k}) {
-        vec = vec && ((uintptr_t)t->data % 16 == 0);
-        for (int i = 1; i < 4; ++i) vec = vec && (t->nb[i] % 16 == 0);
-    }
-    if (bf16) {
-        if (vec) chunked_kernels<true, true>(a, stream);
-        else chunked_kernels<true, false>(a, stream);
-    } else {
-        if (vec) chunked_kernels<false, true>(a, stream);
-        else chunked_kernels<false, false>(a, stream);
-    }
+    if (bf16)
+        chunked_kernels<true>(a, stream);
+    else
+        chunked_kernels<false>(a, stream);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || L.slots == 1) return e;
     // the last slots - 1 tokens run on the step kernel, starting from the chunked
