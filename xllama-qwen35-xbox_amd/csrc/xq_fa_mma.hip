@@ -114,14 +114,18 @@ struct DecCfg {
     // as one 1 KiB operand per (part, pair tile, block), 16 bytes per lane, then the
     // pairs' score factors; in registers beside the accumulators they would spill
     static constexpr bool QFQ = QUANT && QF;
-    static constexpr int QOPS = QFQ ? 2 * MT * NB * 1024 + 64 * MT : 0;
+    static constexpr int QOPW = 2 * MT * NB * 1024;
     static constexpr int QRB = INTQ ? D + 8 * NB : 0;       // LDS Q image row bytes (int8 path; d_q then 4*NB spare bytes that keep the stride)
     static constexpr int RING_W = 2 * 2 * SLICE;            // per wave: 2 stages x (K, V)
     static constexpr int ML = QFQ ? 0 : 2 * MT;             // mask loads per slice
     static constexpr int MASK_W = ML * 512;             // per wave: 2 stages x MT x 2 f16 pairs per lane
-    static constexpr int FIXED = NPP * QRB + QOPS + 2 * 8 * NPP * 4 + 64;
+    static constexpr int FIXED = NPP * QRB + (QFQ ? QOPW + 64 * MT : 0) + 2 * 8 * NPP * 4 + 64;
     static constexpr bool NW8 = 8 * (RING_W + MASK_W) + FIXED <= 160 * 1024 && !(MT == 2 && D == 256);
     static constexpr int NW = NW8 ? 8 : 4;
+    // Float K: the same operand image where it fits beside the rings (all but two
+    // pair tiles of f16 records); the waves then hold it in registers
+    static constexpr bool QLDS = !QUANT && NW * (RING_W + MASK_W) + QOPW + 2 * NW * NPP * 4 + 64 <= 160 * 1024;
+    static constexpr int QOPS = QFQ ? QOPW + 64 * MT : QLDS ? QOPW : 0;
     static constexpr int RING = NW * RING_W;
     static constexpr int QIMG = RING;                       // Q image after the K/V rings
     static constexpr int MASKR = QIMG + NPP * QRB + QOPS;    // mask rings after the Q image
@@ -530,12 +534,14 @@ __global__ __launch_bounds__((64 * DecCfg<KT, D, MT, QF>::NW)) void fa_dec(FaArg
     //      DMA into the wave's ring stage 1, ahead of stage 0's units, and are
     //      waited for alone (loads complete in order), so Q does not wait behind
     //      the ring; stage 1's units follow once the rows are read.
-    //      Float K: the f16 hi / lo B operands straight from Q, then the units.
-    constexpr bool QSTAGE = QUANT && PPW * D * 4 <= 2 * SLICE;
+    //      Float Q (float K, or range calls): the same rows as f16 hi + lo score
+    //      operands in LDS. Two pair tiles of f16 records leave no room for them:
+    //      there every wave forms its B operands from Q itself.
+    constexpr bool QSTAGE = (QUANT || C::QLDS) && PPW * D * 4 <= 2 * SLICE;
     uint8_t* sQ = smem + C::QIMG;
     float* sQf = (float*)(sQ + 2 * MT * NB * 1024);  // QFQ: the pairs' score factors
     h8 qh[QUANT ? 1 : MT][QUANT ? 1 : NB], ql[QUANT ? 1 : MT][QUANT ? 1 : NB];
-    if constexpr (QUANT) {
+    if constexpr (QUANT || C::QLDS) {
         constexpr int LPB = kQK / VD;
         float x[PPW][VD];
         if constexpr (QSTAGE) {
@@ -585,34 +591,41 @@ __global__ __launch_bounds__((64 * DecCfg<KT, D, MT, QF>::NW)) void fa_dec(FaArg
         for (int k = 0; k < PPW; ++k) {
             const int p = wave + k * NW;
             if (p >= NPP) break;
-            if constexpr (QFQ) {
-                // the row's power of two: its largest element (Inf as the largest
-                // finite exponent) to [2^14, 2^15); then f16 hi + lo in the score
-                // operand's layout, VD neighbouring slots of one lane's 16 bytes (one
-                // wave per pair: with every wave converting all pairs the prologue
-                // took 19 k cycles, of 47 k in all on a nine-query q4_0 call)
-                float amax = 0.0f;
+            if constexpr (!INTQ) {
+                // f16 hi + lo in the score operand's layout, VD neighbouring slots of
+                // one lane's 16 bytes (one wave per pair: with every wave converting
+                // all pairs the prologue took 19 k cycles, of 47 k in all on a
+                // nine-query q4_0 range call, and E5M2 records at D 256 21.4 against
+                // 15.6 us per 1024-row decode, f16 at D 128 13.6 against 11.1).
+                // Quantized K: the row times its power of two,
+                // its largest element (Inf as the largest finite exponent) to
+                // [2^14, 2^15).
+                int up = 0;
+                if constexpr (QFQ) {
+                    float amax = 0.0f;
 #pragma unroll
-                for (int j = 0; j < VD; ++j) amax = fmaxf(amax, fabsf(x[k][j]));
-                const int e = min((int)(__float_as_uint(wave_max(amax)) >> 23), 254);
-                const int up = 141 - e;
+                    for (int j = 0; j < VD; ++j) amax = fmaxf(amax, fabsf(x[k][j]));
+                    up = 141 - min((int)(__float_as_uint(wave_max(amax)) >> 23), 254);
+                    if (lane == 0) sQf[p] = __builtin_ldexpf(a.scale * kLog2e, -up);
+                }
                 const int el = (lane * VD) % kQK;  // in its block
                 const int slot = KT == XQ_TYPE_Q4_0 ? 8 * ((el % 16) / 4) + el / 16 * 4 + el % 4 : el;  // 8 lg + slot
                 uint8_t* op = sQ + ((p / 16) * NB + lane * VD / kQK) * 1024 + (slot / 8) * 256 + (p % 16) * 16 + (slot % 8) * 2;
                 uint32_t hb[VD], lb[VD];
 #pragma unroll
                 for (int j = 0; j < VD; ++j) {
-                    const float xv = __builtin_ldexpf(x[k][j], up);
-                    hb[j] = f32_to_f16_bits(xv);
-                    // an infinite element keeps a zero low part: its products stay infinite
-                    lb[j] = __builtin_isfinite(xv) ? f32_to_f16_bits(xv - f16_bits_to_f32(hb[j])) : 0u;
+                    const float xv = QFQ ? __builtin_ldexpf(x[k][j], up) : x[k][j];
+                    hb[j] = f32_to_f16_bits(xv);  // NaN as ggml's f16 conversion
+                    lb[j] = f32_to_f16_bits(xv - f16_bits_to_f32(hb[j]));
+                    // (quantized K: an infinite element keeps a zero low part: its
+                    // products stay infinite)
+                    if (HI_ONLY || (QFQ && !__builtin_isfinite(xv))) lb[j] = 0u;
                 }
 #pragma unroll
                 for (int j = 0; j < VD; j += 2) {
                     *(uint32_t*)(op + 2 * j) = hb[j] | (hb[j + 1] << 16);
                     *(uint32_t*)(op + MT * NB * 1024 + 2 * j) = lb[j] | (lb[j + 1] << 16);
                 }
-                if (lane == 0) sQf[p] = __builtin_ldexpf(a.scale * kLog2e, -up);
                 continue;
             }
             uint8_t* img = sQ + p * QRB;
@@ -698,6 +711,16 @@ __global__ __launch_bounds__((64 * DecCfg<KT, D, MT, QF>::NW)) void fa_dec(FaArg
     // dqb[m][q]: d_q of block 4q + lg of the lane's pair (the B operand of the
     // 4-block scale product)
     float dqb[INTQ ? MT : 1][INTQ ? NB / 4 : 1];
+    if constexpr (C::QLDS) {
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+            for (int c = 0; c < NB; ++c) {
+                const uint8_t* op = sQ + (m * NB + c) * 1024 + 16 * lane;
+                qh[m][c] = *(const h8*)op;
+                ql[m][c] = *(const h8*)(op + MT * NB * 1024);
+            }
+    }
     float qf[MT];  // QFQ: the pair's score factor, scale * log2 e / its power of two
     if constexpr (QFQ) {
 #pragma unroll
