@@ -1,0 +1,54 @@
+"""Mask rows that start in the middle of a dword (odd KV lengths, views two bytes
+into a buffer): the bits of the same mask laid out on 4 bytes, at the ends of a
+wave slice and of the call, with rows masked there."""
+import numpy as np
+import pytest
+
+import xqattn
+from conftest import case_note
+from fa_cases import dst_array, make_fa_case
+from xqattn import workloads as wl
+
+pytestmark = pytest.mark.gpu
+
+
+def _run(torch, case, mask, softcap=0.0):
+    dev = [xqattn.DevTensor.from_host(t) for t in (case.q, case.k, case.v)]
+    d = xqattn.DevTensor.empty_like_host(case.dst)
+    xqattn.flash_attn_ext(*dev, mask, None, d, xqattn.fa_params(case.scale, softcap=softcap))
+    torch.cuda.synchronize()
+    return dst_array(case, d.to_host_bytes())
+
+
+@pytest.mark.parametrize("kv", [wl.Q8_0, wl.Q4_0, wl.F16, wl.E5M2], ids=lambda t: wl.TYPE_NAME[t])
+@pytest.mark.parametrize("d,hkv,group,n_q,rows", [
+    (128, 1, 4, 1, 1), (128, 2, 2, 3, 17), (128, 2, 4, 8, 255), (256, 2, 6, 4, 129), (256, 1, 6, 2, 431),
+    (256, 1, 20, 1, 143), (128, 2, 4, 2, 256),
+])
+def test_fa_mask_alignment(torch_gpu, kv, d, hkv, group, n_q, rows):
+    torch = torch_gpu
+    cfg = wl.FaConfig("mask", n_q, hkv * group, hkv, d, rows, 1, kv, causal_prefix=max(0, rows - n_q))
+    case_note(f"mask alignment {wl.TYPE_NAME[kv]} D {d} G {group} n_q {n_q} rows {rows}")
+    case = make_fa_case(cfg, seed=51)
+    bits = wl.fa_causal_mask(cfg)[0].copy()
+    rng = np.random.RandomState(3)
+    bits[:, rng.rand(rows) < 0.2] = np.float16(-1.5).view(np.uint16)
+    if rows > 2:
+        bits[0, rows // 2] = bits[n_q - 1, 1] = 0xFC00
+    pitch = rows + (rows & 1) + 2
+    flat = np.full((n_q, pitch), 0x7E00, np.uint16)  # NaN around the rows
+    flat[:, :rows] = bits
+    def view(off, row_pitch, src):
+        buf = torch.full((off + src.size + 8,), 0x7E00, dtype=torch.int16, device="cuda")
+        buf[off:off + src.size] = torch.from_numpy(np.ascontiguousarray(src).reshape(-1).view(np.int16)).cuda()
+        t = xqattn.DevTensor(wl.F16, (rows, n_q, 1, 1), (2, 2 * row_pitch, 2 * row_pitch * n_q, 2 * row_pitch * n_q), buf)
+        t.t = buf[off:]
+        return t
+    for softcap in (0.0, 5.0):  # softcap: the rows are re-laid first
+        want = _run(torch, case, view(2, pitch, flat), softcap)
+        assert np.isfinite(want).all()
+        odd = rows + 1 - (rows & 1) if rows & 1 else rows + 1
+        tight = np.full((n_q, odd), 0x7E00, np.uint16)
+        tight[:, :rows] = bits
+        for off, p, src in ((0, odd, tight), (1, odd, tight), (1, pitch, flat)):
+            assert np.array_equal(_run(torch, case, view(off, p, src), softcap), want), (off, p, softcap)

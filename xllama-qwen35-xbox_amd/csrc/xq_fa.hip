@@ -1006,7 +1006,8 @@ hipError_t fa_launch(const FaLaunch& L, hipStream_t stream) {
                      (fa_mma_rows_ok(a.L) || L.qk_mode == kQkInt8 || (kt != XQ_TYPE_Q8_0 && kt != XQ_TYPE_Q4_0));
     if (L.engine == XQ_FA_ENGINE_MFMA && !mma) return hipErrorInvalidValue;
     if (mma) {
-        if (!fa_mma_mask_ok(a)) {
+        a.hi_only = kt != XQ_TYPE_Q8_0 && kt != XQ_TYPE_Q4_0 && L.q_round_f16 ? 1 : 0;
+        if (!fa_mma_mask_ok(a, kt, D)) {
             const size_t base = fa_workspace_bytes(n_rows, D, L.qk_mode, kt, L.n_splits);
             if (L.workspace_bytes < base + fa_mask_pack_bytes(L.mask, a.L, NQ)) return hipErrorInvalidValue;
             uint32_t* packed = (uint32_t*)(ws + base);

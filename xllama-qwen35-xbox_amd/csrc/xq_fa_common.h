@@ -28,6 +28,22 @@ template <> struct ChunkT<16> { using T = uint4; };
 template <> struct ChunkT<8> { using T = uint2; };
 template <> struct ChunkT<4> { using T = uint32_t; };
 
+// Division of numbers up to max_x by one the host knows: x / d = mulhi(x,
+// floor(2^32 / d) + 1) for x below 2^32 / d (one multiply, against about 20
+// instructions of the general division). m 0: d is 1; m 1: max_x lies beyond that,
+// the general division.
+struct UDiv {
+    uint32_t d, m;
+    UDiv() = default;
+    UDiv(uint32_t n, uint64_t max_x)
+        : d(n), m(n <= 1 ? 0u : max_x * n < ((uint64_t)1 << 32) ? (uint32_t)(((uint64_t)1 << 32) / n) + 1u : 1u) {}
+    __host__ __device__ __forceinline__ uint32_t quot(uint32_t x) const {
+        if (m == 0u) return x;
+        if (m == 1u) return x / d;
+        return (uint32_t)(((uint64_t)x * m) >> 32);
+    }
+};
+
 struct FaArgs {
     const uint8_t* k;
     const uint8_t* v;
@@ -50,7 +66,9 @@ struct FaArgs {
     int32_t H, Hkv, G, NQ, B, QT, n_qtiles, n_splits, rk3, rv3;
     float scale, softcap, max_bias, m0, m1;
     int32_t n_head_log2;
-    uint32_t g_magic;  // fa_dec: division of a pair index by G
+    // fa_dec
+    uint32_t n_wg;
+    UDiv d_tiles, d_hkv, d_splits, d_rk3, d_rv3, d_g;
     int32_t poison;
     // matrix-core engine: f32 Q rows (quantised inside the kernel), hi-only
     // f16 Q for the NATIVE policy
@@ -98,8 +116,9 @@ struct FaLaunch;
 hipError_t fa_mma_launch(FaArgs a, const FaLaunch& L, hipStream_t stream);
 // The matrix-core engine's 32-bit row indices.
 inline bool fa_mma_rows_ok(int64_t rows) { return rows < (int64_t)1 << 30; }
-// Mask layout the matrix-core engine can read (4-byte aligned rows).
-bool fa_mma_mask_ok(const FaArgs& a);
+// Whether the matrix-core engine reads the mask where it lies (else its rows are
+// re-laid on 4 bytes first).
+bool fa_mma_mask_ok(const FaArgs& a, int kt, int d);
 // Separate split-merge kernel (used when the merge cannot run inside pass 1).
 hipError_t fa_reduce_launch(const FaArgs& a, int d, hipStream_t stream);
 

@@ -99,7 +99,7 @@ constexpr float kPOff = 4.0f;          // weights are exp2(x - max - 4), in (0, 
 // Mask source of calls without a mask: one zero f16 pair.
 __device__ uint32_t g_fa_zero_mask[1];
 
-template <int KT, int D, int MT, bool QF = false>
+template <int KT, int D, int MT, bool QF = false, bool MIS = false>
 struct DecCfg {
     static constexpr int REC = rec_bytes(KT, D);
     static constexpr int SLICE = kSub * REC;
@@ -117,8 +117,11 @@ struct DecCfg {
     static constexpr int QOPW = 2 * MT * NB * 1024;
     static constexpr int QRB = INTQ ? D + 8 * NB : 0;       // LDS Q image row bytes (int8 path; d_q then 4*NB spare bytes that keep the stride)
     static constexpr int RING_W = 2 * 2 * SLICE;            // per wave: 2 stages x (K, V)
-    static constexpr int ML = QFQ ? 0 : 2 * MT;             // mask loads per slice
-    static constexpr int MASK_W = ML * 512;             // per wave: 2 stages x MT x 2 f16 pairs per lane
+    // mask dwords per lane and pair tile: its four elements; of rows that are not
+    // 4-byte aligned (MIS) the three that hold them
+    static constexpr int MD = MIS ? 3 : 2;
+    static constexpr int ML = QFQ ? 0 : MD * MT;            // mask loads per slice
+    static constexpr int MASK_W = ML * 512;                 // per wave: 2 stages x MT x MD dwords per lane
     static constexpr int FIXED = NPP * QRB + (QFQ ? QOPW + 64 * MT : 0) + 2 * 8 * NPP * 4 + 64;
     static constexpr bool NW8 = 8 * (RING_W + MASK_W) + FIXED <= 160 * 1024 && !(MT == 2 && D == 256);
     static constexpr int NW = NW8 ? 8 : 4;
@@ -350,13 +353,14 @@ XQ_DEV int acc_dim(int c, int t, int lg, int i) {
     return KT == XQ_TYPE_Q4_0 ? 32 * c + 16 * t + 4 * lg + i : 32 * c + 8 * lg + 2 * i + t;
 }
 
-template <int KT, int D, int MT, bool SOFTCAP, bool HI_ONLY, bool QF = false>
-__global__ __launch_bounds__((64 * DecCfg<KT, D, MT, QF>::NW)) void fa_dec(FaArgs a) {
-    using C = DecCfg<KT, D, MT, QF>;
+template <int KT, int D, int MT, bool SOFTCAP, bool HI_ONLY, bool QF = false, bool MIS = false>
+__global__ __launch_bounds__((64 * DecCfg<KT, D, MT, QF, MIS>::NW)) void fa_dec(FaArgs a) {
+    using C = DecCfg<KT, D, MT, QF, MIS>;
+    static_assert(C::NW == DecCfg<KT, D, MT, QF>::NW, "a query's bits do not depend on its mask's alignment");
     constexpr int REC = C::REC, SLICE = C::SLICE, CS = C::CS, CPS = C::CPS, NIS = C::NIS;
     constexpr int NB = C::NB, NPP = C::NPP, NW = C::NW, QRB = C::QRB;
     constexpr bool QUANT = C::QUANT, INTQ = C::INTQ, QFQ = C::QFQ;
-    constexpr int ML = C::ML;
+    constexpr int ML = C::ML, MD = C::MD;
     constexpr int BB = KT == XQ_TYPE_Q8_0 ? 34 : 18;
     constexpr int NT = 64 * NW;
     constexpr uint32_t kNegInfH2 = 0xfc00fc00u;  // f16 pair (-inf, -inf)
@@ -365,24 +369,27 @@ __global__ __launch_bounds__((64 * DecCfg<KT, D, MT, QF>::NW)) void fa_dec(FaArg
     __shared__ float sM[NW][NPP], sL[NW][NPP];
     __shared__ int sProg[NW];  // slices each wave has finished (issue-priority balancing)
 
-    const uint32_t n_wg = (uint32_t)a.n_splits * a.n_qtiles * a.Hkv * a.B;
-    uint32_t wg = xcd_remap(blockIdx.x, n_wg);
+    // every argument the prologue needs, asked for at once: left to their uses, the
+    // scalar loads go out one dependent group after another
+    asm volatile("" ::"s"(a.k), "s"(a.v), "s"(a.q), "s"(a.mask), "s"(a.positions), "s"(a.k_nb1), "s"(a.k_nb2), "s"(a.k_nb3),
+                 "s"(a.v_nb1), "s"(a.v_nb2), "s"(a.v_nb3), "s"(a.q_nb1), "s"(a.q_nb2), "s"(a.q_nb3), "s"(a.L), "s"(a.split_rows),
+                 "s"(a.n_wg), "s"(a.d_tiles.m), "s"(a.d_hkv.m), "s"(a.d_splits.m), "s"(a.d_rk3.m), "s"(a.d_rv3.m), "s"(a.d_g.m));
+    uint32_t wg = xcd_remap(blockIdx.x, a.n_wg);
     // logical order: pair tile fastest, then KV head, split, sequence, so the
     // heads reading the same rows are neighbours on one XCD (shared L2)
-    const int qt = wg % a.n_qtiles;
-    wg /= a.n_qtiles;
-    const int g_kv = wg % a.Hkv;
-    wg /= a.Hkv;
-    const int split = wg % a.n_splits;
-    const int b = wg / a.n_splits;
+    uint32_t rest = a.d_tiles.quot(wg);
+    const int qt = wg - rest * a.d_tiles.d;
+    wg = rest;
+    rest = a.d_hkv.quot(wg);
+    const int g_kv = wg - rest * a.d_hkv.d;
+    wg = rest;
+    const int b = a.d_splits.quot(wg);
+    const int split = wg - b * a.d_splits.d;
     // the tile's pairs: p0 .. p0 + npa - 1 of the KV head's n_q x G (query, head)
     // pairs, query-major
     const int p0 = qt * NPP;
     const int npa = min(NPP, a.NQ * a.G - p0);
-    auto pair_q = [&](int p) {
-        const uint32_t i = (uint32_t)(p0 + p);
-        return (int)(a.g_magic ? __umulhi(i, a.g_magic) : i);
-    };
+    auto pair_q = [&](int p) { return (int)a.d_g.quot((uint32_t)(p0 + p)); };
     auto pair_h = [&](int p) { return g_kv * a.G + (p0 + p) - pair_q(p) * a.G; };
     const int wave = wave_id();
     const int lane = lane_id();
@@ -409,8 +416,8 @@ __global__ __launch_bounds__((64 * DecCfg<KT, D, MT, QF>::NW)) void fa_dec(FaArg
         r_end = min(r_end, lmax);
         r_all = min(r_end, lmin);
     }
-    const uint8_t* kb = a.k + (int64_t)(b / a.rk3) * a.k_nb3 + (int64_t)g_kv * a.k_nb2;
-    const uint8_t* vb = a.v + (int64_t)(b / a.rv3) * a.v_nb3 + (int64_t)g_kv * a.v_nb2;
+    const uint8_t* kb = a.k + (int64_t)a.d_rk3.quot(b) * a.k_nb3 + (int64_t)g_kv * a.k_nb2;
+    const uint8_t* vb = a.v + (int64_t)a.d_rv3.quot(b) * a.v_nb3 + (int64_t)g_kv * a.v_nb2;
 
     // ---- per-wave ring [stage][K | V][SLICE]; chunk c = 64 i + lane of a
     //      slice is (row c / (REC/CS), byte (c % (REC/CS)) * CS)
@@ -489,30 +496,49 @@ __global__ __launch_bounds__((64 * DecCfg<KT, D, MT, QF>::NW)) void fa_dec(FaArg
     // slice's first row joins it) plus the lane's 32-bit offset moff[m] (its
     // pair's row and head, then element 4lg; the host keeps a plane below 2^31
     // bytes), so a full slice's mask loads take no vector instructions.
+    // MIS: rows that may start in the middle of a dword (odd KV lengths, views). The
+    // lane reads the dwords around its four elements, from its row's base rounded
+    // down, and shifts them together at use. A dword is read only if it holds an
+    // element of the row.
     const int mcols = a.mask ? (int)a.L : 0;
     uint8_t* mring = smem + C::MASKR + wave * C::MASK_W;
     const uint8_t* mplane = a.mask ? a.mask + (int64_t)(b % a.m_ne3) * a.m_nb3 : (const uint8_t*)g_fa_zero_mask;
+    uint32_t msh[MIS ? MT : 1];  // MIS: bytes (0 or 2) the lane's elements start into its first dword
+    if constexpr (MIS) {
+        const uint32_t sub = (uint32_t)(uintptr_t)mplane & 3u;
+        mplane -= sub;
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+            moff[m] += sub;
+            msh[m] = moff[m] & 2u;
+            moff[m] -= msh[m];
+        }
+    }
+    auto mask_slot = [&](int st, int m, int k) { return mring + ((st * MT + m) * MD + k) * 256; };
     auto load_mask = [&](int t, int st) {
         if constexpr (QFQ) return;
-        if (!a.mask) {
+        if (!MIS && !a.mask) {
 #pragma unroll
             for (int m = 0; m < MT; ++m)
 #pragma unroll
-                for (int k = 0; k < 2; ++k) lds_dma<4>(mplane, 0u, mring + (st * MT + m) * 512 + k * 256);
+                for (int k = 0; k < MD; ++k) lds_dma<4>(mplane, 0u, mask_slot(st, m, k));
         } else if (t + kSub <= mcols) {
             const uint8_t* mt = mplane + 2 * (int64_t)t;
 #pragma unroll
             for (int m = 0; m < MT; ++m)
 #pragma unroll
-                for (int k = 0; k < 2; ++k) lds_dma<4>(mt, moff[m] + 4u * k, mring + (st * MT + m) * 512 + k * 256);
+                for (int k = 0; k < MD; ++k)
+                    lds_dma<4>(mt, moff[m] + (k < 2 ? 4u * k : 4u + 2u * msh[MIS ? m : 0]), mask_slot(st, m, k));
         } else {
 #pragma unroll
             for (int m = 0; m < MT; ++m)
 #pragma unroll
-                for (int k = 0; k < 2; ++k) {
-                    const int r = t + 4 * lg + 2 * k;
-                    const uint32_t o = r < mcols ? moff[m] + (uint32_t)(2 * t + 4 * k) : moff[m] - 8u * lg;
-                    lds_dma<4>(mplane, o, mring + (st * MT + m) * 512 + k * 256);
+                for (int k = 0; k < MD; ++k) {
+                    // the dword's first element
+                    const int r = t + 4 * lg + 2 * k - (MIS ? (int)(msh[MIS ? m : 0] >> 1) : 0);
+                    const bool live = r < mcols && (k < 2 || msh[MIS ? m : 0]);
+                    const uint32_t o = live ? moff[m] + (uint32_t)(2 * t + 4 * k) : moff[m] - 8u * lg;
+                    lds_dma<4>(mplane, o, mask_slot(st, m, k));
                 }
         }
     };
@@ -1038,11 +1064,15 @@ __global__ __launch_bounds__((64 * DecCfg<KT, D, MT, QF>::NW)) void fa_dec(FaArg
         // -- the mask pairs of this slice, then the K unit (and mask) of slice j+2
         //    into the stage this slice's K and mask used
         uint32_t mw[MT][2];
-        const uint8_t* ms = mring + S * MT * 512 + 4 * lane;
 #pragma unroll
         for (int m = 0; m < MT; ++m) {
-            mw[m][0] = QFQ ? 0u : lds_u32(ms + m * 512);
-            mw[m][1] = QFQ ? 0u : lds_u32(ms + m * 512 + 256);
+#pragma unroll
+            for (int k = 0; k < 2; ++k) mw[m][k] = QFQ ? 0u : lds_u32(mask_slot(S, m, k) + 4 * lane);
+            if constexpr (MIS) {
+                const uint32_t w2 = lds_u32(mask_slot(S, m, 2) + 4 * lane);
+                mw[m][0] = __builtin_amdgcn_alignbyte(mw[m][1], mw[m][0], msh[m]);
+                mw[m][1] = __builtin_amdgcn_alignbyte(w2, mw[m][1], msh[m]);
+            }
         }
         if (n2) {
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // K and mask reads of this stage done
@@ -1437,43 +1467,49 @@ __global__ __launch_bounds__((64 * DecCfg<KT, D, MT, QF>::NW)) void fa_dec(FaArg
 
 using DecFn = void (*)(FaArgs);
 
-// Variant of (type, head dim, pair tiles) for the call's softcap and Q policy
-// (hi-only f16 Q exists for float K only; f32 Q on quantized K for range calls,
-// which have no softcap).
+// Variant of (type, head dim, pair tiles) for the call: softcap, hi-only f16 Q
+// (float K), f32 Q on quantized K (range calls, which have neither mask nor
+// softcap), mask rows that are not 4-byte aligned.
+struct DecForm {
+    bool softcap, hi_only, qf, mis;
+};
+
 template <int KT, int D, int MT>
-static DecFn dec_inst(bool softcap, bool hi_only, bool qf) {
-    if constexpr (is_quant(KT)) {
-        if (qf) {
-            if constexpr (DecCfg<KT, D, MT, true>::FITS)
-                return softcap ? nullptr : fa_dec<KT, D, MT, false, false, true>;
-            else
-                return nullptr;
-        }
+static DecFn dec_inst(const DecForm& f) {
+    constexpr bool Q = is_quant(KT);
+    if (f.qf) {
+        if constexpr (Q && DecCfg<KT, D, MT, true>::FITS)
+            return f.softcap || f.mis ? nullptr : fa_dec<KT, D, MT, false, false, true>;
+        else
+            return nullptr;
     }
-    if constexpr (DecCfg<KT, D, MT>::FITS) {
-        if constexpr (is_quant(KT)) {
-            return softcap ? fa_dec<KT, D, MT, true, false> : fa_dec<KT, D, MT, false, false>;
-        } else {
-            if (softcap) return hi_only ? fa_dec<KT, D, MT, true, true> : fa_dec<KT, D, MT, true, false>;
-            return hi_only ? fa_dec<KT, D, MT, false, true> : fa_dec<KT, D, MT, false, false>;
-        }
-    } else {
+    if (f.mis) {
+        if constexpr (DecCfg<KT, D, MT, false, true>::FITS)
+            return f.softcap || f.hi_only ? nullptr : fa_dec<KT, D, MT, false, false, false, true>;
+        else
+            return nullptr;
+    }
+    if constexpr (!DecCfg<KT, D, MT>::FITS) {
         return nullptr;
+    } else if constexpr (Q) {
+        return f.softcap ? fa_dec<KT, D, MT, true, false> : fa_dec<KT, D, MT, false, false>;
+    } else {
+        if (f.softcap) return f.hi_only ? fa_dec<KT, D, MT, true, true> : fa_dec<KT, D, MT, true, false>;
+        return f.hi_only ? fa_dec<KT, D, MT, false, true> : fa_dec<KT, D, MT, false, false>;
     }
 }
 
 template <int KT, int D>
-static DecFn dec_for(int mt, int* waves, bool softcap, bool hi_only, bool qf) {
+static DecFn dec_for(int mt, int* waves, const DecForm& f) {
     if (mt != 1 && mt != 2) return nullptr;
-    *waves = mt == 1 ? (qf ? DecCfg<KT, D, 1, true>::NW : DecCfg<KT, D, 1>::NW)
-                     : (qf ? DecCfg<KT, D, 2, true>::NW : DecCfg<KT, D, 2>::NW);
-    return mt == 1 ? dec_inst<KT, D, 1>(softcap, hi_only, qf) : dec_inst<KT, D, 2>(softcap, hi_only, qf);
+    *waves = mt == 1 ? (f.qf ? DecCfg<KT, D, 1, true>::NW : DecCfg<KT, D, 1>::NW)
+                     : (f.qf ? DecCfg<KT, D, 2, true>::NW : DecCfg<KT, D, 2>::NW);
+    return mt == 1 ? dec_inst<KT, D, 1>(f) : dec_inst<KT, D, 2>(f);
 }
 
-// qf: f32 Q on quantized K (float K always takes f32 Q)
-static DecFn dec_lookup(int kt, int d, int mt, int* waves, bool qf, bool softcap = false, bool hi_only = false) {
+static DecFn dec_lookup(int kt, int d, int mt, int* waves, const DecForm& f) {
 #define XQ_DEC_CASE(T, DD) \
-    case T: return dec_for<T, DD>(mt, waves, softcap, hi_only, qf);
+    case T: return dec_for<T, DD>(mt, waves, f);
     if (d == 128) {
         switch (kt) {
             XQ_DEC_CASE(XQ_TYPE_Q8_0, 128)
@@ -1496,12 +1532,21 @@ static DecFn dec_lookup(int kt, int d, int mt, int* waves, bool qf, bool softcap
 bool fa_mma_available(int kt, int d, int qk_mode, int n_pairs) {
     if (n_pairs < 1 || n_pairs > 32) return false;
     int w = 0;
-    return dec_lookup(kt, d, (n_pairs + 15) / 16, &w, is_quant(kt) && qk_mode != kQkInt8) != nullptr;
+    return dec_lookup(kt, d, (n_pairs + 15) / 16, &w, DecForm{false, false, is_quant(kt) && qk_mode != kQkInt8, false}) != nullptr;
 }
 
-// The mask rows are read as 4-byte pairs: every row base must be 4-byte aligned.
-bool fa_mma_mask_ok(const FaArgs& a) {
+static int pair_tiles(const FaArgs& a, int d) { return (min(a.NQ * a.G, fa_max_pairs(d, a.G)) + 15) / 16; }
+
+static bool mask_aligned(const FaArgs& a) {
     return !a.mask || ((uintptr_t)a.mask % 4 == 0 && a.m_nb1 % 4 == 0 && a.m_nb2 % 4 == 0 && a.m_nb3 % 4 == 0);
+}
+
+// The mask is read as dwords: rows that are not 4-byte aligned have a variant of
+// their own, but for softcap and hi-only Q. (Re-laying the rows first, a kernel of
+// its own, took a 377-row decode from 13.4 to 15.5 us.)
+bool fa_mma_mask_ok(const FaArgs& a, int kt, int d) {
+    int w = 0;
+    return mask_aligned(a) || dec_lookup(kt, d, pair_tiles(a, d), &w, DecForm{a.softcap != 0.0f, a.hi_only != 0, false, true}) != nullptr;
 }
 
 hipError_t fa_mma_launch(FaArgs a, const FaLaunch& L, hipStream_t stream) {
@@ -1509,26 +1554,28 @@ hipError_t fa_mma_launch(FaArgs a, const FaLaunch& L, hipStream_t stream) {
     const int kt = L.k->type;
     // tiles of 16 or 32 (query, head) pairs, packed across queries: 9 queries of 6
     // heads are 4 tiles of 16 pairs (whole queries per tile: 5)
-    const int n_pairs = a.NQ * a.G, max_pairs = fa_max_pairs(D, a.G);
-    const int mt = (min(n_pairs, max_pairs) + 15) / 16;
+    const int n_pairs = a.NQ * a.G, mt = pair_tiles(a, D);
     a.n_qtiles = (n_pairs + 16 * mt - 1) / (16 * mt);
-    // x / G = mulhi(x, floor(2^32 / G) + 1) for x below 2^32 / G (0: G is 1)
-    a.g_magic = a.G > 1 ? (uint32_t)(((uint64_t)1 << 32) / a.G) + 1u : 0u;
-    if ((uint64_t)(n_pairs + 32) * a.G >= (uint64_t)1 << 31) return hipErrorInvalidValue;
     if (!fa_mma_rows_ok(a.L)) return hipErrorInvalidValue;
-    a.hi_only = is_quant(kt) ? 0 : (L.q_round_f16 ? 1 : 0);
     int waves = 0;
-    DecFn fn = dec_lookup(kt, D, mt, &waves, is_quant(kt) && L.qk_mode != kQkInt8, a.softcap != 0.0f, a.hi_only != 0);
+    DecFn fn = dec_lookup(kt, D, mt, &waves,
+                          DecForm{a.softcap != 0.0f, a.hi_only != 0, is_quant(kt) && L.qk_mode != kQkInt8, !mask_aligned(a)});
     if (!fn) return hipErrorInvalidValue;
     a.q = (const uint8_t*)L.q->data;
     a.q_nb1 = (int64_t)L.q->nb[1];
     a.q_nb2 = (int64_t)L.q->nb[2];
     a.q_nb3 = (int64_t)L.q->nb[3];
-    if (!fa_mma_mask_ok(a)) return hipErrorInvalidValue;
     // the mask loads address a sequence's plane with 32-bit lane offsets
     if (a.mask && (int64_t)(a.NQ - 1) * a.m_nb1 + (int64_t)(a.m_ne2 - 1) * a.m_nb2 + 2 * a.L + 4 >= ((int64_t)1 << 31))
         return hipErrorInvalidValue;
     const uint32_t n_wg = (uint32_t)a.n_splits * a.n_qtiles * a.Hkv * a.B;
+    a.n_wg = n_wg;
+    a.d_tiles = UDiv(a.n_qtiles, n_wg);
+    a.d_hkv = UDiv(a.Hkv, n_wg);
+    a.d_splits = UDiv(a.n_splits, n_wg);
+    a.d_rk3 = UDiv(a.rk3, a.B);
+    a.d_rv3 = UDiv(a.rv3, a.B);
+    a.d_g = UDiv(a.G, (uint64_t)n_pairs + 16 * mt);
     launch("fa_dec", fn, dim3(n_wg), dim3(64 * waves), stream, a);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || a.n_splits == 1) return e;
