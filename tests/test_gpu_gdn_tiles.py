@@ -27,7 +27,10 @@ def _run(case, n, b0=0, v_shift=0):
         buf[v_shift:v_shift + host[2].nbytes] = dev[2].t
         dev[2].t = buf[v_shift:]
     dst = xqattn.DevTensor.from_host(part(case.dst, 2))
-    xqattn.gated_delta_net(*dev, dst, case.slots, mode=xqattn.GDN_CHUNKED)
+    # nothing of the workspace is read before it is written (0xff: NaN in every type)
+    size = xqattn.gated_delta_net_workspace(dev[0], dev[2], case.slots, xqattn.GDN_CHUNKED)
+    ws = torch.full((size + 512,), 0xff, dtype=torch.uint8, device="cuda")
+    xqattn.gated_delta_net(*dev, dst, case.slots, mode=xqattn.GDN_CHUNKED, workspace=ws)
     torch.cuda.synchronize()
     return out_array(type(case)(case.T, case.slots, n, *host, part(case.dst, 2)), dst.to_host_bytes())
 

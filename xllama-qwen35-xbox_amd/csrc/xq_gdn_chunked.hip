@@ -77,11 +77,14 @@ constexpr int kColBlocks = 128 / kCols;
 // Workspace record of one (sequence, v-head, chunk), byte offsets. Records are
 // ordered (sequence, chunk, v-head): the prep's workgroups running at a time
 // write neighbouring records.
-constexpr int kRecTHi = 0;                       // f16 [64][64]
+constexpr int kRecTHi = 0;                       // f16 tiles (8 KB apart: the hi and lo planes)
 constexpr int kRecTLo = kRecTHi + 64 * 64 * 2;
 constexpr int kRecDec = kRecTLo + 64 * 64 * 2;  // f32 e^G[64], e^{G_C - G}[64], e^{G_C}, range flag at 129, max|v|[8] at 136
 constexpr int kRecVmax = 136;                   // largest |v| of the chunk per 16-column block (floats)
 constexpr int kRecRange = 129;                  // 1.0f when the chunk's q / k leave the operands' range, else 0
+// T tile (w, j), j <= w, of rows 16w .. and columns 16j ..: [16][16] f16 in each plane;
+// the tiles above the diagonal are zero and not stored
+XQ_DEV constexpr int t_tile(int w, int j) { return (w * (w + 1) / 2 + j) * 512; }
 // P tiles: tile (w, jt), jt <= w, of scan wave w
 // is 1 KB at kRecP + (w (w + 1) / 2 + jt) KB; lane l's 16 bytes at 16 l are its
 // four values of P[16w + l % 16][16jt + 4(l / 16) + i] as f16 hi, then f16 lo
@@ -537,17 +540,20 @@ __global__ __launch_bounds__(256, BF16 ? 2 : 1) void gdn_chunk_prep(GdnChunkArgs
         uint8_t* rec = a.ws + (((int64_t)b * a.n_chunks + n) * 32 + h) * kRecBytes;
         {
             const int t = tid >> 2, j0 = 16 * (tid & 3);
+            const bool lower = j0 < 16 * (wave + 1);  // the tiles above the diagonal are zero and never read
             h8 th[2], tl[2];
 #pragma unroll
             for (int e = 0; e < 16; ++e) {
                 const float tv = sT[t * FP + j0 + e] * sBeta[e2][j0 + e];  // T = M diag(beta)
                 th[e >> 3][e & 7] = f16_hi(tv), tl[e >> 3][e & 7] = f16_lo(tv);
             }
-            const int o = (t * 64 + j0) * 2;
+            const int o = t_tile(wave, tid & 3) + 32 * (t & 15);
+            if (lower) {
 #pragma unroll
-            for (int u = 0; u < 2; ++u) {
-                *(h8*)(rec + kRecTHi + o + 16 * u) = th[u];
-                *(h8*)(rec + kRecTLo + o + 16 * u) = tl[u];
+                for (int u = 0; u < 2; ++u) {
+                    *(h8*)(rec + kRecTHi + o + 16 * u) = th[u];
+                    *(h8*)(rec + kRecTLo + o + 16 * u) = tl[u];
+                }
             }
         }
         if (tid < 64) {
@@ -668,7 +674,10 @@ XQ_DEV void scan_load(const GdnChunkArgs& a, int b, int h, int cb, int n, int wa
         const __amdgpu_buffer_rsrc_t r = rec_rsrc(rec);
 #pragma unroll
         for (int ks = 0; ks < 2; ++ks) {
-            const uint32_t o = ((uint32_t)(16 * wave + lr) * 64u + 32u * ks + 8u * lg) * 2u;
+            // (the zero tiles above the diagonal are not in memory: a lane of theirs
+            // addresses past the resource and reads 0)
+            const int j = 2 * ks + (lg >> 1);
+            const uint32_t o = j <= wave ? (uint32_t)(t_tile(wave, j) + 32 * lr + 16 * (lg & 1)) : 0x80000000u;
             L.th[ks] = __builtin_bit_cast(h8, __builtin_amdgcn_raw_buffer_load_b128(r, o, kRecTHi, 0));
             L.tl[ks] = __builtin_bit_cast(h8, __builtin_amdgcn_raw_buffer_load_b128(r, o, kRecTLo, 0));
         }
