@@ -52,3 +52,20 @@ def test_fa_mask_alignment(torch_gpu, kv, d, hkv, group, n_q, rows):
         tight[:, :rows] = bits
         for off, p, src in ((0, odd, tight), (1, odd, tight), (1, pitch, flat)):
             assert np.array_equal(_run(torch, case, view(off, p, src), softcap), want), (off, p, softcap)
+
+
+def test_fa_mask_misaligned_rows_far_apart(torch_gpu):
+    """Two mask rows 2^31 + 2 bytes apart: beyond the 32-bit offsets the kernel reads
+    masks with, so their rows are re-laid, as before."""
+    torch = torch_gpu
+    rows, n_q, pitch = 131, 2, (1 << 30) + 1
+    cfg = wl.FaConfig("mask", n_q, 4, 2, 128, rows, 1, wl.Q8_0, causal_prefix=rows - n_q)
+    case_note("mask rows 2^31 + 2 bytes apart")
+    case = make_fa_case(cfg, seed=52)
+    bits = np.ascontiguousarray(wl.fa_causal_mask(cfg)[0][:, :rows]).view(np.int16)
+    def view(row_pitch):
+        buf = torch.empty((n_q - 1) * row_pitch + rows + 9, dtype=torch.int16, device="cuda")
+        for i in range(n_q):
+            buf[i * row_pitch:i * row_pitch + rows] = torch.from_numpy(bits[i].copy()).cuda()
+        return xqattn.DevTensor(wl.F16, (rows, n_q, 1, 1), (2, 2 * row_pitch, 2 * row_pitch * n_q, 2 * row_pitch * n_q), buf)
+    assert np.array_equal(_run(torch, case, view(pitch)), _run(torch, case, view(rows + 1)))

@@ -1,6 +1,7 @@
 // xq_fa.hip — GGML_OP_FLASH_ATTN_EXT decode / short multi-query verify on gfx950.
 //
-// Three kernels per call:
+// The vector-ALU engine (fa_qprep, fa_pass1), and the kernels that the matrix-core
+// engine shares with it or needs beside its own (fa_reduce, fa_mask_pack):
 //   fa_qprep  — Q rows -> "Q image" rows in the workspace: f32 (optionally
 //               rounded to f16), or ggml q8_0 (quantize_row_q8_0, x86 rules)
 //               laid out to line up byte-for-byte with the K block layout so the
@@ -14,9 +15,11 @@
 //               value phase gives each wave a quarter of the head dims and each
 //               16-lane row a quarter of the tile rows; partial (acc, m, l) per
 //               split, or the final output when there is a single split;
-//   fa_mask_pack — only for the matrix-core engine when the mask rows are not
-//               4-byte aligned (odd KV length): copies the mask rows the call
-//               reads into 4-byte aligned rows in the workspace;
+//   fa_mask_pack — only for the matrix-core engine, for mask rows that are not
+//               4-byte aligned (odd KV length) and that fa_dec has no variant for
+//               (softcap, NATIVE policy on f16 K, a mask plane of 2^31 bytes or
+//               more): copies the rows the call reads into 4-byte aligned rows
+//               in the workspace;
 //   fa_reduce — merges the splits of one (sequence, query, head) in ascending
 //               split order (the consistent KV-reduction order of
 //               shaders/rkva/rkva_range_reduce.hlsl:12-46, with the non-finite

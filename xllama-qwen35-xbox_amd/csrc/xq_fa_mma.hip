@@ -490,8 +490,7 @@ __global__ __launch_bounds__((64 * DecCfg<KT, D, MT, QF, MIS>::NW)) void fa_dec(
     // same DMA group as K and V, so the loop holds no register-destination loads.
     // Rows at or past the mask's end read the row's first pair (they lie past every
     // pair's limit and are replaced by -inf); the pair at the last row, when L is
-    // odd, reads the aligned dword that holds it (the host requires 4-byte aligned
-    // mask rows).
+    // odd, reads the aligned dword that holds it.
     // The address is the sequence's mask plane (wave-uniform, in SGPRs; the
     // slice's first row joins it) plus the lane's 32-bit offset moff[m] (its
     // pair's row and head, then element 4lg; the host keeps a plane below 2^31
@@ -1541,12 +1540,20 @@ static bool mask_aligned(const FaArgs& a) {
     return !a.mask || ((uintptr_t)a.mask % 4 == 0 && a.m_nb1 % 4 == 0 && a.m_nb2 % 4 == 0 && a.m_nb3 % 4 == 0);
 }
 
+// The mask loads address a sequence's plane with 32-bit lane offsets.
+static bool mask_plane_ok(const FaArgs& a) {
+    return !a.mask || (int64_t)(a.NQ - 1) * a.m_nb1 + (int64_t)(a.m_ne2 - 1) * a.m_nb2 + 2 * a.L + 4 < ((int64_t)1 << 31);
+}
+
 // The mask is read as dwords: rows that are not 4-byte aligned have a variant of
-// their own, but for softcap and hi-only Q. (Re-laying the rows first, a kernel of
-// its own, took a 377-row decode from 13.4 to 15.5 us.)
+// their own, but for softcap and hi-only Q, and where the plane they lie in is too
+// wide (its re-laid rows may not be). (Re-laying the rows first, a kernel of its
+// own, took a 377-row decode from 13.4 to 15.5 us.)
 bool fa_mma_mask_ok(const FaArgs& a, int kt, int d) {
     int w = 0;
-    return mask_aligned(a) || dec_lookup(kt, d, pair_tiles(a, d), &w, DecForm{a.softcap != 0.0f, a.hi_only != 0, false, true}) != nullptr;
+    return mask_aligned(a) ||
+           (mask_plane_ok(a) &&
+            dec_lookup(kt, d, pair_tiles(a, d), &w, DecForm{a.softcap != 0.0f, a.hi_only != 0, false, true}) != nullptr);
 }
 
 hipError_t fa_mma_launch(FaArgs a, const FaLaunch& L, hipStream_t stream) {
@@ -1565,9 +1572,7 @@ hipError_t fa_mma_launch(FaArgs a, const FaLaunch& L, hipStream_t stream) {
     a.q_nb1 = (int64_t)L.q->nb[1];
     a.q_nb2 = (int64_t)L.q->nb[2];
     a.q_nb3 = (int64_t)L.q->nb[3];
-    // the mask loads address a sequence's plane with 32-bit lane offsets
-    if (a.mask && (int64_t)(a.NQ - 1) * a.m_nb1 + (int64_t)(a.m_ne2 - 1) * a.m_nb2 + 2 * a.L + 4 >= ((int64_t)1 << 31))
-        return hipErrorInvalidValue;
+    if (!mask_plane_ok(a)) return hipErrorInvalidValue;
     const uint32_t n_wg = (uint32_t)a.n_splits * a.n_qtiles * a.Hkv * a.B;
     a.n_wg = n_wg;
     a.d_tiles = UDiv(a.n_qtiles, n_wg);
