@@ -137,8 +137,9 @@ enum xq_fa_split_mode {
 };
 
 /* Which pass-1 kernel computes the scores and the value product.
- *  XQ_FA_ENGINE_AUTO: the matrix-core kernel where it exists (q8_0/q4_0 K with
- *    integer scores, F16/E5M2 K), else the VALU kernel. Its value products
+ *  XQ_FA_ENGINE_AUTO: the matrix-core kernel where it exists (every KV type; q8_0/q4_0
+ *    K with integer scores, in range calls with f32 Q as f16 hi + lo against the exact
+ *    integers), else the VALU kernel. Its value products
  *    (quantized V: weight x block scale; F16/E5M2 V: the weight) enter the
  *    matrix cores as f16 hi + lo, about 22 significant bits, against the exact
  *    V values, with f32 accumulation.

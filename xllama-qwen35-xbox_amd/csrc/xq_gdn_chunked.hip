@@ -42,7 +42,7 @@
 // so the chunk rows and T, P they share are read from HBM once.
 //
 // Against forming P and converting and transposing f32 rows in the scan: 1531 f32
-// tokens of one sequence 144 -> 100 us per call.
+// tokens of one sequence 144 -> 97 us per call (with T's ten lower tiles).
 //
 // Range. The recurrence is linear in (V, S): the scan runs on V and S times a
 // power of two 2^a per (sequence, v-head, column block), chosen from the largest
@@ -1211,8 +1211,8 @@ static void scan_launch(const GdnChunkArgs& a, hipStream_t stream) {
 // them and takes 2.9 or 5.2 us, one per CU. In tenths of 0.25 us per chunk, over the
 // rounds that 256 B workgroups of one tile, 128 B of two and 64 B of four make
 // (4096 tokens, us per call with 1 / 2 / 4 tiles): 1 sequence 151 / 210 / 354, 2
-// sequences 289 / 237 / 384, 3 445 / 442 / 413, 4 584 / 480 / 439, 8 1133 / 933 / 863;
-// 5 sequences of 1000 tokens 186 / 187 / 212.
+// sequences 289 / 237 / 384, 3 445 / 442 / 413, 4 584 / 480 / 439, 8 1133 / 933 / 863 (839
+// since T is stored as its lower tiles, which every form gains from); 5 sequences of 1000 tokens 186 / 187 / 212.
 // (f32 rows, with K in two planes, leave room for one workgroup per CU whatever the
 // tiles, so two tiles pay from two sequences on: with one and two, 2 x 2000 tokens
 // took 261 and 195 us, 3 x 1000 214 and 190, 8 x 1000 564 and 412 in one build.)

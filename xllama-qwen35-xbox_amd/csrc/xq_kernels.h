@@ -72,7 +72,8 @@ constexpr int qimg_words(int qkm, int kt, int d) {
 // 16-pair kernel variant (one wave count, one slice-to-wave assignment), so a
 // query's bits do not depend on how many queries share the call.
 constexpr int fa_max_pairs(int d, int g) { return d == 256 && g <= 16 ? 16 : 32; }
-// Queries per tile for a call with n_q queries and GQA group g.
+// Queries per tile for a call with n_q queries and GQA group g: the vector-ALU
+// engine's tiles (the matrix-core engine packs its pair tiles across queries).
 constexpr int fa_query_tile(int d, int g, int n_q) {
     return g >= fa_max_pairs(d, g) ? 1 : (fa_max_pairs(d, g) / g < n_q ? fa_max_pairs(d, g) / g : n_q);
 }
