@@ -753,19 +753,26 @@ XQ_DEV float v_value(const T& w, int ct) {
     }
 }
 
-// The token-by-token recurrence for a scan workgroup's 16 columns, in f32: the
-// chunked form's fallback for a (sequence, v-head) whose q or k rows leave
-// the range its operands hold in some chunk (qk_in_range). Lanes 16j .. 16j +
-// 15 of wave w own column 16 cb + 4w + j, lane part r its key dims 8r .. 8r +
-// 7; each token's dot products reduce over the 16 lanes.
-template <bool BF16>
-XQ_DEV void scan_sequential(const GdnChunkArgs& a, int b, int h, int cb, int wave, int lane) {
-    const int kh = h % 16, r = lane & 15, c = kCols * cb + 4 * wave + (lane >> 4);
-    const float* st = a.state + (int64_t)b * (a.s_nb3 / 4) + (int64_t)h * 16384 + (int64_t)c * 128 + 8 * r;
-    float s[8];
+// The token-by-token recurrence, in f32, for the 16-column blocks of a scan
+// workgroup that bit j of `blocks` names (block NC cb + j): the chunked form's
+// fallback where q, k, g or beta leave the range its operands hold in some chunk
+// of the (sequence, v-head), and for a block whose v or entering state holds an
+// Inf or NaN. Lanes 16i .. 16i + 15 of wave w own column 4w + i of every block,
+// lane part r its key dims 8r .. 8r + 7; each token's dot products reduce over the
+// 16 lanes. Bound by that chain, so a workgroup's blocks run in one loop, their
+// chains side by side (one after another, eight sequences of 256 bf16 tokens, four
+// blocks a workgroup, took 1805 us against 637 us with a workgroup per block).
+template <bool BF16, int NC>
+XQ_DEV void scan_sequential(const GdnChunkArgs& a, int b, int h, int cb, int wave, int lane, uint32_t blocks) {
+    const int kh = h % 16, r = lane & 15, c0 = kCols * NC * cb + 4 * wave + (lane >> 4);
+    const int64_t so = (int64_t)h * 16384 + (int64_t)c0 * 128 + 8 * r;
+    const float* st = a.state + (int64_t)b * (a.s_nb3 / 4) + so;
+    float s[NC][8];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) s[e] = st[e];
-    float* out = a.dst + (int64_t)b * (a.dst_nb2 / 4);
+    for (int j = 0; j < NC; ++j)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) s[j][e] = st[kCols * 128 * j + e];
+    float* out = a.dst + (int64_t)b * (a.dst_nb2 / 4) + h * 128 + c0;
     for (int t = 0; t < a.T; ++t) {
         float kx[8], qx[8];
         load8<BF16, false>(a.k + (int64_t)b * a.k_nb3 + (int64_t)t * a.k_nb2 + (int64_t)kh * a.k_nb1, 8 * r, kx);
@@ -773,30 +780,48 @@ XQ_DEV void scan_sequential(const GdnChunkArgs& a, int b, int h, int cb, int wav
         const float g = *(const float*)(a.g + (int64_t)b * a.g_nb3 + (int64_t)t * a.g_nb2 + (int64_t)h * a.g_nb1);
         const float be = *(const float*)(a.beta + (int64_t)b * a.b_nb3 + (int64_t)t * a.b_nb2 + (int64_t)h * a.b_nb1);
         const uint8_t* vr = a.v + (int64_t)b * a.v_nb3 + (int64_t)t * a.v_nb2 + (int64_t)h * a.v_nb1;
-        const float vv = BF16 ? bf16_bits_to_f32(((const uint16_t*)vr)[c]) : ((const float*)vr)[c];
         const float dk = expf(g);
-        float kv = 0.0f;
+        float kv[NC], y[NC];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            s[e] *= dk;
-            kv = fmaf(s[e], kx[e], kv);
+        for (int j = 0; j < NC; ++j) {
+            kv[j] = 0.0f;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                s[j][e] *= dk;
+                kv[j] = fmaf(s[j][e], kx[e], kv[j]);
+            }
         }
 #pragma unroll
-        for (int o = 1; o < 16; o <<= 1) kv += __shfl_xor(kv, o);
-        const float d = (vv - kv) * be;
-        float y = 0.0f;
+        for (int o = 1; o < 16; o <<= 1)
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            s[e] = fmaf(kx[e], d, s[e]);
-            y = fmaf(s[e], qx[e], y);
+            for (int j = 0; j < NC; ++j) kv[j] += __shfl_xor(kv[j], o);
+#pragma unroll
+        for (int j = 0; j < NC; ++j) {
+            const int c = c0 + kCols * j;
+            const float vv = BF16 ? bf16_bits_to_f32(((const uint16_t*)vr)[c]) : ((const float*)vr)[c];
+            const float d = (vv - kv[j]) * be;
+            y[j] = 0.0f;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                s[j][e] = fmaf(kx[e], d, s[j][e]);
+                y[j] = fmaf(s[j][e], qx[e], y[j]);
+            }
         }
 #pragma unroll
-        for (int o = 1; o < 16; o <<= 1) y += __shfl_xor(y, o);
-        if (r == 0) out[(int64_t)t * 4096 + h * 128 + c] = y * a.scale;
+        for (int o = 1; o < 16; o <<= 1)
+#pragma unroll
+            for (int j = 0; j < NC; ++j) y[j] += __shfl_xor(y[j], o);
+#pragma unroll
+        for (int j = 0; j < NC; ++j)
+            if (r == 0 && ((blocks >> j) & 1u)) out[(int64_t)t * 4096 + kCols * j] = y[j] * a.scale;
     }
-    float* so = a.state_out + (int64_t)b * (a.so_nb3 / 4) + (int64_t)h * 16384 + (int64_t)c * 128 + 8 * r;
+    float* sf = a.state_out + (int64_t)b * (a.so_nb3 / 4) + so;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) so[e] = s[e];
+    for (int j = 0; j < NC; ++j)
+        if ((blocks >> j) & 1u) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) sf[kCols * 128 * j + e] = s[j][e];
+        }
 }
 
 // NC: column tiles of 16 value columns per workgroup. NTY: the outputs Y are
@@ -883,10 +908,20 @@ __global__ __launch_bounds__(256) void gdn_chunk_scan(GdnChunkArgs a) {
         }
     }
     __syncthreads();
-    if (sOut) {  // workgroup-uniform
-        for (int j = 0; j < NC; ++j) scan_sequential<!F32>(a, b, h, NC * cb + j, wave, lane);
-        return;
+    // the blocks that run token by token (workgroup-uniform): all of them where q, k,
+    // g or beta leave the chunked form's range, and one whose v or entering state
+    // holds an Inf or NaN (the chunked products would carry it into earlier tokens of
+    // its chunk: a zero of T times it is NaN). They run before the chunks, which store
+    // nothing for them, so nothing of the entering state is written before it is read.
+    uint32_t seq = 0;
+#pragma unroll
+    for (int j = 0; j < NC; ++j) seq |= sOut || sAm[j] >= 0x7f800000u ? 1u << j : 0u;
+    if (seq) {
+        scan_sequential<!F32, NC>(a, b, h, cb, wave, lane, seq);
+        if (seq == (1u << NC) - 1u) return;
     }
+    const bool mine = NC == 1 || !((seq >> vb) & 1u);  // the lane's block runs in chunks
+    const int Ty = mine ? a.T : 0;                      // tokens whose outputs it stores
     int pa = 0;  // the power a of the lane's block
     {
         const uint32_t mb = sAm[vb];
@@ -1081,7 +1116,7 @@ __global__ __launch_bounds__(256) void gdn_chunk_scan(GdnChunkArgs a) {
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 const int tl = 16 * wave + 4 * lg + q;  // token within the chunk
-                if (nn * kChunk + tl < a.T) {
+                if (nn * kChunk + tl < Ty) {
                     uint32_t yv[NC];
 #pragma unroll
                     for (int ct = 0; ct < NC; ++ct) yv[ct] = __builtin_bit_cast(uint32_t, Y[ct][q] * yscale);
@@ -1160,25 +1195,13 @@ __global__ __launch_bounds__(256) void gdn_chunk_scan(GdnChunkArgs a) {
 
     // ---- final state (transposed layout: element (i, c) of head h at h*16384 + c*128 + i)
     float* so = a.state_out + (int64_t)b * (a.so_nb3 / 4) + (int64_t)h * 16384;
+    if (mine) {
 #pragma unroll
-    for (int a2 = 0; a2 < 2; ++a2)
+        for (int a2 = 0; a2 < 2; ++a2)
 #pragma unroll
-        for (int ct = 0; ct < NC; ++ct)
-            *(float4*)(so + (int64_t)(col0 + ct) * 128 + 16 * (2 * wave + a2) + 4 * lg) =
-                make_float4(S[a2][ct][0] * unscale, S[a2][ct][1] * unscale, S[a2][ct][2] * unscale, S[a2][ct][3] * unscale);
-
-    // an Inf or NaN among a column block's v or entering state: the chunked
-    // products carry it into earlier tokens of its chunk (a zero of T times it is
-    // NaN), in its own columns only, so the block runs again token by token, as
-    // the recurrence spreads it
-    bool again = false;
-#pragma unroll
-    for (int j = 0; j < NC; ++j) again |= sAm[j] >= 0x7f800000u;  // workgroup-uniform
-    if (again) {
-        __threadfence();  // the block's stores above come first
-        __syncthreads();
-        for (int j = 0; j < NC; ++j)
-            if (sAm[j] >= 0x7f800000u) scan_sequential<!F32>(a, b, h, NC * cb + j, wave, lane);
+            for (int ct = 0; ct < NC; ++ct)
+                *(float4*)(so + (int64_t)(col0 + ct) * 128 + 16 * (2 * wave + a2) + 4 * lg) =
+                    make_float4(S[a2][ct][0] * unscale, S[a2][ct][1] * unscale, S[a2][ct][2] * unscale, S[a2][ct][3] * unscale);
     }
 }
 
