@@ -69,3 +69,42 @@ def test_fa_mask_misaligned_rows_far_apart(torch_gpu):
             buf[i * row_pitch:i * row_pitch + rows] = torch.from_numpy(bits[i].copy()).cuda()
         return xqattn.DevTensor(wl.F16, (rows, n_q, 1, 1), (2, 2 * row_pitch, 2 * row_pitch * n_q, 2 * row_pitch * n_q), buf)
     assert np.array_equal(_run(torch, case, view(pitch)), _run(torch, case, view(rows + 1)))
+
+
+@pytest.mark.parametrize("kv", [wl.Q8_0, wl.Q4_0, wl.F16, wl.E5M2], ids=lambda t: wl.TYPE_NAME[t])
+@pytest.mark.parametrize("planes,step", [
+    ("seq", 2),   # one plane per sequence, nb[3] = 2 mod 4
+    ("head", 2),  # one plane per head, nb[2] = 2 mod 4
+    ("row", 1),   # strides of an odd number of bytes: elements between byte boundaries of halves
+    ("seq", 1),
+])
+def test_fa_mask_plane_strides(torch_gpu, kv, planes, step):
+    """Masks whose planes lie `step` mod 4 bytes apart: the bits of the same mask on
+    4-byte aligned rows. Two sequences, three queries, per-sequence or per-head planes."""
+    torch = torch_gpu
+    rows, n_q, heads, seqs = 141, 3, 8, 2
+    cfg = wl.FaConfig("mask", n_q, heads, 2, 128, rows, seqs, kv, causal_prefix=rows - n_q)
+    case_note(f"mask planes {planes} {step} mod 4 {wl.TYPE_NAME[kv]}")
+    case = make_fa_case(cfg, seed=53)
+    n2, n3 = (heads, 1) if planes == "head" else (1, seqs)
+    rng = np.random.RandomState(5)
+    bits = np.where(rng.rand(n3, n2, n_q, rows) < 0.3, np.uint16(0xFC00),
+                    rng.randn(n3, n2, n_q, rows).astype(np.float16).view(np.uint16)).astype(np.uint16)
+    bits[..., 7] = 0  # every query sees a row
+    def view(nb1, nb2, nb3):
+        buf = np.full(nb3 * n3 + 64, 0x7E, np.uint8)  # NaN between the rows
+        for i3 in range(n3):
+            for i2 in range(n2):
+                for i in range(n_q):
+                    at = i3 * nb3 + i2 * nb2 + i * nb1
+                    buf[at:at + 2 * rows] = bits[i3, i2, i].view(np.uint8)
+        return xqattn.DevTensor(wl.F16, (rows, n_q, n2, n3), (2, nb1, nb2, nb3), torch.from_numpy(buf).cuda())
+    row = 2 * rows + 2  # a multiple of 4
+    want = _run(torch, case, view(row, n_q * row, n2 * n_q * row))
+    assert np.isfinite(want).all()
+    nb1 = row + (step if planes == "row" else 0)
+    nb2 = n_q * nb1 + (step if planes == "head" else 0)
+    nb3 = n2 * nb2 + (step if planes == "seq" else 0)
+    assert max(nb1 % 4 if planes == "row" else 0, nb2 % 4 if planes == "head" else 0,
+               nb3 % 4 if planes == "seq" else 0) == step
+    assert np.array_equal(_run(torch, case, view(nb1, nb2, nb3)), want)

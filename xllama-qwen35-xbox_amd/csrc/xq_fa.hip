@@ -18,8 +18,8 @@
 //   fa_mask_pack — only for the matrix-core engine, for mask rows that are not
 //               4-byte aligned (odd KV length) and that fa_dec has no variant for
 //               (softcap, NATIVE policy on f16 K, a mask plane of 2^31 bytes or
-//               more): copies the rows the call reads into 4-byte aligned rows
-//               in the workspace;
+//               more, strides of an odd number of bytes): copies the rows the call
+//               reads into 4-byte aligned rows in the workspace;
 //   fa_reduce — merges the splits of one (sequence, query, head) in ascending
 //               split order (the consistent KV-reduction order of
 //               shaders/rkva/rkva_range_reduce.hlsl:12-46, with the non-finite
@@ -824,7 +824,8 @@ __global__ __launch_bounds__(256) void fa_mask_pack(const uint8_t* __restrict__ 
                                                     uint32_t* __restrict__ dst) {
     const int row = blockIdx.x / n_part;  // (b * ne2 + h) * n_q + q
     const int qi = row % n_q, h = (row / n_q) % ne2, b = row / (n_q * ne2);
-    const uint16_t* s = (const uint16_t*)(src + qi * nb1 + h * nb2 + b * nb3);
+    typedef uint16_t u16u __attribute__((aligned(1)));  // rows may start at any byte
+    const u16u* s = (const u16u*)(src + qi * nb1 + h * nb2 + b * nb3);
     const int64_t pairs = mask_pack_cols(L) / 2;
     uint32_t* d = dst + (int64_t)row * pairs;
     const int64_t c0 = (int64_t)(blockIdx.x % n_part) * kPackPairs + threadIdx.x;

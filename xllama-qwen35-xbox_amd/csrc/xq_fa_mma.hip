@@ -1546,13 +1546,14 @@ static bool mask_plane_ok(const FaArgs& a) {
 }
 
 // The mask is read as dwords: rows that are not 4-byte aligned have a variant of
-// their own, but for softcap and hi-only Q, and where the plane they lie in is too
-// wide (its re-laid rows may not be). (Re-laying the rows first, a kernel of its
-// own, took a 377-row decode from 13.4 to 15.5 us.)
+// their own, but for softcap and hi-only Q, where the plane they lie in is too
+// wide (its re-laid rows may not be), and where a row can start at an odd byte
+// (the variant takes its elements from whole halves of a dword). (Re-laying the
+// rows first, a kernel of its own, took a 377-row decode from 13.4 to 15.5 us.)
 bool fa_mma_mask_ok(const FaArgs& a, int kt, int d) {
     int w = 0;
     return mask_aligned(a) ||
-           (mask_plane_ok(a) &&
+           (mask_plane_ok(a) && (a.m_nb1 | a.m_nb2 | a.m_nb3) % 2 == 0 &&
             dec_lookup(kt, d, pair_tiles(a, d), &w, DecForm{a.softcap != 0.0f, a.hi_only != 0, false, true}) != nullptr);
 }
 
