@@ -68,6 +68,7 @@ struct FaArgs {
     int32_t n_head_log2;
     // fa_dec
     uint32_t n_wg;
+    int32_t tile_pairs;  // (query, head) pairs per tile
     UDiv d_tiles, d_hkv, d_splits, d_rk3, d_rv3, d_g;
     int32_t poison;
     // matrix-core engine: f32 Q rows (quantised inside the kernel), hi-only

@@ -387,8 +387,8 @@ __global__ __launch_bounds__((64 * DecCfg<KT, D, MT, QF, MIS>::NW)) void fa_dec(
     const int split = wg - b * a.d_splits.d;
     // the tile's pairs: p0 .. p0 + npa - 1 of the KV head's n_q x G (query, head)
     // pairs, query-major
-    const int p0 = qt * NPP;
-    const int npa = min(NPP, a.NQ * a.G - p0);
+    const int p0 = qt * a.tile_pairs;
+    const int npa = min(a.tile_pairs, a.NQ * a.G - p0);
     auto pair_q = [&](int p) { return (int)a.d_g.quot((uint32_t)(p0 + p)); };
     auto pair_h = [&](int p) { return g_kv * a.G + (p0 + p) - pair_q(p) * a.G; };
     const int wave = wave_id();
@@ -1560,10 +1560,18 @@ bool fa_mma_mask_ok(const FaArgs& a, int kt, int d) {
 hipError_t fa_mma_launch(FaArgs a, const FaLaunch& L, hipStream_t stream) {
     const int D = (int)L.q->ne[0];
     const int kt = L.k->type;
-    // tiles of 16 or 32 (query, head) pairs, packed across queries: 9 queries of 6
-    // heads are 4 tiles of 16 pairs (whole queries per tile: 5)
-    const int n_pairs = a.NQ * a.G, mt = pair_tiles(a, D);
-    a.n_qtiles = (n_pairs + 16 * mt - 1) / (16 * mt);
+    // Tiles of up to 16 or 32 (query, head) pairs. Packed across queries they are
+    // fewer (9 queries of 6 heads: 4 tiles of 16 pairs, whole queries per tile 5),
+    // which pays where it saves a round of the 256 CUs: one workgroup fits on each
+    // (8 queries of 6 heads over 4097 q8_0 rows 18.0 us packed, 26.9 us whole). Where
+    // it does not, whole queries leave less Q to convert and fewer pairs to merge per
+    // tile (64 rows 9.5 us whole, 10.2 us packed; 1025 rows 15.4 and 15.9). A pair's
+    // bits do not depend on its tile.
+    const int n_pairs = a.NQ * a.G, mt = pair_tiles(a, D), whole = a.QT * a.G;
+    auto tiles = [&](int per_tile) { return (n_pairs + per_tile - 1) / per_tile; };
+    auto rounds = [&](int per_tile) { return ((int64_t)a.n_splits * tiles(per_tile) * a.Hkv * a.B + 255) / 256; };
+    a.tile_pairs = rounds(16 * mt) < rounds(whole) ? 16 * mt : whole;
+    a.n_qtiles = tiles(a.tile_pairs);
     if (!fa_mma_rows_ok(a.L)) return hipErrorInvalidValue;
     int waves = 0;
     DecFn fn = dec_lookup(kt, D, mt, &waves,
