@@ -185,35 +185,60 @@ __global__ __launch_bounds__(256) void gdn_step_kernel(GdnStepArgs a) {
 template <bool BF16, bool VEC, int CPT>
 static void step_launch(const GdnStepArgs& a, hipStream_t stream) {
     const dim3 grid(a.B * 32 * (128 / (16 * CPT)));
-    if (a.T == 1)
-        launch("gdn_step", gdn_step_kernel<BF16, VEC, CPT, true>, grid, dim3(256), stream, a);
-    else
-        launch("gdn_step", gdn_step_kernel<BF16, VEC, CPT, false>, grid, dim3(256), stream, a);
+    if constexpr (CPT == 2 || CPT == 8) {  // step_columns' choices for one token
+        if (a.T == 1) {
+            launch("gdn_step", gdn_step_kernel<BF16, VEC, CPT, true>, grid, dim3(256), stream, a);
+            return;
+        }
+    }
+    launch("gdn_step", gdn_step_kernel<BF16, VEC, CPT, false>, grid, dim3(256), stream, a);
 }
 
-// Columns per 16-lane row. With eight, one 256-thread workgroup owns all 128
-// columns (64 KB of state) of a (sequence, v-head), so its whole state read is in
-// flight at once; 8 sequences x 32 heads are one workgroup per CU. A single token
-// is bound by that traffic: 8 sequences take 5.7 us per call with eight columns,
-// 5.8-6.8 us with two or four, 6 sequences 5.2 us with two against 5.4 us. Several
-// tokens are bound by the chain of a row's columns, run one after another for
-// every token, and by CUs that hold no workgroup: fewer columns per row pay until
-// the rows' repeated loads of q and k do not (us per call, f32 rows, with 1 / 2 / 4
-// / 8 columns):
-//   1 sequence, 5 tokens and their snapshots   5.3  5.9  7.6 10.9
-//   4 sequences, 5 tokens                     11.6  9.4  9.0 11.3
-//   1 sequence, 40 tokens                     15.7 21.9 32.9 55.3
-//   8 sequences, 40 tokens                    52.9 38.8 41.6 59.7
-//   16 sequences, 40 tokens (bf16 rows)        110   80   86   75
-static int step_columns(int T, int B) {
+// Columns per 16-lane row (same bits whatever the count). With eight, one
+// 256-thread workgroup owns all 128 columns (64 KB of state) of a (sequence,
+// v-head), so its whole state read is in flight at once; 8 sequences x 32 heads are
+// one workgroup per CU. us per call with 1 / 2 / 4 / 8 columns, f32 rows (bf16 rows
+// within a few percent, but for the last lines):
+//   one token: bound by the state's traffic
+//     6 sequences                             6.3   5.4   6.2   5.5
+//     7 sequences                             7.0   6.5   6.7   5.7
+//     8 sequences                             7.5   6.7   6.6   5.9
+//   several tokens, up to three quarters of their states kept: bound by the chain of a row's columns,
+//   run one after another for every token, and by CUs that hold no workgroup; fewer
+//   columns per row pay until the rows' repeated loads of q and k do not
+//     1 sequence, 5 tokens                    4.8   5.1   7.2  10.6
+//     4 sequences, 5 tokens                   7.6   6.8   7.9  11.1
+//     6 sequences, 5 tokens                  10.3   8.1   9.3  11.4
+//     8 sequences, 3 tokens                  11.0   7.6   7.8   9.1  (2 tokens 9.3 7.7 6.9 7.8)
+//     1 sequence, 40 tokens                  16.8  22.8  33.5  55.7
+//     8 sequences, 40 tokens                 55.9  40.3  41.7  57.6
+//     12 sequences, 40 tokens                80.4  58.9  52.7  68.4
+//     16 sequences, 40 tokens                 104  71.8  64.8  71.1  (bf16 rows 112 76.5 77.3 71.3)
+//   more of the states kept: bound by their stores as the sequences grow; eight
+//   columns store 64 KB runs (6 sequences, 8 tokens: 6 states 22.3 18.2 18.0 18.5, all
+//   eight 26.1 21.1 21.5 20.6)
+//     1 sequence, 5 tokens                    5.5   6.0   8.0  11.5
+//     3 sequences, 5 tokens                   8.8   8.1   8.4  11.9  (17 tokens 22.2 21.5 19.4 30.4)
+//     4 sequences, 3 tokens                   8.8   7.2   7.2   8.9
+//     4 sequences, 5 tokens                  11.5   9.7   9.4  12.0
+//     5 sequences, 2 tokens                   9.2   7.0   7.6   7.4
+//     5 sequences, 8 tokens                  21.1  18.2  18.9  17.1
+//     8 sequences, 8 tokens                  35.7  31.3  28.4  27.9
+//     10 sequences, 8 tokens                 43.6  37.7  35.1  38.6
+//     16 sequences, 8 tokens                 70.1  66.5  59.4  57.2
+static int step_columns(int T, int B, int kept) {
     if (T == 1) return B <= 6 ? 2 : 8;
-    if (T <= 8) return B <= 1 ? 1 : B <= 4 ? 2 : B <= 12 ? 4 : 8;
+    if (4 * kept > 3 * T) {
+        if (B <= 4) return B == 1 ? 1 : B == 2 ? 2 : T <= (B == 3 ? 8 : 3) ? 2 : 4;
+        return B <= 8 ? (T == 2 && B <= 6 ? 2 : 8) : B <= 12 ? 4 : 8;
+    }
+    if (T <= 8) return B == 1 ? 1 : B <= 6 ? 2 : B <= 12 ? 4 : 8;
     return B <= 3 ? 1 : B <= 8 ? 2 : B <= 12 ? 4 : 8;
 }
 
 template <bool BF16, bool VEC>
 static void step_dispatch(const GdnStepArgs& a, hipStream_t stream) {
-    switch (step_columns(a.T, a.B)) {
+    switch (step_columns(a.T, a.B, min(a.slots, a.T))) {
     case 1: step_launch<BF16, VEC, 1>(a, stream); break;
     case 2: step_launch<BF16, VEC, 2>(a, stream); break;
     case 4: step_launch<BF16, VEC, 4>(a, stream); break;
