@@ -1,5 +1,5 @@
-"""The KV append's units: a wave converts 256-element units, one or four of them
-by the size of the call, so records end inside units and calls inside waves.
+"""The KV append's units: a wave converts 256-element units, one or (large appends to
+records of 16 or 32 bits per element) four of them, so records end inside units and calls inside waves.
 Bytes against the oracle's quantizers."""
 import numpy as np
 import pytest

@@ -45,7 +45,7 @@ typedef uint32_t u32x4u __attribute__((ext_vector_type(4), aligned(1)));
 // consecutive elements: a wave's load is 1 KiB of contiguous source, and a
 // 32-element block is eight lanes, whose maximum takes three DPP steps and no
 // LDS. UN such 256-element units per wave, every load issued before the first is
-// used. 8192 tokens x 4 heads x 256 to q8_0 (42.5 MB): 10.2 us per launch (4.2
+// used. 8192 tokens x 4 heads x 256 to q8_0 (42.5 MB): 9.2 us per launch (4.6
 // TB/s), against 30 us with one lane per 32-element block behind an LDS copy of
 // the record (one record per wave, eight of its 64 lanes at work).
 template <int KT, int D, int UN>
@@ -160,13 +160,25 @@ template <int KT, int D>
 static void kv_store_dispatch(const float* src, const int32_t* positions, int64_t n_rec, int32_t n_head_kv,
                               int32_t q8_variant, uint8_t* dst, int32_t capacity, hipStream_t stream) {
     const int64_t units = (n_rec + 256 / D - 1) / (256 / D);
-    // four units per wave once that still gives every CU four workgroups
-    if (units >= 256 * 4 * 4 * 4)
-        launch("kv_store", kv_store_kernel<KT, D, 4>, dim3((uint32_t)((units + 15) / 16)), dim3(256), stream, src,
-               positions, (uint32_t)n_rec, (uint32_t)n_head_kv, q8_variant, dst, capacity);
-    else
-        launch("kv_store", kv_store_kernel<KT, D, 1>, dim3((uint32_t)((units + 3) / 4)), dim3(256), stream, src,
-               positions, (uint32_t)n_rec, (uint32_t)n_head_kv, q8_variant, dst, capacity);
+    // Records of 16 and 32 bits per element: four units per wave once that still gives
+    // every CU four workgroups. The narrower ones, whose conversion takes longer than
+    // their loads, one unit whatever the size: more waves hide it better. us per append
+    // of K and V, 4 heads x 256, with 1 / 2 / 4 units:
+    //   tokens       f16               f32               e5m2              q8_0              q4_0
+    //   3000    8.2  8.5  8.6   10.1 10.4 10.3    9.4  9.8 10.4    9.2  9.3 10.1    9.1  9.3  9.7
+    //   6000   15.8 15.5 15.5   18.7 18.1 17.3   15.8 17.2 17.9   15.2 16.6 17.8   15.4 16.3 17.1
+    //   8192   20.8 19.8 18.9   23.7 23.0 22.1   19.7 20.7 22.4   19.0 20.2 21.6   18.8 19.6 20.9
+    //   16384  35.2 33.1 33.2   43.2 41.3 45.4   32.8 34.0 35.4   31.4 32.7 34.2   31.7 32.5 31.7
+    constexpr bool wide = KT == XQ_TYPE_F32 || KT == XQ_TYPE_F16 || KT == XQ_TYPE_BF16;
+    if constexpr (wide) {
+        if (units >= 256 * 4 * 4 * 4) {
+            launch("kv_store", kv_store_kernel<KT, D, 4>, dim3((uint32_t)((units + 15) / 16)), dim3(256), stream, src,
+                   positions, (uint32_t)n_rec, (uint32_t)n_head_kv, q8_variant, dst, capacity);
+            return;
+        }
+    }
+    launch("kv_store", kv_store_kernel<KT, D, 1>, dim3((uint32_t)((units + 3) / 4)), dim3(256), stream, src,
+           positions, (uint32_t)n_rec, (uint32_t)n_head_kv, q8_variant, dst, capacity);
 }
 
 template <int KT>
