@@ -44,15 +44,16 @@ def test_gdn_chunked_nonfinite_block_in_place(torch_gpu, tokens, bf16):
     assert _same(got, want)
 
 
-@pytest.mark.parametrize("bf16,seqs", [(True, 2), (True, 8), (False, 2)])
-def test_gdn_chunked_several_nonfinite_blocks(torch_gpu, bf16, seqs):
-    """Two blocks of one workgroup, all blocks of one, and none."""
+@pytest.mark.parametrize("bf16,seqs,tokens", [(True, 2, 131), (True, 2, 965), (True, 8, 131), (False, 2, 131)])
+def test_gdn_chunked_several_nonfinite_blocks(torch_gpu, bf16, seqs, tokens):
+    """Two blocks of one workgroup, all blocks of one, and none (two bf16 sequences take
+    two column tiles from 16 chunks on)."""
     def edit(v, st):
         v[1, 70, 3, 5] = np.nan
         v[1, 3, 3, 55] = np.inf
         st[0, 9, ::16, 1] = -np.inf
-    case_note(f"several non-finite blocks bf16 {bf16} B {seqs}")
-    case = make_gdn_case(131, 1, B=seqs, bf16=bf16, vs_edit=edit)
+    case_note(f"several non-finite blocks bf16 {bf16} B {seqs} T {tokens}")
+    case = make_gdn_case(tokens, 1, B=seqs, bf16=bf16, vs_edit=edit)
     alone = np.concatenate([_run(case, 1, b) for b in range(seqs)])
     assert np.isnan(alone).any()
     assert _same(_run(case, seqs), alone)

@@ -68,3 +68,14 @@ def test_gdn_chunked_tiles_nonfinite_block(torch_gpu, bf16):
     got = _run(case, 4)
     assert np.array_equal(got.view(np.uint32)[~np.isnan(got)], alone.view(np.uint32)[~np.isnan(got)])
     assert np.array_equal(np.isnan(got), np.isnan(alone))
+
+
+@pytest.mark.parametrize("pad", [0, 3])
+@pytest.mark.parametrize("tokens", [960, 965, 1025])  # 15, 16 and 17 chunks
+def test_gdn_chunked_tiles_long_bf16(torch_gpu, tokens, pad):
+    """Two and six bf16 sequences take two column tiles from 16 chunks on, one below."""
+    case_note(f"column tiles long T {tokens} pad {pad}")
+    case = make_gdn_case(tokens, 1, B=6, bf16=True, pad=pad)
+    alone = np.concatenate([_run(case, 1, b) for b in range(6)])
+    for n in (2, 6):
+        assert np.array_equal(_run(case, n), alone[:n]), f"{n} sequences"

@@ -1231,23 +1231,33 @@ static void scan_launch(const GdnChunkArgs& a, hipStream_t stream) {
 // Column tiles per scan workgroup for bf16 rows. A workgroup of one tile (66 KB of
 // LDS) takes 1.75 us per chunk alone on a CU and shares the CU evenly with a
 // second one; one of two or four tiles fetches the chunk's K, Q, T and P once for
-// them and takes 2.9 or 5.2 us, one per CU. In tenths of 0.25 us per chunk, over the
-// rounds that 256 B workgroups of one tile, 128 B of two and 64 B of four make
-// (4096 tokens, us per call with 1 / 2 / 4 tiles): 1 sequence 151 / 210 / 354, 2
-// sequences 289 / 237 / 384, 3 445 / 442 / 413, 4 584 / 480 / 439, 8 1133 / 933 / 863 (839
-// since T is stored as its lower tiles, which every form gains from); 5 sequences of 1000 tokens 186 / 187 / 212.
+// them and takes 2.9 or 5.2 us, one per CU. The sums below are the us of a
+// 2000-token call: 62 per sequence with one tile, 117 per pair of sequences with two,
+// 207 per four with four; below 16 chunks, where the one-tile form's operands stay
+// in the caches, 58. Measured, us per call with 1 / 2 / 4 tiles:
+//   sequences   300 tokens          1000 tokens         2000 tokens
+//   1           28    34    45      50    68   103      84   116   186
+//   2           37    36    48      72    72   106     128   130   196   (4000: 253 244 371)
+//   3           47    54    49     103   123   112     191   229   212
+//   4           57    59    54     129   131   119     247   239   220
+//   5           66    74    81     158   182   208     324   342   396
+//   6           72    75    81     189   190   215     379   355   408
+//   7           84    95    86     221   240   223     439   455   422
+//   8           91    95    87     252   245   227     518   468   435
+//   9          100   113   116     290   300   317     559   567   605
+//   10         111   118   119     321   308   324     616   578   616
 // (f32 rows, with K in two planes, leave room for one workgroup per CU whatever the
 // tiles, so two tiles pay from two sequences on: with one and two, 2 x 2000 tokens
-// took 261 and 195 us, 3 x 1000 214 and 190, 8 x 1000 564 and 412 in one build.)
-static int scan_tiles_bf16(int B) {
-    const int one = 70 * B, two = 117 * ((B + 1) / 2), four = 209 * ((B + 3) / 4);
+// took 234 and 178 us, 3 x 1000 191 and 172, 8 x 1000 510 and 376.)
+static int scan_tiles_bf16(int B, int n_chunks) {
+    const int one = (n_chunks < 16 ? 58 : 62) * B, two = 117 * ((B + 1) / 2), four = 207 * ((B + 3) / 4);
     return one <= two && one <= four ? 1 : two <= four ? 2 : 4;
 }
 
 template <bool BF16>
 static void chunked_kernels(const GdnChunkArgs& a, hipStream_t stream) {
     launch("gdn_chunk_prep", gdn_chunk_prep<BF16>, dim3(16, a.n_chunks, (uint32_t)a.B), dim3(256), stream, a);
-    int nc = BF16 ? scan_tiles_bf16(a.B) : a.B > 1 ? 2 : 1;
+    int nc = BF16 ? scan_tiles_bf16(a.B, a.n_chunks) : a.B > 1 ? 2 : 1;
     // a lane reads its columns of a V row with one load, aligned to 4 bytes
     if (((uintptr_t)a.v | a.v_nb1 | a.v_nb2 | a.v_nb3) % 4) nc = 1;
     if constexpr (BF16) {
