@@ -108,3 +108,31 @@ def test_fa_mask_plane_strides(torch_gpu, kv, planes, step):
     assert max(nb1 % 4 if planes == "row" else 0, nb2 % 4 if planes == "head" else 0,
                nb3 % 4 if planes == "seq" else 0) == step
     assert np.array_equal(_run(torch, case, view(nb1, nb2, nb3)), want)
+
+
+def test_fa_mask_relay_many_rows(torch_gpu):
+    """2^23 mask rows of 1025 elements to re-lay (softcap, rows of 2 mod 4 bytes): two
+    parts a row would be 2^24 workgroups of 256 threads, one more than a launch
+    holds. Every sequence reads the same Q, K, V and mask (strides of 0), so all of
+    them give the bits of the call with one."""
+    torch = torch_gpu
+    rows, n_q, heads, d, seqs = 1025, 8, 32, 128, 32768
+    cfg = wl.FaConfig("many", n_q, heads, 1, d, rows, 1, wl.F16, causal_prefix=rows - n_q)
+    case_note("2^23 mask rows to re-lay")
+    case = make_fa_case(cfg, seed=54)
+    params = xqattn.fa_params(case.scale, softcap=5.0, split_mode=xqattn.SPLIT_NONE)
+    q, k, v, m = (xqattn.DevTensor.from_host(t) for t in (case.q, case.k, case.v, case.mask))
+    one = xqattn.DevTensor.empty_like_host(case.dst)
+    xqattn.flash_attn_ext(q, k, v, m, None, one, params)
+    many = [xqattn.DevTensor(t.type, (*t.ne[:3], seqs), (*t.nb[:3], 0), t.t) for t in (q,)]
+    many += [k, v, xqattn.DevTensor(m.type, (rows, n_q, heads, seqs), (2, m.nb[1], 0, 0), m.t)]
+    assert m.nb[1] == 2 * rows
+    out = torch.zeros(seqs, n_q * heads * d, dtype=torch.float32, device="cuda")
+    dst = xqattn.DevTensor(wl.F32, (d, heads, n_q, seqs), (4, 4 * d, 4 * d * heads, 4 * d * heads * n_q),
+                           out.view(torch.uint8).reshape(-1))
+    xqattn.flash_attn_ext(*many, None, dst, params)
+    torch.cuda.synchronize()
+    want = one.t.view(torch.int32).reshape(-1)
+    assert (want != 0).any()
+    for s in range(0, seqs, 1024):
+        assert (out[s:s + 1024].view(torch.int32) == want).all(), f"sequences from {s}"

@@ -828,14 +828,15 @@ __global__ __launch_bounds__(256) void fa_mask_pack(const uint8_t* __restrict__ 
     const u16u* s = (const u16u*)(src + qi * nb1 + h * nb2 + b * nb3);
     const int64_t pairs = mask_pack_cols(L) / 2;
     uint32_t* d = dst + (int64_t)row * pairs;
-    const int64_t c0 = (int64_t)(blockIdx.x % n_part) * kPackPairs + threadIdx.x;
+    for (int64_t c0 = (int64_t)(blockIdx.x % n_part) * kPackPairs; c0 < pairs; c0 += (int64_t)n_part * kPackPairs) {
 #pragma unroll
-    for (int i = 0; i < kPackPairs / 256; ++i) {
-        const int64_t c = c0 + 256 * i;
-        if (c >= pairs) break;
-        const uint32_t lo = s[2 * c];
-        const uint32_t hi = 2 * c + 1 < L ? s[2 * c + 1] : 0xFC00u;
-        d[c] = lo | (hi << 16);
+        for (int i = 0; i < kPackPairs / 256; ++i) {
+            const int64_t c = c0 + 256 * i + threadIdx.x;
+            if (c >= pairs) break;
+            const uint32_t lo = s[2 * c];
+            const uint32_t hi = 2 * c + 1 < L ? s[2 * c + 1] : 0xFC00u;
+            d[c] = lo | (hi << 16);
+        }
     }
 }
 
@@ -1016,7 +1017,10 @@ hipError_t fa_launch(const FaLaunch& L, hipStream_t stream) {
             if (L.workspace_bytes < base + fa_mask_pack_bytes(L.mask, a.L, NQ)) return hipErrorInvalidValue;
             uint32_t* packed = (uint32_t*)(ws + base);
             const int n_pack = NQ * a.m_ne2 * a.m_ne3;
-            const uint32_t n_part = (uint32_t)((mask_pack_cols(a.L) / 2 + kPackPairs - 1) / kPackPairs);
+            // (a launch holds less than 2^32 threads: with that many rows a workgroup
+            // takes several parts of one)
+            const int64_t parts = (mask_pack_cols(a.L) / 2 + kPackPairs - 1) / kPackPairs;
+            const uint32_t n_part = (uint32_t)max((int64_t)1, min(parts, (int64_t)0xffffff / n_pack));
             launch("fa_mask_pack", fa_mask_pack, dim3((uint32_t)n_pack * n_part), dim3(256), stream, a.mask, a.m_nb1,
                    a.m_nb2, a.m_nb3, NQ, a.m_ne2, a.L, n_part, packed);
             a.mask = (const uint8_t*)packed;
