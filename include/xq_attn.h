@@ -230,6 +230,18 @@ xq_status xq_fa_range(const float* q, const int32_t* positions, int32_t n_q, int
                       int32_t kv_type, int32_t origin, int32_t active, float kq_scale,
                       int32_t split_mode, float* out, float* lse, void* workspace,
                       size_t workspace_bytes, void* stream);
+/* xq_fa_range with the engine chosen as in xq_fa_params (xq_fa_range takes AUTO).
+ * On q8_0 / q4_0 storage the matrix-core engine holds a Q row as f16 hi + lo
+ * scaled by one power of two and the products weight x V block scale as f16 hi + lo
+ * scaled by another; the VALU engine keeps both as single f32 values. Against
+ * float64 the matrix cores are the closer on rows whose parts are of like size
+ * (3.4e-7 against 6.4e-7); a 32-channel block of V 2^-14 of its row's largest
+ * comes out within 5e-5 of itself, within 2e-6 with the VALU engine. */
+xq_status xq_fa_range_engine(const float* q, const int32_t* positions, int32_t n_q, int32_t n_head,
+                             const void* k, const void* v, int32_t n_head_kv, int32_t head_dim,
+                             int32_t kv_type, int32_t origin, int32_t active, float kq_scale,
+                             int32_t split_mode, int32_t engine, float* out, float* lse, void* workspace,
+                             size_t workspace_bytes, void* stream);
 
 /* Merge of position-split results: n_parts results of the same rows
  * (query, head) over disjoint KV ranges, each OUT [rows][head_dim] F32 and

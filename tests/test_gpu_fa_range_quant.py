@@ -13,13 +13,14 @@ from xqattn import workloads as wl
 pytestmark = pytest.mark.gpu
 
 
-def _call(torch, q, positions, kraw, vraw, hkv, kv, origin, active, scale, split=xqattn.SPLIT_AUTO):
+def _call(torch, q, positions, kraw, vraw, hkv, kv, origin, active, scale, split=xqattn.SPLIT_AUTO,
+          engine=xqattn.ENGINE_AUTO):
     n_q, n_head, d = q.shape
     out = torch.empty(n_q, n_head, d, dtype=torch.float32, device="cuda")
     lse = torch.empty(n_q, n_head, dtype=torch.float32, device="cuda")
     xqattn.fa_range(torch.from_numpy(q).cuda(), torch.from_numpy(positions).cuda(), n_head,
                     torch.from_numpy(kraw.reshape(-1)).cuda(), torch.from_numpy(vraw.reshape(-1)).cuda(),
-                    hkv, d, kv, origin, active, scale, out, lse, split_mode=split)
+                    hkv, d, kv, origin, active, scale, out, lse, split_mode=split, engine=engine)
     torch.cuda.synchronize()
     return out.cpu().numpy(), lse.cpu().numpy()
 
@@ -69,3 +70,34 @@ def test_fa_range_quant_nonfinite_query_stays_in_its_rows(torch_gpu, kv, bad):
     assert np.isnan(got[0, 7]).all() and np.isnan(lse[0, 7])
     got[0, 7], lse[0, 7] = clean[0, 7], clse[0, 7]
     assert np.array_equal(got, clean) and np.array_equal(lse, clse)
+
+
+@pytest.mark.parametrize("split", [xqattn.SPLIT_NONE, xqattn.SPLIT_REFERENCE], ids=["one_split", "splits"])
+@pytest.mark.parametrize("kv", [wl.Q8_0, wl.Q4_0], ids=lambda t: wl.TYPE_NAME[t])
+@pytest.mark.parametrize("d,hkv,group,n_q,active", [
+    (128, 2, 1, 1, 17), (128, 2, 4, 8, 300), (128, 1, 12, 2, 64), (256, 4, 6, 9, 1000), (256, 1, 20, 2, 515),
+    (256, 2, 3, 1, 1),
+])
+def test_fa_range_quant_engines(torch_gpu, kv, d, hkv, group, n_q, active, split):
+    """The vector-ALU form (f32 Q and f32 products, which AUTO leaves to ranges beyond
+    the matrix cores' row indices) and the matrix-core form: both within 1e-5 of
+    float64, and a query's limit inside, before and past the rows."""
+    n_head, origin, scale = hkv * group, 500, float(1.0 / np.sqrt(d))
+    kraw = oracle.quantize(kv, wl.normal(31, (active, hkv, d)))
+    vraw = oracle.quantize(kv, wl.normal(32, (active, hkv, d)))
+    q = wl.normal(33, (n_q, n_head, d))
+    positions = np.arange(origin + active - n_q, origin + active, dtype=np.int32)
+    if n_q > 2:
+        positions[:3] = origin + active // 2, origin - 1, origin + 5 * active
+    kf = oracle.dequant(kv, kraw.reshape(-1, kraw.shape[-1]), d).reshape(active, hkv, d)
+    vf = oracle.dequant(kv, vraw.reshape(-1, vraw.shape[-1]), d).reshape(active, hkv, d)
+    ref, rlse = range_f64(q, positions, n_head, kf, vf, hkv, origin, active, scale)
+    seen = np.isfinite(rlse)
+    for engine in (xqattn.ENGINE_VALU, xqattn.ENGINE_MFMA):
+        case_note(f"range quant {wl.TYPE_NAME[kv]} D {d} G {group} n_q {n_q} split {split} engine {engine}")
+        got, lse = _call(torch_gpu, q, positions, kraw, vraw, hkv, kv, origin, active, scale, split, engine)
+        assert np.abs(got - ref).max() < 1e-5 * np.abs(ref).max()
+        assert np.array_equal(np.isfinite(lse), seen)
+        assert np.abs(lse[seen] - rlse[seen]).max() < 1e-5 * np.abs(rlse[seen]).max()
+    auto = _call(torch_gpu, q, positions, kraw, vraw, hkv, kv, origin, active, scale, split)
+    assert np.array_equal(auto[0], got) and np.array_equal(auto[1], lse), "AUTO is the matrix cores"

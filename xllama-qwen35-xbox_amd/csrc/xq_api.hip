@@ -443,11 +443,11 @@ xq_status xq_fa_range_workspace(int32_t n_q, int32_t n_head, int32_t n_head_kv, 
     return ok();
 }
 
-xq_status xq_fa_range(const float* q, const int32_t* positions, int32_t n_q, int32_t n_head,
-                      const void* k, const void* v, int32_t n_head_kv, int32_t head_dim,
-                      int32_t kv_type, int32_t origin, int32_t active, float kq_scale,
-                      int32_t split_mode, float* out, float* lse, void* workspace,
-                      size_t workspace_bytes, void* stream) {
+xq_status xq_fa_range_engine(const float* q, const int32_t* positions, int32_t n_q, int32_t n_head,
+                             const void* k, const void* v, int32_t n_head_kv, int32_t head_dim,
+                             int32_t kv_type, int32_t origin, int32_t active, float kq_scale,
+                             int32_t split_mode, int32_t engine, float* out, float* lse, void* workspace,
+                             size_t workspace_bytes, void* stream) {
     if (!q || !positions || !k || !v || !out || !lse) return fail(XQ_ERR_BAD_ARG, "null pointer");
     if (n_q < 1 || n_head < 1 || n_head_kv < 1 || active < 0) return fail(XQ_ERR_BAD_ARG, "bad range arguments");
     xq_tensor tq, tk, tv, td;
@@ -455,6 +455,7 @@ xq_status xq_fa_range(const float* q, const int32_t* positions, int32_t n_q, int
     xq_fa_params p{};
     p.scale = kq_scale;
     p.split_mode = split_mode;
+    p.engine = engine;
     FaPlan P;
     xq_status st = fa_check(&tq, &tk, &tv, nullptr, nullptr, &td, &p, &P);
     if (st != XQ_OK) return st;
@@ -475,7 +476,7 @@ xq_status xq_fa_range(const float* q, const int32_t* positions, int32_t n_q, int
     L.n_splits = P.n_splits;
     L.split_rows = P.split_rows;
     L.poison = 1;
-    L.engine = XQ_FA_ENGINE_AUTO;
+    L.engine = engine;
     L.positions = positions;
     L.origin = origin;
     L.workspace = workspace;
@@ -483,6 +484,15 @@ xq_status xq_fa_range(const float* q, const int32_t* positions, int32_t n_q, int
     const hipError_t e = xq::fa_launch(L, (hipStream_t)stream);
     if (e != hipSuccess) return fail(XQ_ERR_HIP, "fa_range launch: %s", hipGetErrorString(e));
     return ok();
+}
+
+xq_status xq_fa_range(const float* q, const int32_t* positions, int32_t n_q, int32_t n_head,
+                      const void* k, const void* v, int32_t n_head_kv, int32_t head_dim,
+                      int32_t kv_type, int32_t origin, int32_t active, float kq_scale,
+                      int32_t split_mode, float* out, float* lse, void* workspace,
+                      size_t workspace_bytes, void* stream) {
+    return xq_fa_range_engine(q, positions, n_q, n_head, k, v, n_head_kv, head_dim, kv_type, origin, active, kq_scale,
+                              split_mode, XQ_FA_ENGINE_AUTO, out, lse, workspace, workspace_bytes, stream);
 }
 
 // ------------------------------------------------------------ gated delta net

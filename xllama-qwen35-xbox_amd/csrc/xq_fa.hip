@@ -1004,7 +1004,7 @@ hipError_t fa_launch(const FaLaunch& L, hipStream_t stream) {
         a.part_ml = (float2*)(ws + off);
     }
 
-    // f32 Q on quantized K (range calls) keeps the VALU engine only for rows beyond
+    // f32 Q on quantized K (range calls): under AUTO the VALU engine only for rows beyond
     // the matrix-core engine's 32-bit indices: 28 672 q8_0 rows, 24 over 4 heads at
     // D 256, one query, fa_dec 20.8 us against 76 us and 4.7 us for the Q image
     const bool mma = L.engine != XQ_FA_ENGINE_VALU && fa_mma_available(kt, D, L.qk_mode, QT * G) &&

@@ -38,7 +38,7 @@ ENGINE_AUTO, ENGINE_MFMA, ENGINE_VALU = 0, 1, 2
 EXPORTS = (
     "xq_supports_flash_attn_ext", "xq_flash_attn_ext_workspace", "xq_flash_attn_ext",
     "xq_flash_attn_ext_noalloc",
-    "xq_fa_range_workspace", "xq_fa_range", "xq_fa_lse_merge", "xq_fa_split_count", "xq_fa_split_rows",
+    "xq_fa_range_workspace", "xq_fa_range", "xq_fa_range_engine", "xq_fa_lse_merge", "xq_fa_split_count", "xq_fa_split_rows",
     "xq_fa_params_from_env",
     "xq_supports_gated_delta_net", "xq_gated_delta_net_workspace", "xq_gated_delta_net",
     "xq_kv_store", "xq_kv_record_bytes", "xq_last_error", "xq_abi_version",
@@ -125,6 +125,7 @@ def load() -> ctypes.CDLL:
         "xq_flash_attn_ext_noalloc": (i32, [T, T, T, T, T, T, P, FP, P]),
         "xq_fa_range_workspace": (i32, [i32, i32, i32, i32, i32, i32, i32, ctypes.POINTER(sz)]),
         "xq_fa_range": (i32, [P, P, i32, i32, P, P, i32, i32, i32, i32, i32, f32, i32, P, P, P, sz, P]),
+        "xq_fa_range_engine": (i32, [P, P, i32, i32, P, P, i32, i32, i32, i32, i32, f32, i32, i32, P, P, P, sz, P]),
         "xq_fa_lse_merge": (i32, [P, P, i32, i64, i32, P, P, P]),
         "xq_fa_split_count": (i32, [i64, i32]),
         "xq_fa_split_rows": (i64, [i64, i32]),
@@ -281,7 +282,7 @@ def flash_attn_ext_noalloc(q: DevTensor, k: DevTensor, v: DevTensor, mask, sinks
 
 
 def fa_range(q, positions, n_head, k, v, n_head_kv, head_dim, kv_type, origin, active, kq_scale,
-             out, lse, split_mode=SPLIT_AUTO, workspace=None, stream=None):
+             out, lse, split_mode=SPLIT_AUTO, workspace=None, stream=None, engine=ENGINE_AUTO):
     lib = load()
     n_q = positions.numel()
     n = ctypes.c_size_t(0)
@@ -289,10 +290,11 @@ def fa_range(q, positions, n_head, k, v, n_head_kv, head_dim, kv_type, origin, a
                                      ctypes.byref(n)), "fa_range_workspace")
     ws = _workspace(n.value + 256, workspace)
     wp, wn = _aligned_ptr(ws)
-    _check(lib.xq_fa_range(q.data_ptr(), positions.data_ptr(), n_q, n_head, k.data_ptr(), v.data_ptr(),
-                           n_head_kv, head_dim, kv_type, origin, active, kq_scale, split_mode,
-                           out.data_ptr(), lse.data_ptr(), ctypes.c_void_p(wp), wn, _stream(stream)),
-           "fa_range")
+    head = (q.data_ptr(), positions.data_ptr(), n_q, n_head, k.data_ptr(), v.data_ptr(), n_head_kv, head_dim,
+            kv_type, origin, active, kq_scale, split_mode)
+    tail = (out.data_ptr(), lse.data_ptr(), ctypes.c_void_p(wp), wn, _stream(stream))
+    st = lib.xq_fa_range(*head, *tail) if engine == ENGINE_AUTO else lib.xq_fa_range_engine(*head, engine, *tail)
+    _check(st, "fa_range")
     return ws
 
 
