@@ -101,3 +101,43 @@ def test_fa_range_quant_engines(torch_gpu, kv, d, hkv, group, n_q, active, split
         assert np.abs(lse[seen] - rlse[seen]).max() < 1e-5 * np.abs(rlse[seen]).max()
     auto = _call(torch_gpu, q, positions, kraw, vraw, hkv, kv, origin, active, scale, split)
     assert np.array_equal(auto[0], got) and np.array_equal(auto[1], lse), "AUTO is the matrix cores"
+
+
+@pytest.mark.parametrize("split", [xqattn.SPLIT_NONE, xqattn.SPLIT_REFERENCE], ids=["one_split", "splits"])
+@pytest.mark.parametrize("signs", ["mixed", "same", "one_zero", "opposite"])
+@pytest.mark.parametrize("scale_bits", [0x7C00, 0xFC00, 0x7E00], ids=["inf", "neg_inf", "nan"])
+@pytest.mark.parametrize("kv", [wl.Q8_0, wl.Q4_0], ids=lambda t: wl.TYPE_NAME[t])
+def test_fa_range_quant_nonfinite_k_scale(torch_gpu, kv, scale_bits, signs, split):
+    """An Inf or NaN block scale in one K record. The block's 32 products are +-Inf or
+    NaN each: a row whose products differ in sign, or that holds a zero, scores NaN;
+    one sign scores +Inf (the query's rows are poisoned) or -Inf (weight 0). Both
+    engines give the oracle's pattern, and its finite rows."""
+    n_q, hkv, group, d, active, origin, row, blk = 4, 2, 6, 256, 700, 50, 400, 5
+    n_head, scale = hkv * group, 1.0 / 16
+    kraw = oracle.quantize(kv, wl.normal(41, (active, hkv, d)))
+    vraw = oracle.quantize(kv, wl.normal(42, (active, hkv, d)))
+    bb = kraw.shape[-1] // (d // 32)
+    rec = kraw[row, 1, blk * bb:(blk + 1) * bb]
+    rec[:2] = np.frombuffer(np.uint16(scale_bits).tobytes(), np.uint8)
+    q = wl.normal(43, (n_q, n_head, d))
+    if signs != "mixed":
+        rec[2:] = np.arange(1, 33, dtype=np.uint8) if kv == wl.Q8_0 else 0x9F  # 1 .. 32; nibbles 7 and 1
+        cut = q[:, :, 32 * blk:32 * blk + 32]
+        cut[:] = np.abs(cut) * (-1.0 if signs == "opposite" else 1.0)
+        if signs == "one_zero":
+            cut[0, :, 7] = 0.0
+            rec[4] = 0 if kv == wl.Q8_0 else 0x89
+    positions = np.array([origin + 699, origin + row, origin + row - 1, origin + 5000], np.int32)
+    want, wlse, _ = oracle.range_attn(q, positions, n_head, kraw, vraw, hkv, d, kv, origin, active, scale,
+                                      xqattn.split_count(active, split))
+    bad = np.isnan(wlse)
+    assert not bad[2].any() and not bad[:, :group].any()
+    inf = scale_bits != 0x7E00
+    skipped = inf and signs in ("same", "opposite") and (scale_bits == 0xFC00) != (signs == "opposite")
+    assert bad[0, group:].all() != skipped
+    for engine in (xqattn.ENGINE_VALU, xqattn.ENGINE_MFMA):
+        case_note(f"K scale {scale_bits:#x} {signs} {wl.TYPE_NAME[kv]} split {split} engine {engine}")
+        got, lse = _call(torch_gpu, q, positions, kraw, vraw, hkv, kv, origin, active, scale, split, engine)
+        assert np.array_equal(np.isnan(lse), bad) and np.isnan(got[bad]).all()
+        assert np.abs(got[~bad] - want[~bad]).max() < 1e-5 * np.abs(want[~bad]).max()
+        assert np.abs(lse[~bad] - wlse[~bad]).max() < 1e-5 * np.abs(wlse[~bad]).max()

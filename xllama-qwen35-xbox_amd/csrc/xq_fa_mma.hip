@@ -203,6 +203,12 @@ XQ_DEV h8 k_block_f16(const uint8_t* rec, int b, int g, uint32_t k6400) {
     return __builtin_bit_cast(h8, uint4{h[0], h[1], h[2], h[3]});
 }
 
+// Slot of element el of a block in the score operands: 8 lg + place in lane group lg's eight
+template <int KT>
+XQ_DEV int q_slot(int el) {
+    return KT == XQ_TYPE_Q4_0 ? 8 * ((el % 16) / 4) + el / 16 * 4 + el % 4 : el;
+}
+
 // V^T operands of one q8_0 block: the signed bytes 0 (tile 0) and 1 (tile 1)
 // of the rows' 16-bit words x0..x3 as f16 pairs (rows 0,1 and rows 2,3),
 // exact. Each pair is two SDWA conversions of sign-extended bytes, the second
@@ -634,7 +640,7 @@ __global__ __launch_bounds__((64 * DecCfg<KT, D, MT, QF, MIS>::NW)) void fa_dec(
                     if (lane == 0) sQf[p] = __builtin_ldexpf(a.scale * kLog2e, -up);
                 }
                 const int el = (lane * VD) % kQK;  // in its block
-                const int slot = KT == XQ_TYPE_Q4_0 ? 8 * ((el % 16) / 4) + el / 16 * 4 + el % 4 : el;  // 8 lg + slot
+                const int slot = q_slot<KT>(el);  // 8 lg + slot
                 uint8_t* op = sQ + ((p / 16) * NB + lane * VD / kQK) * 1024 + (slot / 8) * 256 + (p % 16) * 16 + (slot % 8) * 2;
                 uint32_t hb[VD], lb[VD];
 #pragma unroll
@@ -791,16 +797,15 @@ __global__ __launch_bounds__((64 * DecCfg<KT, D, MT, QF, MIS>::NW)) void fa_dec(
 #pragma unroll
                 for (int i = 0; i < 4; ++i) s[m][i] = 0.0f;
             // blocks in batches of four: dks[m][4j + i] = d_k(row 4lg + i, block
-            // c0 + j) * the pair's factor, then s += dks * (K . Q of the block). An
-            // Inf block scale enters as NaN: its row's score is never finite, and
-            // the range's poisoning must see it whatever the dot's sign
+            // c0 + j) * the pair's factor, then s += dks * (K . Q of the block)
+            bool inf = false;
 #pragma unroll
             for (int c0 = 0; c0 < NB; c0 += 4) {
                 const float dk = (float)*(const _Float16*)(Ks + lr * REC + BB * (c0 + lg));
-                const float dkl = __builtin_isfinite(dk) ? dk : NAN;
+                inf |= __builtin_isinf(dk);
                 f16v dks[MT];
 #pragma unroll
-                for (int m = 0; m < MT; ++m) dks[m] = __builtin_amdgcn_mfma_f32_16x16x1f32(dkl, qf[m], f16v{}, 0, 0, 0);
+                for (int m = 0; m < MT; ++m) dks[m] = __builtin_amdgcn_mfma_f32_16x16x1f32(dk, qf[m], f16v{}, 0, 0, 0);
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
                     const h8 kf = k_block_f16<KT>(Ks + lr * REC, c0 + j, lg, k6400);
@@ -813,6 +818,34 @@ __global__ __launch_bounds__((64 * DecCfg<KT, D, MT, QF, MIS>::NW)) void fa_dec(
                         for (int i = 0; i < 4; ++i) s[m][i] = fmaf(dot[i], dks[m][4 * j + i], s[m][i]);
                     }
                 }
+            }
+            // With an infinite d_k a block is a sum of 32 products q * (k * d_k), each
+            // +-Inf or (k or q zero) NaN: the sign of the dot decides, as above, only
+            // where all 32 have one sign; elsewhere the score is NaN
+            if (__builtin_amdgcn_ballot_w64(inf) != 0) {
+                uint32_t mixed = 0;  // bit 4m + i
+#pragma unroll 1
+                for (int mi = 0; mi < 4 * MT; ++mi) {
+#pragma unroll 1
+                    for (int c = 0; c < NB; ++c) {
+                        const uint8_t* blk = Ks + (4 * lg + (mi & 3)) * REC + BB * c;
+                        if ((lds_u16(blk) & 0x7fffu) != 0x7c00u) continue;
+                        const uint8_t* qc = sQ + ((mi >> 2) * NB + c) * 1024 + lr * 16;
+                        int sum = 0;
+#pragma unroll 1
+                        for (int e = 0; e < kQK; ++e) {
+                            const int k = KT == XQ_TYPE_Q4_0 ? (int)((blk[2 + (e & 15)] >> (e & 16 ? 4 : 0)) & 15u) - 8 : (int)(int8_t)blk[2 + e];
+                            const int at = q_slot<KT>(e);
+                            const float qh = f16_bits_to_f32(lds_u16(qc + (at / 8) * 256 + (at % 8) * 2));  // 0 where Q is
+                            sum += ((k > 0) - (k < 0)) * ((qh > 0.0f) - (qh < 0.0f));
+                        }
+                        if (abs(sum) != kQK) mixed |= 1u << mi;
+                    }
+                }
+#pragma unroll
+                for (int m = 0; m < MT; ++m)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) s[m][i] = (mixed >> (4 * m + i)) & 1u ? NAN : s[m][i];
             }
         } else if constexpr (QUANT) {
 #pragma unroll
