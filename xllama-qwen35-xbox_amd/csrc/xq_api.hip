@@ -556,7 +556,7 @@ xq_status xq_gated_delta_net_workspace(const xq_tensor* q, const xq_tensor* v, i
     if (mode < XQ_GDN_AUTO || mode > XQ_GDN_CHUNKED) return fail(XQ_ERR_BAD_ARG, "bad mode");
     const int64_t T = v->ne[2], B = v->ne[3];
     *bytes = gdn_pick(mode, T) == XQ_GDN_CHUNKED
-                 ? xq::gdn_chunked_workspace_bytes(T, B, slots, q->type == XQ_TYPE_BF16)
+                 ? xq::gdn_chunked_workspace_bytes(T, B, slots)
                  : 0;
     return ok();
 }
@@ -578,7 +578,7 @@ xq_status xq_gated_delta_net(const xq_tensor* q, const xq_tensor* k, const xq_te
     const int64_t T = v->ne[2], B = v->ne[3];
     hipError_t e;
     if (gdn_pick(mode, T) == XQ_GDN_CHUNKED) {
-        const size_t need = xq::gdn_chunked_workspace_bytes(T, B, slots, q->type == XQ_TYPE_BF16);
+        const size_t need = xq::gdn_chunked_workspace_bytes(T, B, slots);
         if (need && (!workspace || workspace_bytes < need))
             return fail(XQ_ERR_WORKSPACE, "workspace of %zu bytes needed, %zu given", need, workspace_bytes);
         e = xq::gdn_chunked_launch(L, (hipStream_t)stream);

@@ -71,7 +71,7 @@ typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef float f4 __attribute__((ext_vector_type(4)));
 
 constexpr int kChunk = 64;
-constexpr int kCols = 16;            // value columns per scan workgroup
+constexpr int kCols = 16;            // value columns per tile of a scan workgroup
 constexpr int kColBlocks = 128 / kCols;
 
 // Workspace record of one (sequence, v-head, chunk), byte offsets. Records are
@@ -126,27 +126,18 @@ typedef uint32_t w4_bf16 __attribute__((ext_vector_type(4), aligned(2)));
 XQ_DEV uint4 ld_words_f32(const uint8_t* p) { return __builtin_bit_cast(uint4, *(const w4_f32*)p); }
 XQ_DEV uint4 ld_words_bf16(const uint8_t* p) { return __builtin_bit_cast(uint4, *(const w4_bf16*)p); }
 
-// Eight consecutive elements of an input row (bf16 or f32) as f32; VEC reads them
-// as 16-byte words, else element by element.
-template <bool BF16, bool VEC>
+// Eight consecutive elements of an input row (bf16 or f32) as f32, element by
+// element; load8v reads f32 ones as two 16-byte words.
+template <bool BF16>
 XQ_DEV void load8(const uint8_t* row, int i0, float (&x)[8]) {
-    if constexpr (VEC && BF16) {
-        const uint4 w = ld_words_bf16(row + 2 * i0);
-        const uint32_t u[4] = {w.x, w.y, w.z, w.w};
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            x[2 * e] = bf16_bits_to_f32(u[e] & 0xffffu);
-            x[2 * e + 1] = bf16_bits_to_f32(u[e] >> 16);
-        }
-    } else if constexpr (VEC) {
-        const uint4 w0 = ld_words_f32(row + 4 * i0), w1 = ld_words_f32(row + 4 * i0 + 16);
-        const uint32_t u[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
+    for (int e = 0; e < 8; ++e) x[e] = BF16 ? bf16_bits_to_f32(((const uint16_t*)row)[i0 + e]) : ((const float*)row)[i0 + e];
+}
+XQ_DEV void load8v(const uint8_t* row, int i0, float (&x)[8]) {
+    const uint4 w0 = ld_words_f32(row + 4 * i0), w1 = ld_words_f32(row + 4 * i0 + 16);
+    const uint32_t u[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
 #pragma unroll
-        for (int e = 0; e < 8; ++e) x[e] = __uint_as_float(u[e]);
-    } else {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) x[e] = BF16 ? bf16_bits_to_f32(((const uint16_t*)row)[i0 + e]) : ((const float*)row)[i0 + e];
-    }
+    for (int e = 0; e < 8; ++e) x[e] = __uint_as_float(u[e]);
 }
 
 // f32 words x0 .. x3 as f16 high parts and remainders, pairs (0, 1) and (2, 3): the
@@ -312,7 +303,7 @@ __global__ __launch_bounds__(256, BF16 ? 2 : 1) void gdn_chunk_prep(GdnChunkArgs
                 const int i0 = 32 * qt + 8 * gi;
                 float xk[8];
                 if (ok) {
-                    load8<BF16, true>(kr, i0, xk);
+                    load8v(kr, i0, xk);
                 } else {
 #pragma unroll
                     for (int e = 0; e < 8; ++e) xk[e] = 0.0f;
@@ -331,7 +322,7 @@ __global__ __launch_bounds__(256, BF16 ? 2 : 1) void gdn_chunk_prep(GdnChunkArgs
                 const int i0 = 32 * ks + 8 * lg;
                 float xq[8];
                 if (t0 + tq < a.T) {
-                    load8<BF16, true>(qr, i0, xq);
+                    load8v(qr, i0, xq);
                 } else {
 #pragma unroll
                     for (int e = 0; e < 8; ++e) xq[e] = 0.0f;
@@ -355,7 +346,7 @@ __global__ __launch_bounds__(256, BF16 ? 2 : 1) void gdn_chunk_prep(GdnChunkArgs
 #pragma unroll
                 for (int gi = 0; gi < 4; ++gi) {
                     float xv[8];
-                    load8<BF16, false>(vr, 32 * qt + 8 * gi, xv);
+                    load8<BF16>(vr, 32 * qt + 8 * gi, xv);
 #pragma unroll
                     for (int e = 0; e < 8; ++e)
                         vm[e2][gi >> 1] = max(vm[e2][gi >> 1], __float_as_uint(xv[e]) & 0x7fffffffu);
@@ -775,8 +766,8 @@ XQ_DEV void scan_sequential(const GdnChunkArgs& a, int b, int h, int cb, int wav
     float* out = a.dst + (int64_t)b * (a.dst_nb2 / 4) + h * 128 + c0;
     for (int t = 0; t < a.T; ++t) {
         float kx[8], qx[8];
-        load8<BF16, false>(a.k + (int64_t)b * a.k_nb3 + (int64_t)t * a.k_nb2 + (int64_t)kh * a.k_nb1, 8 * r, kx);
-        load8<BF16, false>(a.q + (int64_t)b * a.q_nb3 + (int64_t)t * a.q_nb2 + (int64_t)kh * a.q_nb1, 8 * r, qx);
+        load8<BF16>(a.k + (int64_t)b * a.k_nb3 + (int64_t)t * a.k_nb2 + (int64_t)kh * a.k_nb1, 8 * r, kx);
+        load8<BF16>(a.q + (int64_t)b * a.q_nb3 + (int64_t)t * a.q_nb2 + (int64_t)kh * a.q_nb1, 8 * r, qx);
         const float g = *(const float*)(a.g + (int64_t)b * a.g_nb3 + (int64_t)t * a.g_nb2 + (int64_t)h * a.g_nb1);
         const float be = *(const float*)(a.beta + (int64_t)b * a.b_nb3 + (int64_t)t * a.b_nb2 + (int64_t)h * a.b_nb1);
         const uint8_t* vr = a.v + (int64_t)b * a.v_nb3 + (int64_t)t * a.v_nb2 + (int64_t)h * a.v_nb1;
@@ -1209,23 +1200,26 @@ __global__ __launch_bounds__(256) void gdn_chunk_scan(GdnChunkArgs a) {
 
 static int64_t chunked_tokens(int64_t T, int32_t slots) { return slots > 1 ? T - (slots - 1) : T; }
 
-size_t gdn_chunked_workspace_bytes(int64_t T, int64_t B, int32_t slots, bool bf16_rows) {
+size_t gdn_chunked_workspace_bytes(int64_t T, int64_t B, int32_t slots) {
     const int64_t Tc = chunked_tokens(T, slots);
     if (Tc < 1) return 0;
     const int64_t nch = (Tc + kChunk - 1) / kChunk;
-    (void)bf16_rows;  // the same record whatever the row type
     return (size_t)B * 32 * nch * kRecBytes;
 }
 
 bool gdn_chunked_available() { return true; }
 
+// (f32 rows and several tiles: one workgroup per CU, whatever the grid)
 template <bool F32, int NC>
 static void scan_launch(const GdnChunkArgs& a, hipStream_t stream) {
     const uint32_t n_wg = (uint32_t)a.B * 32 * (kColBlocks / NC);
-    if (NC > 1 || n_wg <= 256)
-        launch("gdn_chunk_scan", gdn_chunk_scan<F32, true, NC>, dim3(n_wg), dim3(256), stream, a);
-    else
-        launch("gdn_chunk_scan", gdn_chunk_scan<F32, false, NC>, dim3(n_wg), dim3(256), stream, a);
+    if constexpr (!F32 && NC == 1) {
+        if (n_wg > 256) {
+            launch("gdn_chunk_scan", gdn_chunk_scan<F32, false, NC>, dim3(n_wg), dim3(256), stream, a);
+            return;
+        }
+    }
+    launch("gdn_chunk_scan", gdn_chunk_scan<F32, true, NC>, dim3(n_wg), dim3(256), stream, a);
 }
 
 // Column tiles per scan workgroup for bf16 rows. A workgroup of one tile (66 KB of
@@ -1275,7 +1269,7 @@ hipError_t gdn_chunked_launch(const GdnLaunch& L, hipStream_t stream) {
     // row: row strides of 2^25 bytes or more run token by token instead
     for (const xq_tensor* t : {L.q, L.k, L.v})
         if (t->nb[2] >= ((int64_t)1 << 25)) return gdn_step_launch(L, stream);
-    if (L.workspace_bytes < gdn_chunked_workspace_bytes(T, B, L.slots, L.q->type == XQ_TYPE_BF16))
+    if (L.workspace_bytes < gdn_chunked_workspace_bytes(T, B, L.slots))
         return hipErrorInvalidValue;
     GdnChunkArgs a{};
     a.q = (const uint8_t*)L.q->data;
