@@ -179,8 +179,8 @@ def test_fa_range_vs_reference_semantics(torch_gpu, kv_type, active):
 @pytest.mark.parametrize("kv_type", [wl.F16, wl.Q8_0, wl.Q4_0])
 def test_fa_mask_rows_2byte_aligned(torch_gpu, kv_type, engine):
     """An odd KV length gives mask rows of 2 (mod 4) bytes; a mask view may also
-    start 2 bytes into its buffer. Both run (the matrix-core engine re-lays such
-    a mask in the workspace first) and give the aligned layout's result."""
+    start 2 bytes into its buffer. Both run (the matrix-core engine shifts the
+    elements into place as it reads them) and give the aligned layout's result."""
     torch = torch_gpu
     cfg = wl.FaConfig("odd", 4, 16, 4, 128, 1001, 2, kv_type, causal_prefix=997)
     case_note(f"odd mask rows {wl.TYPE_NAME[kv_type]} engine {engine}")

@@ -103,11 +103,12 @@ void split_policy(int64_t L, int mode, int64_t n_seq_heads, int32_t* n_splits, i
     case XQ_FA_SPLIT_AUTO: {
         // about one workgroup per CU (256 on MI355X) over the (sequence, KV
         // head) pairs, rows a multiple of the 16-row wave slice, and at least
-        // 256 rows per split (two slices per wave of the 8-wave decode): a
-        // short call is bound by latency, and a second slice per wave costs
-        // less than the partial states the extra splits write and merge
-        // (4096 f16 rows over 8 KV heads: 16 splits 15.9 us per call, 32
-        // splits 16.8 us)
+        // 256 rows per split. The count may not depend on the number of queries,
+        // whose pair tiles multiply the workgroups, so the floor lies between what
+        // a single query takes best and several (us per call with 128 / 256 / 512
+        // rows: one query over 4096 f16 rows and 8 KV heads 9.9 / 11.4 / 13.7, over
+        // 2048 q8_0 rows and 4 KV heads 11.7 / 13.7 / 17.5; eight queries over 4097
+        // q8_0 rows and 4 KV heads 25.5 / 17.0 / 19.2)
         k = cdiv(256, n_seq_heads < 1 ? 1 : n_seq_heads);
         const int64_t kmax = cdiv(L, 256);
         if (k > kmax) k = kmax;
