@@ -367,6 +367,12 @@ __global__ __launch_bounds__((64 * DecCfg<KT, D, MT, QF, MIS>::NW)) void fa_dec(
     constexpr int NB = C::NB, NPP = C::NPP, NW = C::NW, QRB = C::QRB;
     constexpr bool QUANT = C::QUANT, INTQ = C::INTQ, QFQ = C::QFQ;
     constexpr int ML = C::ML, MD = C::MD;
+    // A pair's query by the division without branches: less code where a wave forms it
+    // for many pairs (the 8-query q4_0 verify of two pair tiles 75.7 -> 74.6 us, the
+    // 9-query q4_0 range call 54.3 -> 51.7). With one tile and a mask, or Q split in
+    // registers, the schedule that comes with it is the slower one (377 q8_0 rows, 24
+    // heads over 4, 13.5 -> 13.9; f16, 32 over 8, 8 queries, 1000 rows 19.7 -> 20.5).
+    constexpr bool FLAT = QFQ || (MT == 2 && (QUANT || C::QLDS));
     constexpr int BB = KT == XQ_TYPE_Q8_0 ? 34 : 18;
     constexpr int NT = 64 * NW;
     constexpr uint32_t kNegInfH2 = 0xfc00fc00u;  // f16 pair (-inf, -inf)
@@ -379,7 +385,7 @@ __global__ __launch_bounds__((64 * DecCfg<KT, D, MT, QF, MIS>::NW)) void fa_dec(
     // scalar loads go out one dependent group after another
     asm volatile("" ::"s"(a.k), "s"(a.v), "s"(a.q), "s"(a.mask), "s"(a.positions), "s"(a.k_nb1), "s"(a.k_nb2), "s"(a.k_nb3),
                  "s"(a.v_nb1), "s"(a.v_nb2), "s"(a.v_nb3), "s"(a.q_nb1), "s"(a.q_nb2), "s"(a.q_nb3), "s"(a.L), "s"(a.split_rows),
-                 "s"(a.n_wg), "s"(a.d_tiles.m), "s"(a.d_hkv.m), "s"(a.d_splits.m), "s"(a.d_rk3.m), "s"(a.d_rv3.m), "s"(a.d_g.m));
+                 "s"(a.n_wg), "s"(a.d_tiles.m), "s"(a.d_hkv.m), "s"(a.d_splits.m), "s"(a.d_rk3.m), "s"(a.d_rv3.m), "s"(FLAT ? a.d_gf.m : a.d_g.m));
     uint32_t wg = xcd_remap(blockIdx.x, a.n_wg);
     // logical order: pair tile fastest, then KV head, split, sequence, so the
     // heads reading the same rows are neighbours on one XCD (shared L2)
@@ -395,7 +401,7 @@ __global__ __launch_bounds__((64 * DecCfg<KT, D, MT, QF, MIS>::NW)) void fa_dec(
     // pairs, query-major
     const int p0 = qt * a.tile_pairs;
     const int npa = min(a.tile_pairs, a.NQ * a.G - p0);
-    auto pair_q = [&](int p) { return (int)a.d_g.quot((uint32_t)(p0 + p)); };
+    auto pair_q = [&](int p) { return (int)(FLAT ? a.d_gf.quot((uint32_t)(p0 + p)) : a.d_g.quot((uint32_t)(p0 + p))); };
     auto pair_h = [&](int p) { return g_kv * a.G + (p0 + p) - pair_q(p) * a.G; };
     const int wave = wave_id();
     const int lane = lane_id();
@@ -1623,6 +1629,7 @@ hipError_t fa_mma_launch(FaArgs a, const FaLaunch& L, hipStream_t stream) {
     a.d_rk3 = UDiv(a.rk3, a.B);
     a.d_rv3 = UDiv(a.rv3, a.B);
     a.d_g = UDiv(a.G, (uint64_t)n_pairs + 16 * mt);
+    a.d_gf = UDivFlat(a.G);
     launch("fa_dec", fn, dim3(n_wg), dim3(64 * waves), stream, a);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || a.n_splits == 1) return e;
